@@ -263,6 +263,16 @@ NSH_API int nsh_normalized_accumulate_uz_forward(const void* x, const void* weig
                                          int log_weights, void* D, void* log_C,
                                          void* workspace, int64_t workspace_bytes, void* stream);
 
+/* The forward with a check of the weight contract (the reference's
+ * validate=True, ops.py:209-224): *weights_ok, a device int that the caller
+ * has set to a nonzero value, is set to 0 if any weight is NaN, +inf or
+ * (positive mode) negative, weights that the forward box drops included;
+ * it is left alone otherwise.  Outputs as above.  NULL: no check. */
+NSH_API int nsh_normalized_accumulate_uz_forward_checked(
+    const void* x, const void* weights, const int64_t* shifts, int64_t S, int64_t B, int64_t C,
+    int64_t H, int64_t W, int dtype, int log_weights, void* D, void* log_C, int* weights_ok,
+    void* workspace, int64_t workspace_bytes, void* stream);
+
 /* normalized_accumulate_uz backward.  Replaces
  * `normalized_accumulate_uz_backward(x, weights, D, log_C, grad_D, grad_log_C,
  * shifts, log_weights)` (csrc/shift_ops.cpp:254-280; kernels

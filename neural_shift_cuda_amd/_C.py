@@ -68,6 +68,8 @@ _SIGS = {
                                          _I64, _I, _P, _P, _P, _I64, _P], _I),
     "nsh_normalized_accumulate_uz_forward": ([_P, _P, _P, _I64, _I64, _I64, _I64, _I64, _I, _I,
                                               _P, _P, _P, _I64, _P], _I),
+    "nsh_normalized_accumulate_uz_forward_checked": ([_P, _P, _P, _I64, _I64, _I64, _I64, _I64,
+                                                      _I, _I, _P, _P, _P, _P, _I64, _P], _I),
     "nsh_normalized_accumulate_uz_forward_mixed": ([_P, _P, _P, _P, _I64, _I64, _I64, _I64,
                                                     _I64, _I64, _I, _P, _P, _P, _I64, _P], _I),
     "nsh_head_mix_forward": ([_P, _P, _I64, _I64, _I64, _I64, _I, _P, _P], _I),
@@ -394,20 +396,29 @@ def accumulate_uz_backward(x: torch.Tensor, weights: torch.Tensor, grad_U: torch
 
 def normalized_accumulate_uz_forward(x: torch.Tensor, weights: torch.Tensor, shifts: torch.Tensor,
                                      log_weights: bool, *, row_codes: bool = False,
-                                     shared_weights: bool = False) -> List[torch.Tensor]:
-    """[D, log_C] in the accumulator dtype (shift_ops.cpp:218-252)."""
+                                     shared_weights: bool = False,
+                                     weights_ok: Optional[torch.Tensor] = None
+                                     ) -> List[torch.Tensor]:
+    """[D, log_C] in the accumulator dtype (shift_ops.cpp:218-252).
+    `weights_ok`: a one-element int32 tensor holding a nonzero value, set to 0
+    when a weight breaks the op's contract
+    (nsh_normalized_accumulate_uz_forward_checked)."""
     sh, B, C, H, W, S = _check_pair("normalized_accumulate_uz", x, weights, shifts,
                                     "normalized_accumulate_uz: weights must be (S*B, C, H, W)",
                                     shared_weights)
     acc = _acc_dtype(x.dtype)
     code = _code(x, "normalized_accumulate_uz_fwd") | _flags(row_codes, shared_weights)
+    if weights_ok is not None:
+        _check(weights_ok.device == x.device and weights_ok.dtype == torch.int32
+               and weights_ok.numel() == 1,
+               "normalized_accumulate_uz: weights_ok must be one int32 element on x's device")
     D = torch.empty(x.shape, dtype=acc, device=x.device)
     L = torch.empty(x.shape, dtype=acc, device=x.device)
     ws, nws = _norm_workspace(S, B, C, H, W, code, False, x.device)
     with torch.cuda.device(x.device):
-        _call("nsh_normalized_accumulate_uz_forward", x.data_ptr(), weights.data_ptr(),
+        _call("nsh_normalized_accumulate_uz_forward_checked", x.data_ptr(), weights.data_ptr(),
               sh.data_ptr(), S, B, C, H, W, code, int(bool(log_weights)), D.data_ptr(),
-              L.data_ptr(), _ptr(ws), nws, _stream(x))
+              L.data_ptr(), _ptr(weights_ok), _ptr(ws), nws, _stream(x))
     return [D, L]
 
 

@@ -125,6 +125,19 @@ __device__ __forceinline__ void online_final(const Online<A>& st, A& D, A& L) {
     }
 }
 
+// A weight that breaks the op's contract: a NaN or +inf logit; a negative,
+// NaN or +inf positive weight.  The kernels' states already carry every such
+// key they take in (NaN in both outputs), so a forward asked to check the
+// weights (weights_ok) reads the answer off its states and tests a weight
+// itself only where the forward box drops it; a separate pass over the
+// weights is not needed (c3 positive, 1.5 GB of fp32 weights: the check took
+// 2.2 ms as elementwise passes, and the whole forward takes 0.30 ms with or
+// without it).
+template <typename A, bool LOGW>
+__device__ __forceinline__ bool key_bad(A k) {
+    return LOGW ? !(k <= Lim<A>::maxv()) : !(k >= A(0) && k <= Lim<A>::maxv());
+}
+
 __device__ __forceinline__ bool tile_inside_n(int h0, int w0, int TH, int TW, int H, int W, int dx,
                                               int dy) {
     const int h1 = (h0 + TH < H ? h0 + TH : H) - 1;
@@ -136,7 +149,7 @@ template <typename T, int VEC, bool LOGW>
 __global__ __launch_bounds__(kThreads) void normalized_fwd_kernel(
     const T* __restrict__ x, const T* __restrict__ w, const int64_t* __restrict__ shifts, int S,
     int codes, int C, int H, int W, int ntw, int nth, int64_t plane_step,
-    acc_t<T>* __restrict__ Dout, acc_t<T>* __restrict__ Lout) {
+    acc_t<T>* __restrict__ Dout, acc_t<T>* __restrict__ Lout, int* __restrict__ weights_ok) {
     using A = acc_t<T>;
     using G = NGeo<VEC>;
     extern __shared__ __align__(16) unsigned char smem[];
@@ -166,6 +179,7 @@ __global__ __launch_bounds__(kThreads) void normalized_fwd_kernel(
     Online<A> st[VEC];
 #pragma unroll
     for (int k = 0; k < VEC; ++k) online_init<A, LOGW>(st[k]);
+    bool bad = false;  // a weight outside the contract (weights_ok)
 
     for (int s = 0; s < S; ++s, wp += wstep) {
         const ShiftRec r = read_shift(shl, s);
@@ -187,10 +201,12 @@ __global__ __launch_bounds__(kThreads) void normalized_fwd_kernel(
             }
         }
 #pragma unroll
-        for (int k = 0; k < VEC; ++k)
+        for (int k = 0; k < VEC; ++k) {
+            if (weights_ok != nullptr) bad |= key_bad<A, LOGW>(wv[k]);
             online_add<A, LOGW>(st[k], fwd_kept(r, h, w0 + k, H, W) ? wv[k]
                                                                     : masked_key<A, LOGW>(),
                                 xv[k]);
+        }
 
         if (r.inv) {
             // source (h - dx, w - dy), wrapped for a circular mirror
@@ -210,6 +226,7 @@ __global__ __launch_bounds__(kThreads) void normalized_fwd_kernel(
             }
         }
     }
+    if (weights_ok != nullptr && bad) *weights_ok = 0;
     A Dv[VEC], Lv[VEC];
 #pragma unroll
     for (int k = 0; k < VEC; ++k) online_final<A, LOGW>(st[k], Dv[k], Lv[k]);
@@ -658,7 +675,7 @@ normalized_fwd_scatter_kernel(const T* __restrict__ x, const T* __restrict__ w,
                               acc_t<T>* __restrict__ Lout, int* __restrict__ hdr,
                               acc_t<T>* __restrict__ spill, acc_t<T>* __restrict__ part,
                               int ring_stride, int64_t ntiles,
-                              const acc_t<T>* __restrict__ mix) {
+                              const acc_t<T>* __restrict__ mix, int* __restrict__ weights_ok) {
     using A = acc_t<T>;
     using G = SGeo<VEC, ROWS, TPR>;
     extern __shared__ __align__(16) unsigned char smem[];
@@ -859,6 +876,38 @@ normalized_fwd_scatter_kernel(const T* __restrict__ x, const T* __restrict__ w,
         }
     }
 
+    if (weights_ok != nullptr) {
+        // every weight the box kept went into its own pixel's state
+        bool bad = false;
+#pragma unroll
+        for (int k = 0; k < VEC; ++k)
+            bad |= px.act[k] && (sz[k] != sz[k] || (LOGW && sm[k] == Lim<A>::inf()));
+        // The ones it dropped are read again here, a batch of shifts in
+        // flight (a pixel that keeps its weight re-reads its plane's first
+        // element): tested in the ring loop they made every forward with the
+        // box 5% (fp16 logits) to 19% (rows beyond the border) slower.
+        if (!interior && table_any_fbox(shl, S)) {
+            constexpr int NB = 8;
+            for (int s0 = 0; s0 < S; s0 += NB) {
+                A v[NB][VEC];
+#pragma unroll
+                for (int i = 0; i < NB; ++i) {
+                    const ShiftRec rc = read_shift(shl, min(s0 + i, S - 1));
+                    const T* wp = w_bc + static_cast<int64_t>(min(s0 + i, S - 1)) * wstep;
+#pragma unroll
+                    for (int k = 0; k < VEC; ++k) {
+                        const bool kept = fwd_kept(rc, h, ti.w0 + tx + k * TPR, H, W);
+                        v[i][k] = to_acc(*elem_ptr(wp, kept ? 0u : px.own[k]));
+                    }
+                }
+#pragma unroll
+                for (int i = 0; i < NB; ++i)
+#pragma unroll
+                    for (int k = 0; k < VEC; ++k) bad |= key_bad<A, LOGW>(v[i][k]);
+            }
+        }
+        if (bad) *weights_ok = 0;
+    }
     __syncthreads();
     const int th = min(G::TH, H - ti.h0);
     const int tw = min(G::TW, W - ti.w0);
@@ -1331,7 +1380,7 @@ struct NDims {
 
 template <typename T, int VEC, bool LOGW>
 static int n_launch_fwd(const void* x, const void* w, const int64_t* sh, NDims d, void* D, void* L,
-                        hipStream_t st) {
+                        int* weights_ok, hipStream_t st) {
     using G = NGeo<VEC>;
     const int ntw = static_cast<int>(nsh_host::ceil_div(d.W, G::TW));
     const int nth = static_cast<int>(nsh_host::ceil_div(d.H, G::TH));
@@ -1340,7 +1389,7 @@ static int n_launch_fwd(const void* x, const void* w, const int64_t* sh, NDims d
     hipLaunchKernelGGL((normalized_fwd_kernel<T, VEC, LOGW>), dim3(static_cast<unsigned>(tiles)),
                        dim3(kThreads), n_lds<T>(VEC, d.S, false), st, static_cast<const T*>(x),
                        static_cast<const T*>(w), sh, d.S, d.codes, d.C, d.H, d.W, ntw, nth, step,
-                       static_cast<acc_t<T>*>(D), static_cast<acc_t<T>*>(L));
+                       static_cast<acc_t<T>*>(D), static_cast<acc_t<T>*>(L), weights_ok);
     return nsh_host::check_launch("normalized_accumulate_uz_forward");
 }
 
@@ -1472,7 +1521,7 @@ static bool n_use_scatter(const NPlan& p, void* ws, int64_t ws_bytes) {
 // kernel's weight load.
 template <typename T, bool LOGW, int NH = 1>
 static int n_scatter_fwd(const void* x, const void* w, const int64_t* sh, NDims d, void* D,
-                         void* L, const NPlan& p, void* ws, hipStream_t st,
+                         void* L, const NPlan& p, void* ws, int* weights_ok, hipStream_t st,
                          const acc_t<T>* mix = nullptr) {
     using Cfg = NScatterCfg<T, false>;
     using A = acc_t<T>;
@@ -1486,7 +1535,7 @@ static int n_scatter_fwd(const void* x, const void* w, const int64_t* sh, NDims 
                        dim3(static_cast<unsigned>(p.tiles)), dim3(TPR * RW), p.lds, st,
                        static_cast<const T*>(x), static_cast<const T*>(w), sh, d.S, d.codes, d.C, d.H, d.W,
                        p.ntw, p.nth, step, static_cast<A*>(D), static_cast<A*>(L), hdr, spill, part,
-                       p.ring, p.tiles, mix);
+                       p.ring, p.tiles, mix, weights_ok);
     if (int rc = nsh_host::check_launch("normalized_accumulate_uz_forward")) return rc;
     hipLaunchKernelGGL((normalized_fixup_kernel<A, LOGW>), dim3(static_cast<unsigned>(p.tiles)),
                        dim3(256), 0, st, d.H, d.W, RW, TPR * V, p.ntw, p.nth, p.spill, p.ring,
@@ -1562,17 +1611,17 @@ static int64_t n_workspace(const NDims& d, bool bwd) {
 
 template <typename T, bool LOGW>
 static int n_run_fwd(const void* x, const void* w, const int64_t* sh, NDims d, void* D, void* L,
-                     void* ws, int64_t ws_bytes, hipStream_t st) {
+                     void* ws, int64_t ws_bytes, int* weights_ok, hipStream_t st) {
     const NPlan p = n_plan<T>(d, false);
     if (n_use_scatter<T>(p, ws, ws_bytes))
-        return n_scatter_fwd<T, LOGW>(x, w, sh, d, D, L, p, ws, st);
+        return n_scatter_fwd<T, LOGW>(x, w, sh, d, D, L, p, ws, weights_ok, st);
     switch (n_pick_vec<T>(d.W, {x, w, D, L}, d.S, false)) {
-        case 8: if constexpr (sizeof(T) == 2) return n_launch_fwd<T, 8, LOGW>(x, w, sh, d, D, L, st); break;
-        case 4: if constexpr (sizeof(T) <= 4) return n_launch_fwd<T, 4, LOGW>(x, w, sh, d, D, L, st); break;
-        case 2: return n_launch_fwd<T, 2, LOGW>(x, w, sh, d, D, L, st);
+        case 8: if constexpr (sizeof(T) == 2) return n_launch_fwd<T, 8, LOGW>(x, w, sh, d, D, L, weights_ok, st); break;
+        case 4: if constexpr (sizeof(T) <= 4) return n_launch_fwd<T, 4, LOGW>(x, w, sh, d, D, L, weights_ok, st); break;
+        case 2: return n_launch_fwd<T, 2, LOGW>(x, w, sh, d, D, L, weights_ok, st);
         default: break;
     }
-    return n_launch_fwd<T, 1, LOGW>(x, w, sh, d, D, L, st);
+    return n_launch_fwd<T, 1, LOGW>(x, w, sh, d, D, L, weights_ok, st);
 }
 
 template <typename T, bool LOGW>
@@ -1633,12 +1682,10 @@ extern "C" int64_t nsh_normalized_workspace_bytes(int64_t S, int64_t B, int64_t 
     }
 }
 
-extern "C" int nsh_normalized_accumulate_uz_forward(const void* x, const void* weights,
-                                                    const int64_t* shifts, int64_t S, int64_t B,
-                                                    int64_t C, int64_t H, int64_t W, int dtype,
-                                                    int log_weights, void* D, void* log_C,
-                                                    void* workspace, int64_t workspace_bytes,
-                                                    void* stream) {
+extern "C" int nsh_normalized_accumulate_uz_forward_checked(
+    const void* x, const void* weights, const int64_t* shifts, int64_t S, int64_t B, int64_t C,
+    int64_t H, int64_t W, int dtype, int log_weights, void* D, void* log_C, int* weights_ok,
+    void* workspace, int64_t workspace_bytes, void* stream) {
     nsh::NDims d;
     if (int rc = n_check("normalized_accumulate_uz", S, B, C, H, W, dtype, &d)) return rc;
     dtype &= ~NSH_DTYPE_FLAGS;
@@ -1648,11 +1695,22 @@ extern "C" int nsh_normalized_accumulate_uz_forward(const void* x, const void* w
     void* ws = workspace;
     const int64_t nws = workspace ? workspace_bytes : 0;
     switch (dtype) {
-        case NSH_DTYPE_FLOAT16: return NSH_DISPATCH_LOGW(nsh::f16, n_run_fwd, x, weights, shifts, d, D, log_C, ws, nws, st);
-        case NSH_DTYPE_BFLOAT16: return NSH_DISPATCH_LOGW(nsh::bf16, n_run_fwd, x, weights, shifts, d, D, log_C, ws, nws, st);
-        case NSH_DTYPE_FLOAT32: return NSH_DISPATCH_LOGW(float, n_run_fwd, x, weights, shifts, d, D, log_C, ws, nws, st);
-        default: return NSH_DISPATCH_LOGW(double, n_run_fwd, x, weights, shifts, d, D, log_C, ws, nws, st);
+        case NSH_DTYPE_FLOAT16: return NSH_DISPATCH_LOGW(nsh::f16, n_run_fwd, x, weights, shifts, d, D, log_C, ws, nws, weights_ok, st);
+        case NSH_DTYPE_BFLOAT16: return NSH_DISPATCH_LOGW(nsh::bf16, n_run_fwd, x, weights, shifts, d, D, log_C, ws, nws, weights_ok, st);
+        case NSH_DTYPE_FLOAT32: return NSH_DISPATCH_LOGW(float, n_run_fwd, x, weights, shifts, d, D, log_C, ws, nws, weights_ok, st);
+        default: return NSH_DISPATCH_LOGW(double, n_run_fwd, x, weights, shifts, d, D, log_C, ws, nws, weights_ok, st);
     }
+}
+
+extern "C" int nsh_normalized_accumulate_uz_forward(const void* x, const void* weights,
+                                                    const int64_t* shifts, int64_t S, int64_t B,
+                                                    int64_t C, int64_t H, int64_t W, int dtype,
+                                                    int log_weights, void* D, void* log_C,
+                                                    void* workspace, int64_t workspace_bytes,
+                                                    void* stream) {
+    return nsh_normalized_accumulate_uz_forward_checked(x, weights, shifts, S, B, C, H, W, dtype,
+                                                        log_weights, D, log_C, nullptr, workspace,
+                                                        workspace_bytes, stream);
 }
 
 // Head mixing in the weight load: with a (C, heads) mix the scatter path
@@ -1669,9 +1727,9 @@ static int n_run_fwd_mixed(const void* x, const void* hw, const void* mix, const
                     "the scatter path");
     const A* m = static_cast<const A*>(mix);
     switch (heads) {
-        case 2: return nsh::n_scatter_fwd<T, false, 2>(x, hw, sh, d, D, L, p, ws, st, m);
-        case 3: return nsh::n_scatter_fwd<T, false, 3>(x, hw, sh, d, D, L, p, ws, st, m);
-        default: return nsh::n_scatter_fwd<T, false, 4>(x, hw, sh, d, D, L, p, ws, st, m);
+        case 2: return nsh::n_scatter_fwd<T, false, 2>(x, hw, sh, d, D, L, p, ws, nullptr, st, m);
+        case 3: return nsh::n_scatter_fwd<T, false, 3>(x, hw, sh, d, D, L, p, ws, nullptr, st, m);
+        default: return nsh::n_scatter_fwd<T, false, 4>(x, hw, sh, d, D, L, p, ws, nullptr, st, m);
     }
 }
 

@@ -263,16 +263,22 @@ def accumulate_uz_reference(x: torch.Tensor, weights: torch.Tensor, shifts: torc
     return _tree_sum(torch.stack(u_terms)), _tree_sum(torch.stack(z_terms))
 
 
+def _weight_contract(log_weights: bool) -> str:
+    """What the normalized op's weights must be, as the error says it."""
+    return ("log_weights may be finite or -inf (mask), but not NaN or +inf" if log_weights
+            else "positive weights must be finite and nonnegative")
+
+
 def _validate_stable_weights(weights: torch.Tensor, log_weights: bool, *,
                              asynchronous: bool) -> None:
     """Weight contract of the normalized op (reference ops.py:209-224):
-    log weights finite or -inf; positive weights finite and >= 0."""
+    log weights finite or -inf; positive weights finite and >= 0.  (On the GPU
+    the forward kernel checks the weights it reads: normalized_accumulate_uz.)"""
+    message = _weight_contract(log_weights)
     if log_weights:
         ok = torch.isfinite(weights) | (torch.isinf(weights) & (weights < 0))
-        message = "log_weights may be finite or -inf (mask), but not NaN or +inf"
     else:
         ok = torch.isfinite(weights) & (weights >= 0)
-        message = "positive weights must be finite and nonnegative"
     allok = ok.all()
     if asynchronous and weights.is_cuda and hasattr(torch, "_assert_async"):
         torch._assert_async(allok, message)
@@ -496,14 +502,16 @@ def mix_head_planes(w: torch.Tensor, mix: torch.Tensor) -> torch.Tensor:
 
 class _NormalizedAccumulateUZFn(torch.autograd.Function):
     @staticmethod
-    def forward(ctx, x, weights, shifts, log_weights, row_codes=False, shared=False):
+    def forward(ctx, x, weights, shifts, log_weights, row_codes=False, shared=False,
+                weights_ok=None):
         if shifts.dim() != 2 or shifts.size(1) != 3:
             raise ValueError("normalized_accumulate_uz requires shifts of shape (S, 3)")
         shifts_i = _prep_shifts_for_cuda(shifts, x.device)
         x_c, w_c = x.contiguous(), weights.contiguous()
         D, log_C = _C.normalized_accumulate_uz_forward(x_c, w_c, shifts_i, bool(log_weights),
                                                        row_codes=row_codes,
-                                                       shared_weights=shared)
+                                                       shared_weights=shared,
+                                                       weights_ok=weights_ok)
         ctx.save_for_backward(x_c, w_c, D, log_C, shifts_i)
         ctx.log_weights = bool(log_weights)
         ctx.row_codes = row_codes
@@ -521,7 +529,7 @@ class _NormalizedAccumulateUZFn(torch.autograd.Function):
         grad_x, grad_w = _C.normalized_accumulate_uz_backward(
             x, weights, D, log_C, grad_D.contiguous(), grad_log_C.contiguous(), shifts_i,
             ctx.log_weights, row_codes=ctx.row_codes, shared_weights=ctx.shared)
-        return grad_x, _shared_grad(grad_w, ctx.shared), None, None, None, None
+        return grad_x, _shared_grad(grad_w, ctx.shared), None, None, None, None, None
 
 
 class _AccumulateUZScalarFn(torch.autograd.Function):
@@ -664,13 +672,19 @@ def normalized_accumulate_uz(x: torch.Tensor, weights: torch.Tensor, shifts: tor
     box_forward, shared_weights: as in ``accumulate_uz`` (a dropped forward
     term acts as a masked weight)."""
     x_d, w_d = _device_operands(x, weights)
-    if validate:
+    in_kernel = x_d.is_cuda and hasattr(torch, "_assert_async")
+    if validate and not in_kernel:
         _validate_stable_weights(w_d, log_weights, asynchronous=x_d.is_cuda)
     if x_d.is_cuda:
         table, codes = _mirror_table(shifts, periodic_inverse, box_forward)
         _require_cuda_ext("normalized_accumulate_uz", need_normalized=True)
+        # the forward kernel checks every weight as it reads it
+        ok = (torch.ones((), dtype=torch.int32, device=x_d.device)
+              if validate and in_kernel else None)
         D, log_C = _NormalizedAccumulateUZFn.apply(x_d, w_d, table, log_weights, codes,
-                                                   bool(shared_weights))
+                                                   bool(shared_weights), ok)
+        if ok is not None:
+            torch._assert_async(ok, _weight_contract(log_weights))
     else:
         weights = _shared_operand(weights, x.shape[1], shared_weights)
         x_acc, w_acc = _promote_accumulation_inputs(x, weights)
