@@ -304,6 +304,7 @@ __device__ __forceinline__ int clamp_shift(int64_t v) {
 }
 
 __device__ __forceinline__ int64_t mod_pos(int64_t v, int64_t n) {
+    if (v >= -n && v < n) return v < 0 ? v + n : v;  // a wave of such values skips the division
     int64_t r = v % n;
     return r < 0 ? r + n : r;
 }

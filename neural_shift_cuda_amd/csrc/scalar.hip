@@ -5,101 +5,125 @@
 //   gx[q]     = sum_s w[s,b,c] gU[(q-s) mod]
 //   gw[s,b,c] = sum_{p} gU[p] x[(p+s) mod] + gZ[p]
 // The weights are tiny (S*B*C) and x, gU are re-read S times, so the op is
-// bound by LDS and VALU work, not HBM.  One workgroup (512 lanes) owns a
-// 64 x 32 tile of one (b, c) plane: the tile of x (or gU) with a kRmax
-// halo, the plane's S weights and the shift table sit in LDS, and lane tx
-// owns the 4 pixels tx, tx + 16, tx + 32, tx + 48 of its row (strided: the
-// LDS reads of a wave cover 16 consecutive words per row, free of bank
-// conflicts).  gw is a deterministic two-level reduction: each tile forms,
-// for every shift, sum over its pixels of gU[p] x[p+s] + gZ[p] (lane sums,
-// a wave64 xor-shuffle butterfly, the wave sums in fixed order) into a
-// caller workspace of S*B*C*ntiles partials, and a second kernel adds the
-// tiles of each (s, b, c) in index order.
+// bound by the vector ALU (one FMA per pixel and shift and pass) and, if
+// every FMA takes its own LDS read, by LDS.  One workgroup (four waves) owns
+// a 64 x 32 tile of one (b, c) plane; the tile of x (or gU) with a kRmax halo
+// sits in LDS, a lane owns one column and a wave reads 64 consecutive words
+// of a row, free of bank conflicts.
+//
+// Tables are mostly dense windows, so the rows near enough for the LDS tile
+// are laid out as a grid of (dy, dx) over their bounding box (SGrid) and a
+// lane walks the grid column by column: P + 3 values of its column serve four
+// neighbouring dx of its P pixels (11 LDS reads for 32 FMAs; 35 for 128 in
+// gw), instead of one LDS read and a share of the row's decoding per FMA.
+// Tables that repeat a row or fill less than half of their box (a walk of the
+// whole box would then read more than the row-by-row loop) take the
+// row-by-row loop, as do rows beyond the halo (from global memory).  16 x 3 x
+// 256^2, 121 rows, fp32, row by row -> grid: forward 64 -> 31 us, gx 62 -> 30
+// us, gw 79 -> 28 us (0.76 GFLOP a pass: 10 us at the vector ALU's rate; the
+// rest is mostly the tile's prologue, one round of workgroups).
+//
+// gw is a deterministic two-level reduction: a wave forms, for its share of
+// the shifts, the sum over the tile's pixels of gU[p] x[p+s] + gZ[p] (lane
+// sums over 32 rows, then a wave64 DPP reduction) into a caller workspace of
+// S*B*C*ntiles partials, and a second kernel adds the tiles of each
+// (s, b, c) in index order.
 #include <initializer_list>
+#include <type_traits>
 
 #include "nsh_common.hpp"
 #include "scatter.hpp"
 
 namespace nsh {
 
-constexpr int kScVec = 4;
-constexpr int kScTpr = 16;
-constexpr int kScRows = 32;
-using ScG = SGeo<kScVec, kScRows, kScTpr>;
-constexpr int kScThreads = ScG::THREADS;
+constexpr int kScTW = 64;   // tile columns: one per lane of a wave
+constexpr int kScTH = 32;   // tile rows
+constexpr int kScWaves = 4;
+constexpr int kScThreads = 64 * kScWaves;
+constexpr int kScP = kScTH / kScWaves;  // rows per lane of the forward and gx
+constexpr int kScPitch = kScTW + 2 * kRmax;
+constexpr int kScLH = kScTH + 2 * kRmax;
+constexpr int kScChunk = 4;  // neighbouring dx taken from one set of column values
+// rows a chunk's column values may reach past the halo (never used there)
+constexpr int kScPad = kScChunk - 1;
+constexpr int kScTile = (kScLH + kScPad) * kScPitch;
 
-// MODE 0: forward (src = x, writes U and Z);  MODE 1: gx (src = gU).
-template <typename T, int MODE>
-__global__ __launch_bounds__(kScThreads) void scalar_tile_kernel(
-    const void* __restrict__ src_v, const T* __restrict__ w, const int64_t* __restrict__ shifts,
-    int cols, int S, int B, int C, int H, int W, int ntw, int nth, void* __restrict__ out0,
-    acc_t<T>* __restrict__ out1) {
-    using A = acc_t<T>;
-    using G = ScG;
-    constexpr int VEC = kScVec, TPR = kScTpr;
-    extern __shared__ __align__(16) unsigned char smem[];
-    int4* shl = reinterpret_cast<int4*>(smem);
-    A* wl = reinterpret_cast<A*>(smem + shift_lds_bytes(S));
-    A* st = reinterpret_cast<A*>(smem + shift_lds_bytes(S) + static_cast<size_t>(S) * sizeof(A));
+// The table's near rows (|dx|, |dy| <= kRmax) as a grid over their bounding
+// box: cell (dyi, dxi) holds the table row of displacement (dx0 + dxi,
+// dy0 + dyi).  SGN = -1 grids the negated displacements (gx reads q - s).
+constexpr int kScBox = 2 * kRmax + 1;
+constexpr int kScChunks = (kScBox + kScChunk - 1) / kScChunk;
+constexpr int kScRow = kScChunks * kScChunk;  // cells of a grid row, whole chunks
+struct SGrid {
+    int dx0, n, dy0, m;  // first displacement and extent in dx and dy
+    bool dense;          // every near row has its own cell, at least half of them taken
+    bool all_near;       // no row lies beyond the halo
+};
 
-    const TileIdx ti = tile_of(xcd_tile(blockIdx.x, gridDim.x), ntw, nth, G::TH, G::TW);
-    const int64_t HW = static_cast<int64_t>(H) * W;
-    const int64_t BC = static_cast<int64_t>(B) * C;
-    for (int s = threadIdx.x; s < S; s += blockDim.x) wl[s] = to_acc(w[s * BC + ti.bc]);
-    if (MODE == 0)
-        stage_tile<T, A>(st, static_cast<const T*>(src_v) + ti.bc * HW, H, W, ti.h0, ti.w0, G::LH,
-                         G::LW, G::PITCH);
-    else
-        stage_tile<A, A>(st, static_cast<const A*>(src_v) + ti.bc * HW, H, W, ti.h0, ti.w0, G::LH,
-                         G::LW, G::PITCH);
-    stage_shifts(shl, shifts, S, cols, H, W, false);  // ends with a barrier
-
-    const int tx = threadIdx.x % TPR;
-    const int ty = threadIdx.x / TPR;
-    const int h = ti.h0 + ty;
-    const LanePix<VEC, TPR> px = lane_pixels<VEC, TPR>(h, ti.w0, tx, H, W);
-    const int lc = (ty + kRmax) * G::PITCH + tx + kRmax;  // pixel k at lc + k*TPR
-    constexpr int sgn = MODE == 0 ? 1 : -1;
-
-    A u[VEC];
-#pragma unroll
-    for (int k = 0; k < VEC; ++k) u[k] = A(0);
-    A z = A(0);
-    for (int s = 0; s < S; ++s) {
-        const ShiftRec r = read_shift(shl, s);
-        const A ws = wl[s];
-        z += ws;
-        if (shift_in_lds(r)) {
-            const A* sr = st + lc + sgn * (r.dx * G::PITCH + r.dy);
-#pragma unroll
-            for (int k = 0; k < VEC; ++k) u[k] = fma_acc(ws, sr[k * TPR], u[k]);
-        } else {
-            int hh = MODE == 0 ? h + r.dxm : h - r.dxm;
-            hh = MODE == 0 ? (hh >= H ? hh - H : hh) : (hh < 0 ? hh + H : hh);
-#pragma unroll
-            for (int k = 0; k < VEC; ++k) {
-                if (!px.act[k]) continue;
-                const int wq = ti.w0 + tx + k * TPR;
-                int ww = MODE == 0 ? wq + r.dym : wq - r.dym;
-                ww = MODE == 0 ? (ww >= W ? ww - W : ww) : (ww < 0 ? ww + W : ww);
-                const uint32_t i = static_cast<uint32_t>(hh) * W + ww;
-                const A v = MODE == 0 ? to_acc(static_cast<const T*>(src_v)[ti.bc * HW + i])
-                                      : static_cast<const A*>(src_v)[ti.bc * HW + i];
-                u[k] = fma_acc(ws, v, u[k]);
-            }
-        }
+// Builds the grid in `cell` (m rows of kScRow; -1: empty) from the staged
+// table; ends with a barrier.
+template <int SGN>
+__device__ __forceinline__ SGrid stage_grid(const int4* shl, int S, int* cell) {
+    const int lane = threadIdx.x & 63;
+    for (int i = threadIdx.x; i < kScBox * kScRow; i += blockDim.x) cell[i] = -1;
+    // extent and number of the near rows, by every wave for itself
+    int lox = kRmax, hix = -kRmax, loy = kRmax, hiy = -kRmax, near = 0;
+    for (int s = lane; s < S; s += 64) {
+        const int dx = SGN * shl[s].x, dy = SGN * shl[s].y;
+        if (dx < -kRmax || dx > kRmax || dy < -kRmax || dy > kRmax) continue;
+        lox = min(lox, dx);
+        hix = max(hix, dx);
+        loy = min(loy, dy);
+        hiy = max(hiy, dy);
+        ++near;
     }
 #pragma unroll
-    for (int k = 0; k < VEC; ++k) {
-        if (!px.act[k]) continue;
-        const int64_t o = ti.bc * HW + px.own[k];
-        if (MODE == 0) {
-            static_cast<A*>(out0)[o] = u[k];
-            out1[o] = z;
-        } else {
-            static_cast<T*>(out0)[o] = from_acc<T>(u[k]);
-        }
+    for (int o = 32; o > 0; o >>= 1) {
+        lox = min(lox, __shfl_xor(lox, o, 64));
+        hix = max(hix, __shfl_xor(hix, o, 64));
+        loy = min(loy, __shfl_xor(loy, o, 64));
+        hiy = max(hiy, __shfl_xor(hiy, o, 64));
+        near += __shfl_xor(near, o, 64);
     }
+    SGrid g;
+    g.dx0 = __builtin_amdgcn_readfirstlane(lox);
+    g.dy0 = __builtin_amdgcn_readfirstlane(loy);
+    g.n = __builtin_amdgcn_readfirstlane(hix) - g.dx0 + 1;
+    g.m = __builtin_amdgcn_readfirstlane(hiy) - g.dy0 + 1;
+    const int count = __builtin_amdgcn_readfirstlane(near);
+    g.dense = count > 0 && 2 * count >= g.n * g.m;
+    g.all_near = count == S;
+    __syncthreads();
+    if (g.dense) {
+        for (int s = threadIdx.x; s < S; s += blockDim.x) {
+            const int dx = SGN * shl[s].x, dy = SGN * shl[s].y;
+            if (dx < -kRmax || dx > kRmax || dy < -kRmax || dy > kRmax) continue;
+            atomicMax(&cell[(dy - g.dy0) * kScRow + dx - g.dx0], s);
+        }
+        __syncthreads();
+        int taken = 0;  // a repeated row: fewer cells taken than rows
+        for (int i = lane; i < g.m * kScRow; i += 64) taken += cell[i] >= 0;
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) taken += __shfl_xor(taken, o, 64);
+        g.dense = __builtin_amdgcn_readfirstlane(taken) == count;
+    }
+    return g;
+}
+
+// The weights of the grid's cells (0 in an empty one) and, per chunk of four
+// neighbouring dx, which of them are taken.
+template <typename A>
+__device__ __forceinline__ void stage_grid_weights(const SGrid& g, const int* cell, const A* wl,
+                                                   A* kw, int* mask) {
+    for (int i = threadIdx.x; i < g.m * kScRow; i += blockDim.x)
+        kw[i] = cell[i] >= 0 ? wl[cell[i]] : A(0);
+    for (int i = threadIdx.x; i < g.m * kScChunks; i += blockDim.x) {
+        int m = 0;
+#pragma unroll
+        for (int j = 0; j < kScChunk; ++j) m |= cell[i * kScChunk + j] >= 0 ? 1 << j : 0;
+        mask[i] = m;
+    }
+    __syncthreads();
 }
 
 // Sum over the 64 lanes of a wave, returned uniform (in every lane).
@@ -126,93 +150,263 @@ __device__ __forceinline__ double wave_sum(double v) {
     return v;
 }
 
+// The value at (h + dx, w + dy) of a plane, for a row beyond the halo.
+__device__ __forceinline__ uint32_t far_offset(int h, int w, int dxm, int dym, int H, int W) {
+    int hh = h + dxm;
+    hh -= hh >= H ? H : 0;
+    int ww = w + dym;
+    ww -= ww >= W ? W : 0;
+    return static_cast<uint32_t>(hh) * W + ww;
+}
+
+// MODE 0: forward (src = x, writes U and Z);  MODE 1: gx (src = gU).
+template <typename T, int MODE>
+__global__ __launch_bounds__(kScThreads) void scalar_tile_kernel(
+    const void* __restrict__ src_v, const T* __restrict__ w, const int64_t* __restrict__ shifts,
+    int cols, int S, int B, int C, int H, int W, int ntw, int nth, void* __restrict__ out0,
+    acc_t<T>* __restrict__ out1) {
+    using A = acc_t<T>;
+    using Src = std::conditional_t<MODE == 0, T, A>;
+    constexpr int SGN = MODE == 0 ? 1 : -1;
+    constexpr int P = kScP, CH = kScChunk;
+    extern __shared__ __align__(16) unsigned char smem[];
+    int4* shl = reinterpret_cast<int4*>(smem);
+    A* kw = reinterpret_cast<A*>(smem + shift_lds_bytes(S));
+    A* st = kw + kScBox * kScRow;
+    A* wl = st + kScTile;
+    int* cell = reinterpret_cast<int*>(wl + S);
+    int* mask = cell + kScBox * kScRow;
+
+    const TileIdx ti = tile_of(xcd_tile(blockIdx.x, gridDim.x), ntw, nth, kScTH, kScTW);
+    const int64_t HW = static_cast<int64_t>(H) * W;
+    const int64_t BC = static_cast<int64_t>(B) * C;
+    const Src* src = static_cast<const Src*>(src_v) + ti.bc * HW;
+    for (int s = threadIdx.x; s < S; s += blockDim.x) wl[s] = to_acc(w[s * BC + ti.bc]);
+    stage_tile<Src, A>(st, src, H, W, ti.h0, ti.w0, kScLH, kScPitch, kScPitch);
+    stage_shifts(shl, shifts, S, cols, H, W, false);  // ends with a barrier
+    const SGrid g = stage_grid<SGN>(shl, S, cell);
+
+    const int col = threadIdx.x & 63;
+    const int r0 = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) * P;
+    const A* own = st + (r0 + kRmax) * kScPitch + col + kRmax;  // pixel i at own + i * pitch
+    A u[P];
+#pragma unroll
+    for (int i = 0; i < P; ++i) u[i] = A(0);
+    A z = A(0);  // lane sums of the weights, then the wave's
+    if (MODE == 0) {
+        for (int s = col; s < S; s += 64) z += wl[s];
+        z = wave_sum(z);
+    }
+
+    if (g.dense) {
+        stage_grid_weights<A>(g, cell, wl, kw, mask);
+        const int nch = (g.n + CH - 1) / CH;
+        // the next chunk's mask and weights are read one chunk ahead
+        int mn = mask[0];
+        A wn[CH];
+        load_out<A, CH>(kw, wn);
+        for (int dyi = 0; dyi < g.m; ++dyi) {
+            const A* cv = own + g.dx0 * kScPitch + g.dy0 + dyi;
+            for (int c = 0; c < nch; ++c, cv += CH * kScPitch) {
+                const int m = __builtin_amdgcn_readfirstlane(mn);
+                A v[P + CH - 1], ws[CH];
+#pragma unroll
+                for (int i = 0; i < P + CH - 1; ++i) v[i] = cv[i * kScPitch];
+#pragma unroll
+                for (int j = 0; j < CH; ++j) ws[j] = wn[j];
+                const int next = c + 1 < nch ? dyi * kScChunks + c + 1
+                                             : min(dyi + 1, g.m - 1) * kScChunks;
+                mn = mask[next];
+                load_out<A, CH>(kw + next * CH, wn);
+                // an empty cell is skipped, not weighted by 0 (0 x inf)
+                if (m == (1 << CH) - 1) {
+#pragma unroll
+                    for (int j = 0; j < CH; ++j)
+#pragma unroll
+                        for (int i = 0; i < P; ++i) u[i] = fma_acc(ws[j], v[i + j], u[i]);
+                } else {
+#pragma unroll
+                    for (int j = 0; j < CH; ++j)
+                        if (m & (1 << j))
+#pragma unroll
+                            for (int i = 0; i < P; ++i) u[i] = fma_acc(ws[j], v[i + j], u[i]);
+                }
+            }
+        }
+    }
+    const int w_px = ti.w0 + col;
+    const bool wact = w_px < W;
+    for (int s = 0; s < S && !(g.dense && g.all_near); ++s) {
+        const ShiftRec r = read_shift(shl, s);
+        if (shift_in_lds(r)) {
+            if (g.dense) continue;
+            const A ws = wl[s];
+            const A* sr = own + SGN * (r.dx * kScPitch + r.dy);
+#pragma unroll
+            for (int i = 0; i < P; ++i) u[i] = fma_acc(ws, sr[i * kScPitch], u[i]);
+        } else {
+            const A ws = wl[s];
+            // (p - s) mod = (p + (H - dx mod H)) mod
+            const int dxm = MODE == 0 ? r.dxm : (r.dxm ? H - r.dxm : 0);
+            const int dym = MODE == 0 ? r.dym : (r.dym ? W - r.dym : 0);
+#pragma unroll
+            for (int i = 0; i < P; ++i) {
+                const int h = ti.h0 + r0 + i;
+                if (wact && h < H)
+                    u[i] = fma_acc(ws, to_acc(src[far_offset(h, w_px, dxm, dym, H, W)]), u[i]);
+            }
+        }
+    }
+    if (!wact) return;
+#pragma unroll
+    for (int i = 0; i < P; ++i) {
+        const int h = ti.h0 + r0 + i;
+        if (h >= H) continue;
+        const int64_t o = ti.bc * HW + static_cast<uint32_t>(h) * static_cast<uint32_t>(W) + w_px;
+        if (MODE == 0) {
+            static_cast<A*>(out0)[o] = u[i];
+            out1[o] = z;
+        } else {
+            static_cast<T*>(out0)[o] = from_acc<T>(u[i]);
+        }
+    }
+}
+
+// The wave sums of four values at once, lane 15 + 16 j of the result holding
+// that of v[j]: the halves of two values, then the 16-lane rows of two such
+// pairs, trade places in one instruction each (permlane32_swap,
+// permlane16_swap), so four sums take ten instructions instead of 28.
+__device__ __forceinline__ void swap_add(float& a, float b, bool rows16) {
+    const auto r = rows16 ? __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b),
+                                                             false, false)
+                          : __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b),
+                                                             false, false);
+    a = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+__device__ __forceinline__ float wave_sum4(float (&v)[4]) {
+    swap_add(v[0], v[2], false);
+    swap_add(v[1], v[3], false);
+    swap_add(v[0], v[1], true);
+    float t = dpp_add<0x111, 0xf>(v[0]);
+    t = dpp_add<0x112, 0xf>(t);
+    t = dpp_add<0x114, 0xf>(t);
+    return dpp_add<0x118, 0xf>(t);
+}
+__device__ __forceinline__ double wave_sum4(double (&v)[4]) {
+    const int row = (threadIdx.x & 63) >> 4;
+    double t = 0.0;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        const double w = wave_sum(v[j]);
+        t = row == j ? w : t;
+    }
+    return t;
+}
+
 // gw partials of one tile: part[(s*BC + bc)*ntp + tile] =
 //   sum_{p in tile} gU[p] x[(p+s) mod] + gZ[p]
-// Shifts go in blocks of kScGwBlk: each wave leaves its sums in LDS, then
-// kScGwBlk lanes add the waves in order.
-constexpr int kScGwBlk = 8;
-constexpr int kScWaves = kScThreads / 64;
-
+// Every wave holds the whole tile's gU (a lane its column, 32 rows) and takes
+// its share of the shifts: chunks of four neighbouring dx of the grid, or
+// single rows.  A chunk reads the column values of 16 rows at a time.
 template <typename T>
 __global__ __launch_bounds__(kScThreads) void scalar_gw_tile_kernel(
     const T* __restrict__ x, const acc_t<T>* __restrict__ gU, const acc_t<T>* __restrict__ gZ,
     const int64_t* __restrict__ shifts, int cols, int S, int B, int C, int H, int W, int ntw,
     int nth, acc_t<T>* __restrict__ part) {
     using A = acc_t<T>;
-    using G = ScG;
-    constexpr int VEC = kScVec, TPR = kScTpr;
+    constexpr int CH = kScChunk, TH = kScTH, SUB = 16;
     extern __shared__ __align__(16) unsigned char smem[];
     int4* shl = reinterpret_cast<int4*>(smem);
     A* xt = reinterpret_cast<A*>(smem + shift_lds_bytes(S));
-    A* red = xt + G::TILE;  // [kScWaves][kScGwBlk + 1]
+    A* gzw = xt + kScTile;  // the waves' shares of the tile's gZ
+    int* cell = reinterpret_cast<int*>(gzw + kScWaves);
 
     // plain tile order: the partial index is the tile's position in its plane
     const int64_t ntp = static_cast<int64_t>(ntw) * nth;
-    const TileIdx ti = tile_of(blockIdx.x, ntw, nth, G::TH, G::TW);
+    const TileIdx ti = tile_of(blockIdx.x, ntw, nth, kScTH, kScTW);
     const int64_t tile = blockIdx.x - ti.bc * ntp;
     const int64_t HW = static_cast<int64_t>(H) * W;
     const int64_t BC = static_cast<int64_t>(B) * C;
     const T* xp = x + ti.bc * HW;
-    stage_tile<T, A>(xt, xp, H, W, ti.h0, ti.w0, G::LH, G::LW, G::PITCH);
-    stage_shifts(shl, shifts, S, cols, H, W, false);  // ends with a barrier
+    const int col = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int w_px = ti.w0 + col;
+    const bool wact = w_px < W;
 
-    const int tx = threadIdx.x % TPR;
-    const int ty = threadIdx.x / TPR;
-    const int h = ti.h0 + ty;
-    const LanePix<VEC, TPR> px = lane_pixels<VEC, TPR>(h, ti.w0, tx, H, W);
-    const int lc = (ty + kRmax) * G::PITCH + tx + kRmax;
-    const int wave = threadIdx.x / 64;
-    const int lane = threadIdx.x & 63;
-
-    A gu[VEC];
+    constexpr int ZR = TH / kScWaves;  // rows of gZ a wave adds up
+    A gu[TH];
     A gz = A(0);
 #pragma unroll
-    for (int k = 0; k < VEC; ++k) {
-        gu[k] = px.act[k] ? gU[ti.bc * HW + px.own[k]] : A(0);
-        gz += px.act[k] ? gZ[ti.bc * HW + px.own[k]] : A(0);
+    for (int i = 0; i < TH; ++i) {
+        const bool act = wact && ti.h0 + i < H;
+        const int64_t o = ti.bc * HW + (act ? static_cast<uint32_t>(ti.h0 + i) *
+                                                      static_cast<uint32_t>(W) + w_px
+                                            : 0u);
+        gu[i] = act ? gU[o] : A(0);
     }
-    // sum of gZ over the tile (added to every shift's partial)
+#pragma unroll
+    for (int i = 0; i < ZR; ++i) {
+        const int h = ti.h0 + wave * ZR + i;
+        const bool act = wact && h < H;
+        const int64_t o = ti.bc * HW + (act ? static_cast<uint32_t>(h) *
+                                                      static_cast<uint32_t>(W) + w_px
+                                            : 0u);
+        gz += act ? gZ[o] : A(0);
+    }
     gz = wave_sum(gz);
-    if (lane == 0) red[wave * (kScGwBlk + 1) + kScGwBlk] = gz;
-    __syncthreads();
-    A gz_tile = A(0);
+    if (col == 0) gzw[wave] = gz;
+    stage_tile<T, A>(xt, xp, H, W, ti.h0, ti.w0, kScLH, kScPitch, kScPitch);
+    stage_shifts(shl, shifts, S, cols, H, W, false);  // ends with a barrier
+    const SGrid g = stage_grid<1>(shl, S, cell);
+    A gz_tile = A(0);  // the sum of gZ over the tile, part of every shift's sum
 #pragma unroll
-    for (int i = 0; i < kScWaves; ++i) gz_tile += red[i * (kScGwBlk + 1) + kScGwBlk];
+    for (int i = 0; i < kScWaves; ++i) gz_tile += gzw[i];
+    const A* own = xt + kRmax * kScPitch + col + kRmax;
 
-    for (int s0 = 0; s0 < S; s0 += kScGwBlk) {
+    if (g.dense) {
+        const int nch = (g.n + CH - 1) / CH;
+        for (int job = wave; job < g.m * nch; job += kScWaves) {
+            const int dyi = job / nch, dxi = (job - dyi * nch) * CH;
+            const A* cv = own + (g.dx0 + dxi) * kScPitch + g.dy0 + dyi;
+            A acc[CH];
 #pragma unroll
-        for (int j = 0; j < kScGwBlk; ++j) {
-            const int s = s0 + j;
-            if (s >= S) break;
-            const ShiftRec r = read_shift(shl, s);
-            A acc = A(0);
-            if (shift_in_lds(r)) {
-                const A* sr = xt + lc + r.dx * G::PITCH + r.dy;
+            for (int j = 0; j < CH; ++j) acc[j] = A(0);
 #pragma unroll
-                for (int k = 0; k < VEC; ++k) acc = fma_acc(gu[k], sr[k * TPR], acc);
-            } else {
-                int hh = h + r.dxm;
-                hh -= hh >= H ? H : 0;
+            for (int i0 = 0; i0 < TH; i0 += SUB) {
+                A v[SUB + CH - 1];
 #pragma unroll
-                for (int k = 0; k < VEC; ++k) {
-                    if (!px.act[k]) continue;
-                    int ww = ti.w0 + tx + k * TPR + r.dym;
-                    ww -= ww >= W ? W : 0;
-                    acc = fma_acc(gu[k], to_acc(xp[static_cast<uint32_t>(hh) * W + ww]), acc);
-                }
+                for (int i = 0; i < SUB + CH - 1; ++i) v[i] = cv[(i0 + i) * kScPitch];
+#pragma unroll
+                for (int i = 0; i < SUB; ++i)
+#pragma unroll
+                    for (int j = 0; j < CH; ++j) acc[j] = fma_acc(gu[i0 + i], v[i + j], acc[j]);
             }
-            acc = wave_sum(acc);
-            if (lane == 0) red[wave * (kScGwBlk + 1) + j] = acc;
+            static_assert(CH == 4, "one value per 16-lane row");
+            const int s = cell[dyi * kScRow + dxi + (col >> 4)];  // -1 beyond the box
+            const A t = wave_sum4(acc) + gz_tile;
+            if ((col & 15) == 15 && s >= 0)
+                part[(static_cast<int64_t>(s) * BC + ti.bc) * ntp + tile] = t;
         }
-        __syncthreads();
-        if (threadIdx.x < kScGwBlk && s0 + threadIdx.x < S) {
-            A t = A(0);
+    }
+    for (int s = wave; s < S && !(g.dense && g.all_near); s += kScWaves) {
+        const ShiftRec r = read_shift(shl, s);
+        A acc = A(0);
+        if (shift_in_lds(r)) {
+            if (g.dense) continue;
+            const A* sr = own + r.dx * kScPitch + r.dy;
 #pragma unroll
-            for (int i = 0; i < kScWaves; ++i) t += red[i * (kScGwBlk + 1) + threadIdx.x];
-            const int64_t sbc = static_cast<int64_t>(s0 + threadIdx.x) * BC + ti.bc;
-            part[sbc * ntp + tile] = t + gz_tile;
+            for (int i = 0; i < TH; ++i) acc = fma_acc(gu[i], sr[i * kScPitch], acc);
+        } else {
+            const int rows = wact ? min(TH, H - ti.h0) : 0;
+            for (int i = 0; i < rows; ++i) {
+                const int h = ti.h0 + i;
+                const uint32_t o = static_cast<uint32_t>(h) * static_cast<uint32_t>(W) + w_px;
+                acc = fma_acc(gU[ti.bc * HW + o],
+                              to_acc(xp[far_offset(h, w_px, r.dxm, r.dym, H, W)]), acc);
+            }
         }
-        __syncthreads();
+        const A t = wave_sum(acc) + gz_tile;
+        if (col == 0) part[(static_cast<int64_t>(s) * BC + ti.bc) * ntp + tile] = t;
     }
 }
 
@@ -229,8 +423,8 @@ __global__ __launch_bounds__(256) void scalar_gw_final_kernel(const acc_t<T>* __
 }
 
 static void sc_tiles(int H, int W, int* ntw, int* nth) {
-    *ntw = static_cast<int>(nsh_host::ceil_div(W, ScG::TW));
-    *nth = static_cast<int>(nsh_host::ceil_div(H, ScG::TH));
+    *ntw = static_cast<int>(nsh_host::ceil_div(W, kScTW));
+    *nth = static_cast<int>(nsh_host::ceil_div(H, kScTH));
 }
 
 template <typename T, int MODE>
@@ -240,8 +434,9 @@ static int s_tile(const void* src, const void* w, const int64_t* sh, int cols, i
     int ntw, nth;
     sc_tiles(H, W, &ntw, &nth);
     const int64_t tiles = static_cast<int64_t>(B) * C * ntw * nth;
-    const size_t lds = shift_lds_bytes(S) + static_cast<size_t>(S) * sizeof(A) +
-                       static_cast<size_t>(ScG::TILE) * sizeof(A);
+    const size_t lds = shift_lds_bytes(S) +
+                       (kScBox * kScRow + static_cast<size_t>(kScTile) + S) * sizeof(A) +
+                       kScBox * (kScRow + kScChunks) * sizeof(int);
     hipLaunchKernelGGL((scalar_tile_kernel<T, MODE>), dim3(static_cast<unsigned>(tiles)),
                        dim3(kScThreads), lds, st, src, static_cast<const T*>(w), sh, cols, S, B, C,
                        H, W, ntw, nth, out0, static_cast<A*>(out1));
@@ -264,8 +459,8 @@ static int s_gw(const void* x, const void* gU, const void* gZ, const int64_t* sh
     sc_tiles(H, W, &ntw, &nth);
     const int nsplit = ntw * nth;
     const int64_t tiles = static_cast<int64_t>(B) * C * nsplit;
-    const size_t lds = shift_lds_bytes(S) +
-                       (static_cast<size_t>(ScG::TILE) + kScWaves * (kScGwBlk + 1)) * sizeof(A);
+    const size_t lds = shift_lds_bytes(S) + (kScTile + kScWaves) * sizeof(A) +
+                       kScBox * kScRow * sizeof(int);
     hipLaunchKernelGGL((scalar_gw_tile_kernel<T>), dim3(static_cast<unsigned>(tiles)),
                        dim3(kScThreads), lds, st, static_cast<const T*>(x),
                        static_cast<const A*>(gU), static_cast<const A*>(gZ), sh, cols, S, B, C, H,
