@@ -91,8 +91,9 @@ extern "C" {
  * tables up to R = 22, S = 1013, the largest the 1 <= S <= 1024 contract
  * admits).  NSH_WIDE_HALO is ignored when both are set. */
 #define NSH_WIDER_HALO 0x800
-#define NSH_DTYPE_FLAGS \
-    (NSH_SHIFT_CODES | NSH_SHARED_WEIGHTS | NSH_WIDE_HALO | NSH_WIDER_HALO | NSH_NARROW_HALO)
+#define NSH_DTYPE_FLAGS                                                                     \
+    (NSH_SHIFT_CODES | NSH_SHARED_WEIGHTS | NSH_WIDE_HALO | NSH_WIDER_HALO | NSH_NARROW_HALO | \
+     NSH_PERIODIC_INVERSE | NSH_BOX_FORWARD)
 
 /* Flag ORed into `dtype`: a hint that every shift of the table has
  * max(|dx|, |dy|) <= 6, for two passes that then stage a 6-pixel border
@@ -109,6 +110,16 @@ extern "C" {
  * launch, so any table gives the same results with or without it.  An
  * extension with no counterpart in the reference. */
 #define NSH_NARROW_HALO 0x1000
+
+/* Flags ORed into `dtype` of the accumulate_uz and normalized_accumulate_uz
+ * calls: the row codes of NSH_SHIFT_CODES for every row at once, from the
+ * reference's has_inverse flag (no rewritten table): NSH_PERIODIC_INVERSE
+ * takes the mirror of every has_inverse row circularly (code 2 in place of
+ * 1), NSH_BOX_FORWARD drops the forward term of every row where (h + dx,
+ * w + dy) leaves the image (code bit 2).  Ignored with NSH_SHIFT_CODES.
+ * Extensions with no counterpart in the reference. */
+#define NSH_PERIODIC_INVERSE 0x2000
+#define NSH_BOX_FORWARD 0x4000
 
 /* Return codes. */
 #define NSH_OK 0

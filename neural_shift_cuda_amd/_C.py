@@ -17,6 +17,8 @@ trishitmg/neural_shift_cuda), so the guards in ``ops.py`` and
   (default False: the reference's has_inverse flag, nonzero = mirror): True
   marks a table whose third column holds the library's row codes
   (``NSH_SHIFT_CODES``: circular mirrors, in-kernel forward box);
+* a keyword ``rules`` (default 0): NSH_PERIODIC_INVERSE and NSH_BOX_FORWARD,
+  the same extensions for every row of a has_inverse table;
 * and a keyword ``shared_weights`` (default False): True takes weights of
   shape (S*B, 1, H, W) used for every channel (``NSH_SHARED_WEIGHTS``); the
   weight gradient then still comes back per channel, (S*B, C, H, W).
@@ -47,6 +49,8 @@ NSH_SHARED_WEIGHTS = 0x200
 NSH_WIDE_HALO = 0x400
 NSH_WIDER_HALO = 0x800
 NSH_NARROW_HALO = 0x1000  # Metropolis backward: every shift within 6 pixels
+NSH_PERIODIC_INVERSE = 0x2000  # every mirror of a has_inverse table circular
+NSH_BOX_FORWARD = 0x4000  # every forward term dropped where it leaves the image
 NSH_ERR_UNSUPPORTED = 3
 
 _SIGS = {
@@ -250,8 +254,9 @@ def _check_pair(op: str, x: torch.Tensor, weights: torch.Tensor, shifts: torch.T
     return sh, B, C, H, W, S
 
 
-def _flags(row_codes: bool, shared: bool) -> int:
-    return (NSH_SHIFT_CODES if row_codes else 0) | (NSH_SHARED_WEIGHTS if shared else 0)
+def _flags(row_codes: bool, shared: bool, rules: int) -> int:
+    return ((NSH_SHIFT_CODES if row_codes else 0) | (NSH_SHARED_WEIGHTS if shared else 0)
+            | (rules & (NSH_PERIODIC_INVERSE | NSH_BOX_FORWARD)))
 
 
 # Radius of a shift table, per tensor object and version: id -> (weakref,
@@ -326,7 +331,8 @@ def _band_args(band) -> tuple:
 
 def accumulate_uz_forward(x: torch.Tensor, weights: torch.Tensor,
                           shifts: torch.Tensor, *, row_codes: bool = False,
-                          shared_weights: bool = False, band=None) -> List[torch.Tensor]:
+                          shared_weights: bool = False, band=None,
+                          rules: int = 0) -> List[torch.Tensor]:
     """[U, Z] in the accumulator dtype (shift_ops.cpp:160-192).  `band`
     (row_origin, image_height): x holds one horizontal band of a larger
     image, local row h being image row (row_origin + h) mod image_height
@@ -334,7 +340,8 @@ def accumulate_uz_forward(x: torch.Tensor, weights: torch.Tensor,
     sh, B, C, H, W, S = _check_pair("accumulate_uz", x, weights, shifts,
                                     "weights shape must be (S*B, C, H, W)", shared_weights)
     acc = _acc_dtype(x.dtype)
-    code = _code(x, "accumulate_uz_fwd") | _flags(row_codes, shared_weights) | _halo_flag(shifts)
+    code = (_code(x, "accumulate_uz_fwd") | _flags(row_codes, shared_weights, rules)
+            | _halo_flag(shifts))
     U = torch.empty(x.shape, dtype=acc, device=x.device)
     Z = torch.empty(x.shape, dtype=acc, device=x.device)
     ws, nws = _workspace(S, B, C, H, W, code, False, x.device)
@@ -368,7 +375,7 @@ def _grad_in(g: torch.Tensor, like: torch.Tensor, acc: torch.dtype, name: str) -
 def accumulate_uz_backward(x: torch.Tensor, weights: torch.Tensor, grad_U: torch.Tensor,
                            grad_Z: torch.Tensor, shifts: torch.Tensor, *,
                            row_codes: bool = False, shared_weights: bool = False,
-                           band=None) -> List[torch.Tensor]:
+                           band=None, rules: int = 0) -> List[torch.Tensor]:
     """[grad_x, grad_w] in the input dtype (shift_ops.cpp:194-212); grad_w
     is per channel, (S*B, C, H, W), also for shared weights.  `band` as in
     accumulate_uz_forward."""
@@ -377,7 +384,8 @@ def accumulate_uz_backward(x: torch.Tensor, weights: torch.Tensor, grad_U: torch
     acc = _acc_dtype(x.dtype)
     gU = _grad_in(grad_U, x, acc, "grad_U")
     gZ = _grad_in(grad_Z, x, acc, "grad_Z")
-    code = _code(x, "accumulate_uz_bwd") | _flags(row_codes, shared_weights) | _halo_flag(shifts)
+    code = (_code(x, "accumulate_uz_bwd") | _flags(row_codes, shared_weights, rules)
+            | _halo_flag(shifts))
     gx = torch.empty_like(x)
     gw = torch.empty((S * B, C, H, W), dtype=weights.dtype, device=weights.device)
     ws, nws = _workspace(S, B, C, H, W, code, True, x.device)
@@ -397,8 +405,8 @@ def accumulate_uz_backward(x: torch.Tensor, weights: torch.Tensor, grad_U: torch
 def normalized_accumulate_uz_forward(x: torch.Tensor, weights: torch.Tensor, shifts: torch.Tensor,
                                      log_weights: bool, *, row_codes: bool = False,
                                      shared_weights: bool = False,
-                                     weights_ok: Optional[torch.Tensor] = None
-                                     ) -> List[torch.Tensor]:
+                                     weights_ok: Optional[torch.Tensor] = None,
+                                     rules: int = 0) -> List[torch.Tensor]:
     """[D, log_C] in the accumulator dtype (shift_ops.cpp:218-252).
     `weights_ok`: a one-element int32 tensor holding a nonzero value, set to 0
     when a weight breaks the op's contract
@@ -407,7 +415,7 @@ def normalized_accumulate_uz_forward(x: torch.Tensor, weights: torch.Tensor, shi
                                     "normalized_accumulate_uz: weights must be (S*B, C, H, W)",
                                     shared_weights)
     acc = _acc_dtype(x.dtype)
-    code = _code(x, "normalized_accumulate_uz_fwd") | _flags(row_codes, shared_weights)
+    code = _code(x, "normalized_accumulate_uz_fwd") | _flags(row_codes, shared_weights, rules)
     if weights_ok is not None:
         _check(weights_ok.device == x.device and weights_ok.dtype == torch.int32
                and weights_ok.numel() == 1,
@@ -424,7 +432,7 @@ def normalized_accumulate_uz_forward(x: torch.Tensor, weights: torch.Tensor, shi
 
 def normalized_accumulate_uz_forward_mixed(x: torch.Tensor, head_weights: torch.Tensor,
                                            head_mix: torch.Tensor, shifts: torch.Tensor, *,
-                                           row_codes: bool = False
+                                           row_codes: bool = False, rules: int = 0
                                            ) -> Optional[List[torch.Tensor]]:
     """[D, log_C] of the positive-weight forward whose channel-c weights are
     sum_j head_mix[c, j] * head_weights[:, j], formed in the kernels' weight
@@ -451,7 +459,7 @@ def normalized_accumulate_uz_forward_mixed(x: torch.Tensor, head_weights: torch.
            f"{op}: head_mix must be (C, heads)")
     acc = _acc_dtype(x.dtype)
     mix = head_mix.detach().to(device=x.device, dtype=acc).contiguous()
-    code = _code(x, op) | _flags(row_codes, False)
+    code = _code(x, op) | _flags(row_codes, False, rules)
     D = torch.empty(x.shape, dtype=acc, device=x.device)
     L = torch.empty(x.shape, dtype=acc, device=x.device)
     ws, nws = _norm_workspace(S, B, C, H, W, code, False, x.device)
@@ -533,7 +541,8 @@ def normalized_accumulate_uz_backward(x: torch.Tensor, weights: torch.Tensor, D:
                                       log_C: torch.Tensor, grad_D: torch.Tensor,
                                       grad_log_C: torch.Tensor, shifts: torch.Tensor,
                                       log_weights: bool, *, row_codes: bool = False,
-                                      shared_weights: bool = False) -> List[torch.Tensor]:
+                                      shared_weights: bool = False,
+                                      rules: int = 0) -> List[torch.Tensor]:
     """[grad_x, grad_w] (shift_ops.cpp:254-280); grad_w is per channel,
     (S*B, C, H, W), also for shared weights."""
     sh, B, C, H, W, S = _check_pair("normalized_accumulate_uz", x, weights, shifts,
@@ -546,7 +555,7 @@ def normalized_accumulate_uz_backward(x: torch.Tensor, weights: torch.Tensor, D:
     gL = _grad_in(grad_log_C, x, acc, "grad_log_C")
     gx = torch.empty_like(x)
     gw = torch.empty((S * B, C, H, W), dtype=weights.dtype, device=weights.device)
-    code = _code(x, "normalized_accumulate_uz_bwd") | _flags(row_codes, shared_weights)
+    code = _code(x, "normalized_accumulate_uz_bwd") | _flags(row_codes, shared_weights, rules)
     if x.dtype == torch.float64:
         code |= _narrow_halo_flag(sh)
     ws, nws = _norm_workspace(S, B, C, H, W, code, True, x.device)

@@ -248,7 +248,7 @@ __global__ __launch_bounds__(kTPR * ROWS) void accumulate_uz_fwd_kernel(
     int4* shl = reinterpret_cast<int4*>(smem);
     A* xt = reinterpret_cast<A*>(smem + shift_lds_bytes(S));
     const TileIdx ti = tile_of(xcd_tile(blockIdx.x, gridDim.x), ntw, nth, G::TH, G::TW, order, band);
-    stage_shifts(shl, shifts, S, 3, H, W, (codes & kCodesRows) != 0);
+    stage_shifts(shl, shifts, S, 3, H, W, codes);
     stage_tile<T, A>(xt, x + ti.bc * (static_cast<int64_t>(H) * W), H, W, ti.h0, ti.w0, G::LH,
                      G::LW, G::PITCH);
     __syncthreads();
@@ -428,7 +428,7 @@ __global__ __launch_bounds__(kTPR * ROWS) void accumulate_uz_bwd_kernel(
     A* zt = ut + G::TILE;
     const TileIdx ti = tile_of(xcd_tile(blockIdx.x, gridDim.x), ntw, nth, G::TH, G::TW, order, band);
     const int64_t off = ti.bc * (static_cast<int64_t>(H) * W);
-    stage_shifts(shl, shifts, S, 3, H, W, (codes & kCodesRows) != 0);
+    stage_shifts(shl, shifts, S, 3, H, W, codes);
     stage_tile<T, A>(xt, x + off, H, W, ti.h0, ti.w0, G::LH, G::LW, G::PITCH);
     stage_tile<A, A>(ut, gU + off, H, W, ti.h0, ti.w0, G::LH, G::LW, G::PITCH);
     stage_tile<A, A>(zt, gZ + off, H, W, ti.h0, ti.w0, G::LH, G::LW, G::PITCH);
@@ -492,7 +492,7 @@ __device__ __forceinline__ void fwd_scatter_tile(
     const TileIdx ti = tile_of(t, ntw, nth, G::TH, G::TW);
     const int64_t HW = static_cast<int64_t>(H) * W;
 
-    stage_shifts(shl, shifts, S, 3, H, W, (codes & kCodesRows) != 0);
+    stage_shifts(shl, shifts, S, 3, H, W, codes);
     // Every row's x read must come from the LDS tile (|dx|, |dy| <= HALO),
     // and the mirror scatter must reach only adjacent tiles (radius at most
     // the narrowest tile, the partial last one); otherwise the tile runs the
@@ -774,7 +774,7 @@ __global__ __launch_bounds__(TPR * ROWS) void accumulate_uz_bwd_scatter_kernel(
     const int64_t HW = static_cast<int64_t>(H) * W;
     const int64_t off = ti.bc * HW;
 
-    stage_shifts(shl, shifts, S, 3, H, W, (codes & kCodesRows) != 0);
+    stage_shifts(shl, shifts, S, 3, H, W, codes);
     // every row scatters its x term: radius within the halo and at most the
     // narrowest tile (the partial last one), else the gather algorithm
     const int R = table_radius(shl, S, false);

@@ -159,7 +159,7 @@ __global__ __launch_bounds__(kThreads) void normalized_fwd_kernel(
     const TileIdx ti = tile_of(xcd_tile(blockIdx.x, gridDim.x), ntw, nth, G::TH, G::TW);
     const int64_t HW = static_cast<int64_t>(H) * W;
     const T* xp = x + ti.bc * HW;
-    stage_shifts(shl, shifts, S, 3, H, W, (codes & kCodesRows) != 0);
+    stage_shifts(shl, shifts, S, 3, H, W, codes);
     stage_tile<T, A>(xt, xp, H, W, ti.h0, ti.w0, G::LH, G::LW);
     __syncthreads();
 
@@ -270,7 +270,7 @@ __global__ __launch_bounds__(kThreads) void normalized_bwd_kernel(
     const A* Lp = Lg + ti.bc * HW;
     const A* gDp = gDg + ti.bc * HW;
     const A* gLp = gLg + ti.bc * HW;
-    stage_shifts(shl, shifts, S, 3, H, W, (codes & kCodesRows) != 0);
+    stage_shifts(shl, shifts, S, 3, H, W, codes);
     stage_tile<T, A>(xt, xp, H, W, ti.h0, ti.w0, G::LH, G::LW);
     stage_tile_acc<A>(dt, Dp, H, W, ti.h0, ti.w0, G::LH, G::LW);
     stage_tile_acc<A>(lt, Lp, H, W, ti.h0, ti.w0, G::LH, G::LW);
@@ -690,7 +690,7 @@ normalized_fwd_scatter_kernel(const T* __restrict__ x, const T* __restrict__ w,
     const int64_t HW = static_cast<int64_t>(H) * W;
     const int64_t off = ti.bc * HW;
     const T* xp = x + off;
-    stage_shifts(shl, shifts, S, 3, H, W, (codes & kCodesRows) != 0);
+    stage_shifts(shl, shifts, S, 3, H, W, codes);
     stage_tile<T, A>(xt, xp, H, W, ti.h0, ti.w0, G::LH, G::LW, G::PITCH);
     const int R = near_radius(shl, S, true);
     if (blockIdx.x == 0 && threadIdx.x == 0) hdr[0] = R;  // for the fix-up
@@ -1104,7 +1104,7 @@ normalized_bwd_scatter_kernel(const T* __restrict__ x, const T* __restrict__ w,
     const A* Lp = Lg + off;
     const A* gDp = gDg + off;
     const A* gLp = gLg + off;
-    stage_shifts(shl, shifts, S, 3, H, W, (codes & kCodesRows) != 0);
+    stage_shifts(shl, shifts, S, 3, H, W, codes);
     {
         const bool cheap = H >= G::LH && W >= G::LW;
         for (int i = threadIdx.x; i < G::LH * G::LW; i += blockDim.x) {

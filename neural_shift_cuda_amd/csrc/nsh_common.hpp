@@ -254,8 +254,8 @@ __device__ __forceinline__ void load_out(const A* p, A (&v)[VEC]) {
 //   y  = dy clamped likewise
 //   z  = (dx mod H) | has_inv << 31
 //   w  = (dy mod W) | periodic << 31
-// has_inverse column.  Without `codes` it is the reference's flag: nonzero
-// means a mirror term dropped where its source wraps.  With `codes` (the
+// has_inverse column.  Without kCodesRows it is the reference's flag: nonzero
+// means a mirror term dropped where its source wraps.  With it (the
 // caller asked for an extension) a value v in [0, 7] is a row code: bits 0-1
 // select the mirror (0 none, 2 circular: the periodic operator, 1 or 3
 // dropped where its source wraps), bit 2 drops the forward term where
@@ -271,13 +271,19 @@ constexpr int kClamp = 1 << 30;
 // shared by every channel (one plane per (shift, batch) instead of one per
 // (shift, batch, channel): the reference installers' single-head weights,
 // broadcast to the channels).
+// The last two apply a rule to every row of a has_inverse table: its mirrors
+// circular, its forward terms dropped where they leave the image.
 constexpr int kCodesRows = 1;
 constexpr int kCodesSharedW = 2;
+constexpr int kCodesPeriodic = 4;
+constexpr int kCodesBox = 8;
 
 // The kernels' `codes` from the flags a call ORs into its dtype argument.
 __host__ __forceinline__ int dtype_codes(int dtype) {
     return ((dtype & NSH_SHIFT_CODES) ? kCodesRows : 0) |
-           ((dtype & NSH_SHARED_WEIGHTS) ? kCodesSharedW : 0);
+           ((dtype & NSH_SHARED_WEIGHTS) ? kCodesSharedW : 0) |
+           ((dtype & NSH_PERIODIC_INVERSE) ? kCodesPeriodic : 0) |
+           ((dtype & NSH_BOX_FORWARD) ? kCodesBox : 0);
 }
 
 // Weight plane of image (b, c) within one shift block, and the distance
@@ -316,13 +322,17 @@ __host__ __device__ constexpr size_t shift_lds_bytes(int S) {
 }
 
 // Cooperative decode of the whole table into lds[0..S).  Ends with a barrier.
+// The rules of `codes` are applied here: rewriting the table for them took
+// the caller eight small launches per call, about 35 us of GPU time and 45 us
+// on the host.
 __device__ __forceinline__ void stage_shifts(int4* lds, const int64_t* __restrict__ shifts,
-                                             int S, int cols, int H, int W, bool codes) {
+                                             int S, int cols, int H, int W, int codes) {
     for (int s = threadIdx.x; s < S; s += blockDim.x) {
         const int64_t dx = shifts[static_cast<int64_t>(s) * cols + 0];
         const int64_t dy = shifts[static_cast<int64_t>(s) * cols + 1];
         int64_t v = cols >= 3 ? shifts[static_cast<int64_t>(s) * cols + 2] : 0;
-        if (!codes) v = v != 0 ? 1 : 0;
+        if (!(codes & kCodesRows))
+            v = (v != 0 ? ((codes & kCodesPeriodic) ? 2 : 1) : 0) | ((codes & kCodesBox) ? 4 : 0);
         const bool small = v >= 0 && v <= 7;
         const int64_t mir = small ? (v & 3) : 1;
         const bool fbox = small && (v & 4) != 0;

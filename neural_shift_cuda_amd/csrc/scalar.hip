@@ -183,7 +183,7 @@ __global__ __launch_bounds__(kScThreads) void scalar_tile_kernel(
     const Src* src = static_cast<const Src*>(src_v) + ti.bc * HW;
     for (int s = threadIdx.x; s < S; s += blockDim.x) wl[s] = to_acc(w[s * BC + ti.bc]);
     stage_tile<Src, A>(st, src, H, W, ti.h0, ti.w0, kScLH, kScPitch, kScPitch);
-    stage_shifts(shl, shifts, S, cols, H, W, false);  // ends with a barrier
+    stage_shifts(shl, shifts, S, cols, H, W, 0);  // ends with a barrier
     const SGrid g = stage_grid<SGN>(shl, S, cell);
 
     const int col = threadIdx.x & 63;
@@ -356,7 +356,7 @@ __global__ __launch_bounds__(kScThreads) void scalar_gw_tile_kernel(
     gz = wave_sum(gz);
     if (col == 0) gzw[wave] = gz;
     stage_tile<T, A>(xt, xp, H, W, ti.h0, ti.w0, kScLH, kScPitch, kScPitch);
-    stage_shifts(shl, shifts, S, cols, H, W, false);  // ends with a barrier
+    stage_shifts(shl, shifts, S, cols, H, W, 0);  // ends with a barrier
     const SGrid g = stage_grid<1>(shl, S, cell);
     A gz_tile = A(0);  // the sum of gZ over the tile, part of every shift's sum
 #pragma unroll

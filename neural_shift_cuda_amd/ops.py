@@ -91,17 +91,36 @@ def _device_operands(x: torch.Tensor, weights: torch.Tensor
     return x.to(acc), weights.to(acc)
 
 
-def _prep_shifts_for_cuda(shifts: torch.Tensor, device: torch.device) -> torch.Tensor:
+def _prep_shifts_for_cuda(shifts: torch.Tensor, device: torch.device,
+                          radius: bool = False) -> torch.Tensor:
     """(S, 2|3) int64 contiguous table on `device`; values are never narrowed
     (reference ops.py:397-404)."""
     if shifts.dim() != 2 or shifts.size(1) not in (2, 3):
         raise ValueError(f"shifts must be (S, 2) or (S, 3); got {tuple(shifts.shape)}")
     out = shifts.to(device=device, dtype=torch.int64).contiguous()
-    if out is not shifts and not shifts.is_cuda and _HAS_CUDA_EXT:
+    if out is not shifts and _HAS_CUDA_EXT and (radius or not shifts.is_cuda):
         # the kernels' launch shape depends on the table's radius: record it
-        # from the host copy, so that the device copy is never read back
-        _C.remember_table_radius(out, _C.table_radius(shifts))
+        # from the caller's table, so that the copy is never read back (a
+        # device table is read once, where the op will need the radius)
+        r = _C.table_radius(shifts)
+        if r is not None:
+            _C.remember_table_radius(out, r)
     return out
+
+
+def _row_rules(shifts: torch.Tensor, periodic_inverse: bool, box_forward: bool) -> int:
+    """The `rules` of the native calls (applied to every row as the kernels
+    decode the table: the same rows as ``_mirror_table`` writes out)."""
+    if not (periodic_inverse or box_forward):
+        return 0
+    if shifts.dim() != 2 or shifts.size(1) not in (2, 3):
+        raise ValueError(f"shifts must be (S, 2) or (S, 3); got {tuple(shifts.shape)}")
+    if shifts.size(1) != 3:
+        raise ValueError("periodic_inverse / box_forward require shifts with shape (S, 3)")
+    if _C is None:  # the caller's _require_cuda_ext reports it
+        return 0
+    return ((_C.NSH_PERIODIC_INVERSE if periodic_inverse else 0)
+            | (_C.NSH_BOX_FORWARD if box_forward else 0))
 
 
 def _mirror_table(shifts: torch.Tensor, periodic_inverse: bool,
@@ -439,15 +458,14 @@ def _shared_operand(weights: torch.Tensor, C: int, shared: bool) -> torch.Tensor
 
 class _AccumulateUZFn(torch.autograd.Function):
     @staticmethod
-    def forward(ctx, x, weights, shifts, row_codes=False, shared=False):
+    def forward(ctx, x, weights, shifts, rules=0, shared=False):
         if shifts.dim() != 2 or shifts.size(1) != 3:
             raise ValueError("accumulate_uz requires shifts of shape (S, 3)")
-        shifts_i = _prep_shifts_for_cuda(shifts, x.device)
+        shifts_i = _prep_shifts_for_cuda(shifts, x.device, radius=True)
         x_c, w_c = x.contiguous(), weights.contiguous()
-        U, Z = _C.accumulate_uz_forward(x_c, w_c, shifts_i, row_codes=row_codes,
-                                        shared_weights=shared)
+        U, Z = _C.accumulate_uz_forward(x_c, w_c, shifts_i, rules=rules, shared_weights=shared)
         ctx.save_for_backward(x_c, w_c, shifts_i)
-        ctx.row_codes = row_codes
+        ctx.rules = rules
         ctx.shared = shared
         return U, Z
 
@@ -460,7 +478,7 @@ class _AccumulateUZFn(torch.autograd.Function):
             grad_Z = torch.zeros(x.shape, dtype=_C._acc_dtype(x.dtype), device=x.device)
         grad_x, grad_w = _C.accumulate_uz_backward(
             x, weights, grad_U.contiguous(), grad_Z.contiguous(), shifts_i,
-            row_codes=ctx.row_codes, shared_weights=ctx.shared)
+            rules=ctx.rules, shared_weights=ctx.shared)
         return grad_x, _shared_grad(grad_w, ctx.shared), None, None, None
 
 
@@ -502,19 +520,17 @@ def mix_head_planes(w: torch.Tensor, mix: torch.Tensor) -> torch.Tensor:
 
 class _NormalizedAccumulateUZFn(torch.autograd.Function):
     @staticmethod
-    def forward(ctx, x, weights, shifts, log_weights, row_codes=False, shared=False,
-                weights_ok=None):
+    def forward(ctx, x, weights, shifts, log_weights, rules=0, shared=False, weights_ok=None):
         if shifts.dim() != 2 or shifts.size(1) != 3:
             raise ValueError("normalized_accumulate_uz requires shifts of shape (S, 3)")
-        shifts_i = _prep_shifts_for_cuda(shifts, x.device)
+        shifts_i = _prep_shifts_for_cuda(shifts, x.device, radius=x.dtype == torch.float64)
         x_c, w_c = x.contiguous(), weights.contiguous()
         D, log_C = _C.normalized_accumulate_uz_forward(x_c, w_c, shifts_i, bool(log_weights),
-                                                       row_codes=row_codes,
-                                                       shared_weights=shared,
+                                                       rules=rules, shared_weights=shared,
                                                        weights_ok=weights_ok)
         ctx.save_for_backward(x_c, w_c, D, log_C, shifts_i)
         ctx.log_weights = bool(log_weights)
-        ctx.row_codes = row_codes
+        ctx.rules = rules
         ctx.shared = shared
         ctx.set_materialize_grads(False)
         return D, log_C
@@ -528,7 +544,7 @@ class _NormalizedAccumulateUZFn(torch.autograd.Function):
             grad_log_C = torch.zeros_like(log_C)
         grad_x, grad_w = _C.normalized_accumulate_uz_backward(
             x, weights, D, log_C, grad_D.contiguous(), grad_log_C.contiguous(), shifts_i,
-            ctx.log_weights, row_codes=ctx.row_codes, shared_weights=ctx.shared)
+            ctx.log_weights, rules=ctx.rules, shared_weights=ctx.shared)
         return grad_x, _shared_grad(grad_w, ctx.shared), None, None, None, None, None
 
 
@@ -648,10 +664,10 @@ def accumulate_uz(x: torch.Tensor, weights: torch.Tensor, shifts: torch.Tensor, 
     (nekde_drunet_attn_patch.py:117-140) -- without materialising the
     broadcast copy; their gradient is the sum over the channels."""
     if x.is_cuda:
-        table, codes = _mirror_table(shifts, periodic_inverse, box_forward)
+        rules = _row_rules(shifts, periodic_inverse, box_forward)
         x_d, w_d = _device_operands(x, weights)
         _require_cuda_ext("accumulate_uz")
-        return _AccumulateUZFn.apply(x_d, w_d, table, codes, bool(shared_weights))
+        return _AccumulateUZFn.apply(x_d, w_d, shifts, rules, bool(shared_weights))
     weights = _shared_operand(weights, x.shape[1], shared_weights)
     x_acc, w_acc = _promote_accumulation_inputs(x, weights)
     return accumulate_uz_reference(x_acc, w_acc, shifts, periodic_inverse=periodic_inverse,
@@ -676,12 +692,12 @@ def normalized_accumulate_uz(x: torch.Tensor, weights: torch.Tensor, shifts: tor
     if validate and not in_kernel:
         _validate_stable_weights(w_d, log_weights, asynchronous=x_d.is_cuda)
     if x_d.is_cuda:
-        table, codes = _mirror_table(shifts, periodic_inverse, box_forward)
+        rules = _row_rules(shifts, periodic_inverse, box_forward)
         _require_cuda_ext("normalized_accumulate_uz", need_normalized=True)
         # the forward kernel checks every weight as it reads it
         ok = (torch.ones((), dtype=torch.int32, device=x_d.device)
               if validate and in_kernel else None)
-        D, log_C = _NormalizedAccumulateUZFn.apply(x_d, w_d, table, log_weights, codes,
+        D, log_C = _NormalizedAccumulateUZFn.apply(x_d, w_d, shifts, log_weights, rules,
                                                    bool(shared_weights), ok)
         if ok is not None:
             torch._assert_async(ok, _weight_contract(log_weights))
@@ -723,10 +739,10 @@ def normalized_accumulate_uz_mixed(x: torch.Tensor, head_weights: torch.Tensor,
         t.requires_grad for t in (x, head_weights, head_mix))
     if x.is_cuda and not wants_grad:
         x_d, hw_d = _device_operands(x, head_weights)
-        table, codes = _mirror_table(shifts, periodic_inverse, box_forward)
+        rules = _row_rules(shifts, periodic_inverse, box_forward)
         _require_cuda_ext("normalized_accumulate_uz_mixed", need_normalized=True)
         out = _C.normalized_accumulate_uz_forward_mixed(
-            x_d.contiguous(), hw_d.contiguous(), head_mix, table, row_codes=codes)
+            x_d.contiguous(), hw_d.contiguous(), head_mix, shifts, rules=rules)
         if out is not None:
             D, log_C = out
             return (D, log_C) if return_log_degree else D
