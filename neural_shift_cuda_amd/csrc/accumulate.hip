@@ -459,13 +459,12 @@ __global__ __launch_bounds__(kTPR * ROWS) void accumulate_uz_bwd_kernel(
 // The window border (targets outside the tile) is spilled to a workspace
 // block per tile; spill_fixup_kernel then adds, for every pixel
 // within R of a tile edge, the spills of the (up to 8) neighbouring tiles in
-// a fixed order.  Eligibility (host-checked): at least 2 tiles in each
-// direction and edge tiles at least kRmax wide, so each window reaches only
-// adjacent tiles and never its own tile.  With 2 tiles in a direction the
-// neighbour on either side is the same tile, but a pixel near the left edge
-// reads that tile's right border entries and a pixel near the right edge its
-// left border entries (the window's wrap around the torus of tiles), which
-// are distinct words.  Tables with a radius above kRmax take the gather path
+// a fixed order.  Eligibility (host-checked): every tile at least kRmax wide
+// and high, so each window reaches only adjacent tiles.  With 1 or 2 tiles in
+// a direction the neighbour on either side is the same tile (with 1 the tile
+// itself), but a pixel near the left edge reads that tile's right border
+// entries and a pixel near the right edge its left border entries (the
+// window's wrap around the torus of tiles), which are distinct words.  Tables with a radius above kRmax take the gather path
 // inside the same launch.
 // ---------------------------------------------------------------------------
 
@@ -477,8 +476,8 @@ __global__ __launch_bounds__(kTPR * ROWS) void accumulate_uz_bwd_kernel(
 template <typename T, int VEC, int TPR, int ROWS, int D, bool NTL, int HALO>
 __device__ __forceinline__ void fwd_scatter_tile(
     const T* __restrict__ x, const T* __restrict__ w, const int64_t* __restrict__ shifts, int S,
-    int codes, int C, int H, int W, int ntw, int nth, int64_t plane_step, acc_t<T>* __restrict__ U,
-    acc_t<T>* __restrict__ Z, int* __restrict__ hdr, acc_t<T>* __restrict__ spill,
+    int codes, int C, int H, int W, const TileGrid& tg, int64_t plane_step,
+    acc_t<T>* __restrict__ U, acc_t<T>* __restrict__ Z, int* __restrict__ hdr, acc_t<T>* __restrict__ spill,
     int64_t ntiles, Band bd) {
     using A = acc_t<T>;
     using G = SGeo<VEC, ROWS, TPR, true, HALO>;
@@ -489,25 +488,35 @@ __device__ __forceinline__ void fwd_scatter_tile(
     A* mz = mu + G::TILE;
 
     const int64_t t = xcd_tile(blockIdx.x, gridDim.x);
-    const TileIdx ti = tile_of(t, ntw, nth, G::TH, G::TW);
+    const TileIdx ti = tile_of(t, tg, G::TH, G::TW, H, W);
     const int64_t HW = static_cast<int64_t>(H) * W;
 
     stage_shifts(shl, shifts, S, 3, H, W, codes);
     // Every row's x read must come from the LDS tile (|dx|, |dy| <= HALO),
     // and the mirror scatter must reach only adjacent tiles (radius at most
-    // the narrowest tile, the partial last one); otherwise the tile runs the
-    // gather algorithm.  Uniform over the launch.
+    // the narrowest tile); otherwise the tile runs the gather algorithm.
+    // Uniform over the launch.
     const int R = table_radius(shl, S, true);
-    const bool far = table_radius(shl, S, false) > HALO ||
-                     R > min(W - (ntw - 1) * G::TW, H - (nth - 1) * G::TH);
+    const bool far = table_radius(shl, S, false) > HALO || R > tg.narrow;
     if (blockIdx.x == 0 && threadIdx.x == 0) hdr[0] = far ? kFarRadius : R;  // for the fix-up
     if (far) {
         // the gather algorithm reads a kRmax-halo tile (at this tile's pitch)
         stage_tile<T, A>(xt, x + ti.bc * HW, H, W, ti.h0, ti.w0, G::TH + 2 * kRmax,
                          G::TW + 2 * kRmax, G::PITCH);
         __syncthreads();
-        fwd_gather_tile<T, VEC, 1, ROWS, 1, NTL, TPR, G::PITCH>(
-            x, w, S, C, H, W, ti, plane_step, (codes & kCodesSharedW) != 0, U, Z, shl, xt, bd);
+        const bool wsh = (codes & kCodesSharedW) != 0;
+        if (codes & kCodesVec) {
+            fwd_gather_tile<T, VEC, 1, ROWS, 1, NTL, TPR, G::PITCH>(x, w, S, C, H, W, ti,
+                                                                    plane_step, wsh, U, Z, shl,
+                                                                    xt, bd);
+        } else {  // rows or buffers that a vector does not fit: TPR columns at a time
+            for (int k = 0; k < VEC; ++k) {
+                TileIdx tk = ti;
+                tk.w0 += k * TPR;
+                fwd_gather_tile<T, 1, 1, ROWS, 1, NTL, TPR, G::PITCH>(
+                    x, w, S, C, H, W, tk, plane_step, wsh, U, Z, shl, xt + k * TPR, bd);
+            }
+        }
         return;
     }
     stage_tile<T, A>(xt, x + ti.bc * HW, H, W, ti.h0, ti.w0, G::LH, G::LW, G::PITCH, HALO);
@@ -519,7 +528,7 @@ __device__ __forceinline__ void fwd_scatter_tile(
     const int ty = threadIdx.x / TPR;
     const int h = ti.h0 + ty;
     const int hr = band_row(bd, h < H ? h : ti.h0);  // image row (box tests)
-    const LanePix<VEC, TPR> px = lane_pixels<VEC, TPR>(h, ti.w0, tx, H, W);
+    const LanePix<VEC, TPR> px = lane_pixels<VEC, TPR>(ti, ty, tx, W);
     const int lc = (ty + HALO) * G::PITCH + tx + HALO;  // pixel k at lc + k*TPR
     const int64_t b = ti.bc / C;
     const bool wsh = (codes & kCodesSharedW) != 0;
@@ -553,7 +562,7 @@ __device__ __forceinline__ void fwd_scatter_tile(
     // second, select-free copy of the loop (the masks cost about two thirds
     // of the loop's VALU instructions).
     const int R_all = table_radius(shl, S, false);
-    const bool interior = ti.h0 >= R_all && ti.h0 + G::TH + R_all <= H && ti.w0 >= R_all &&
+    const bool interior = ti.th == G::TH && ti.tw == G::TW && ti.h0 >= R_all && ti.h0 + G::TH + R_all <= H && ti.w0 >= R_all &&
                           ti.w0 + G::TW + R_all <= W &&
                           band_rows_inside(bd, ti.h0, ti.h0 + G::TH - 1, -R_all) &&
                           band_rows_inside(bd, ti.h0, ti.h0 + G::TH - 1, R_all);
@@ -648,8 +657,7 @@ __device__ __forceinline__ void fwd_scatter_tile(
         Zt[px.own[k]] = z[k] + mz[lc + k * TPR];
     }
     if (R == 0) return;
-    const int th = min(G::TH, H - ti.h0);
-    const int tw = min(G::TW, W - ti.w0);
+    const int th = ti.th, tw = ti.tw;
     const int n = spill_count(th, tw, R);
     A* su = spill + t * G::SPILL;
     A* sz = spill + (ntiles + t) * G::SPILL;
@@ -664,11 +672,11 @@ __device__ __forceinline__ void fwd_scatter_tile(
 
 #define NSH_FWD_SCATTER_PARAMS                                                                  \
     const T *__restrict__ x, const T *__restrict__ w, const int64_t *__restrict__ shifts, int S, \
-        int codes, int C, int H, int W, int ntw, int nth, int64_t plane_step,                    \
+        int codes, int C, int H, int W, TileGrid tg, int64_t plane_step,                         \
         acc_t<T> *__restrict__ U, acc_t<T> *__restrict__ Z, int *__restrict__ hdr,              \
         acc_t<T> *__restrict__ spill, int64_t ntiles, Band bd
 #define NSH_FWD_SCATTER_ARGS \
-    x, w, shifts, S, codes, C, H, W, ntw, nth, plane_step, U, Z, hdr, spill, ntiles, bd
+    x, w, shifts, S, codes, C, H, W, tg, plane_step, U, Z, hdr, spill, ntiles, bd
 
 template <typename T, int VEC, int TPR, int ROWS, int D, bool NTL, int WPE, int HALO>
 __global__ __launch_bounds__(TPR * ROWS, WPE) void accumulate_uz_fwd_scatter_kernel(
@@ -750,17 +758,22 @@ __device__ __forceinline__ void stage3_tile_bwd(A* xl, const T* __restrict__ xp,
 // as many bytes as it reads (gw), and one 16-byte load and one 16-byte
 // store per lane and shift measured faster than four 4-byte ones; the LDS
 // tiles use the de-interleaved columns of BwdLayout so that these lanes'
-// LDS accesses are conflict-free.
-template <typename T, int VEC, int TPR, int ROWS, int D, bool NTL, int HALO = kRmax>
+// LDS accesses are conflict-free.  Rows that are no multiple of VEC and
+// unaligned buffers take the strided form (CONTIG = false: pixels tx,
+// tx + TPR, ..., moved one by one, row-major tiles of the same pitch).
+// NTS: streaming stores of gw (see launch_bwd_scatter).
+template <typename T, int VEC, int TPR, int ROWS, int D, bool NTL, bool CONTIG, bool NTS,
+          int HALO = kRmax>
 __global__ __launch_bounds__(TPR * ROWS) void accumulate_uz_bwd_scatter_kernel(
     const T* __restrict__ x, const T* __restrict__ w, const acc_t<T>* __restrict__ gU,
     const acc_t<T>* __restrict__ gZ, const int64_t* __restrict__ shifts, int S, int codes, int C,
-    int H, int W, int ntw, int nth, int64_t plane_step, T* __restrict__ gx, acc_t<T>* __restrict__ gxp,
+    int H, int W, TileGrid tg, int64_t plane_step, T* __restrict__ gx, acc_t<T>* __restrict__ gxp,
     T* __restrict__ gw, int* __restrict__ hdr, acc_t<T>* __restrict__ spill, int64_t ntiles,
     Band bd) {
     using A = acc_t<T>;
     using G = SGeo<VEC, ROWS, TPR, false, HALO>;
-    using L = BwdLayout<VEC, G::LW, G::PITCH>;
+    using L = std::conditional_t<CONTIG, BwdLayout<VEC, G::LW, G::PITCH>,
+                                 RowLayout<SGeo<VEC, ROWS, TPR, true, HALO>::PITCH>>;
     static_assert(G::LH * L::PITCH <= G::TILE, "de-interleaved tile exceeds the LDS plan");
     extern __shared__ __align__(16) unsigned char smem[];
     int4* shl = reinterpret_cast<int4*>(smem);
@@ -770,7 +783,7 @@ __global__ __launch_bounds__(TPR * ROWS) void accumulate_uz_bwd_scatter_kernel(
     A* mg = zt + G::TILE;
 
     const int64_t t = xcd_tile(blockIdx.x, gridDim.x);
-    const TileIdx ti = tile_of(t, ntw, nth, G::TH, G::TW);
+    const TileIdx ti = tile_of(t, tg, G::TH, G::TW, H, W);
     const int64_t HW = static_cast<int64_t>(H) * W;
     const int64_t off = ti.bc * HW;
 
@@ -778,7 +791,7 @@ __global__ __launch_bounds__(TPR * ROWS) void accumulate_uz_bwd_scatter_kernel(
     // every row scatters its x term: radius within the halo and at most the
     // narrowest tile (the partial last one), else the gather algorithm
     const int R = table_radius(shl, S, false);
-    const bool far = R > HALO || R > min(W - (ntw - 1) * G::TW, H - (nth - 1) * G::TH);
+    const bool far = R > HALO || R > tg.narrow;
     if (blockIdx.x == 0 && threadIdx.x == 0) hdr[0] = far ? kFarRadius : R;  // for the fix-up
     if (far) {
         // the gather algorithm reads row-major kRmax-halo tiles (at this
@@ -788,9 +801,19 @@ __global__ __launch_bounds__(TPR * ROWS) void accumulate_uz_bwd_scatter_kernel(
         stage_tile<A, A>(ut, gU + off, H, W, ti.h0, ti.w0, GLH, GLW, G::PITCH);
         stage_tile<A, A>(zt, gZ + off, H, W, ti.h0, ti.w0, GLH, GLW, G::PITCH);
         __syncthreads();
-        bwd_gather_tile<T, VEC, 1, ROWS, 1, NTL, TPR, G::PITCH>(
-            x, w, gU, gZ, S, C, H, W, ti, plane_step, (codes & kCodesSharedW) != 0, gx, gw, shl,
-            xt, ut, zt, bd);
+        const bool wsh = (codes & kCodesSharedW) != 0;
+        if constexpr (CONTIG) {
+            bwd_gather_tile<T, VEC, 1, ROWS, 1, NTL, TPR, G::PITCH>(
+                x, w, gU, gZ, S, C, H, W, ti, plane_step, wsh, gx, gw, shl, xt, ut, zt, bd);
+        } else {  // TPR columns at a time
+            for (int k = 0; k < VEC; ++k) {
+                TileIdx tk = ti;
+                tk.w0 += k * TPR;
+                bwd_gather_tile<T, 1, 1, ROWS, 1, NTL, TPR, G::PITCH>(
+                    x, w, gU, gZ, S, C, H, W, tk, plane_step, wsh, gx, gw, shl, xt + k * TPR,
+                    ut + k * TPR, zt + k * TPR, bd);
+            }
+        }
         return;
     }
     stage3_tile_bwd<T, A, L, HALO>(xt, x + off, ut, gU + off, zt, gZ + off, H, W, ti.h0, ti.w0,
@@ -802,14 +825,23 @@ __global__ __launch_bounds__(TPR * ROWS) void accumulate_uz_bwd_scatter_kernel(
     const int ty = threadIdx.x / TPR;
     const int h = ti.h0 + ty;
     const int hr = band_row(bd, h < H ? h : ti.h0);  // image row (box tests)
-    const int wq = ti.w0 + tx * VEC;
-    const bool act = h < H && wq < W;
+    const int wq = ti.w0 + tx * VEC;  // contiguous form
+    const bool act = ty < ti.th && tx * VEC < ti.tw;
     const uint32_t own = static_cast<uint32_t>(act ? h : 0) * static_cast<uint32_t>(W) +
                          static_cast<uint32_t>(act ? wq : 0);
+    const LanePix<VEC, TPR> px = lane_pixels<VEC, TPR>(ti, ty, tx, W);  // strided form
+    auto pcol = [&](int k) { return CONTIG ? wq + k : ti.w0 + tx + k * TPR; };
+    auto pact = [&](int k) { return CONTIG ? act : px.act[k]; };
     // LDS index of the lane's pixel k displaced by (dx, dy):
-    // lb + dx * PITCH + col(HALO + k + dy), the lane's own column folded into
+    // lb + dx * PITCH + lcol(HALO, k, dy), the lane's own column folded into
     // lb (col(VEC tx + c) = tx + col(c) for c >= 0)
-    const int lb = (ty + HALO) * L::PITCH + (L::DI ? tx : tx * VEC);
+    const int lb = (ty + HALO) * L::PITCH + (CONTIG && !L::DI ? tx * VEC : tx);
+    auto lcol = [](int k, int dy) {
+        if constexpr (CONTIG)
+            return L::col(HALO + k + dy);
+        else
+            return HALO + k * TPR + dy;
+    };
     const int64_t b = ti.bc / C;
     const bool wsh = (codes & kCodesSharedW) != 0;
     // planes are addressed as buffers: uniform base, the lane's byte offset
@@ -821,7 +853,7 @@ __global__ __launch_bounds__(TPR * ROWS) void accumulate_uz_bwd_scatter_kernel(
     A xo[VEC], uo[VEC], zo[VEC], gxa[VEC];
 #pragma unroll
     for (int k = 0; k < VEC; ++k) {
-        const int i = lb + L::col(HALO + k);
+        const int i = lb + lcol(k, 0);
         xo[k] = xt[i];
         uo[k] = ut[i];
         zo[k] = zt[i];
@@ -830,10 +862,17 @@ __global__ __launch_bounds__(TPR * ROWS) void accumulate_uz_bwd_scatter_kernel(
     // Weight prefetch ring.  Loads are unconditional (an idle lane reads its
     // plane's first vector; the tail re-reads plane S-1) so that no load sits
     // behind a branch and the wait counters can keep D loads in flight.
-    SlotRaw<T, VEC> wb[D];
+    using Slot = std::conditional_t<CONTIG, SlotRaw<T, VEC>, PixSlot<T, VEC>>;
+    auto slot_fill = [&](const T* wp, Slot& sl) {
+        if constexpr (CONTIG)
+            slot_load_at<T, VEC, NTL>(wp, own_b, sl);
+        else
+            slot_load_pixels<T, VEC, TPR, NTL>(wp, px, sl);
+    };
+    Slot wb[D];
 #pragma unroll
     for (int d = 0; d < D; ++d)
-        slot_load_at<T, VEC, NTL>(w_bc + static_cast<int64_t>(min(d, S - 1)) * wstep, own_b, wb[d]);
+        slot_fill(w_bc + static_cast<int64_t>(min(d, S - 1)) * wstep, wb[d]);
 
     // One shift: take the ring slot and refill it D shifts ahead, then gw_s[q]
     // (streamed out), the mirror term of gx[q], and the x term of gx
@@ -843,23 +882,26 @@ __global__ __launch_bounds__(TPR * ROWS) void accumulate_uz_bwd_scatter_kernel(
     const T* wr = w_bc + static_cast<int64_t>(min(D, S - 1)) * wstep;
     ShiftRec rn = read_shift(shl, 0);
     T* gp = g_bc;  // gw_s plane of this shift
-    auto step = [&](int s, SlotRaw<T, VEC>& slot) {
+    auto step = [&](int s, Slot& slot) {
         const ShiftRec rc = rn;
         rn = read_shift(shl, min(s + 1, S - 1));
         // consume the slot, then refill it D shifts ahead at once
         A wv[VEC];
-        slot_get<T, VEC>(slot, wv);
-        slot_load_at<T, VEC, NTL>(wr, own_b, slot);
+        if constexpr (CONTIG)
+            slot_get<T, VEC>(slot, wv);
+        else
+            slot_get_pixels<T, VEC>(slot, wv);
+        slot_fill(wr, slot);
         wr += s + D + 1 < S ? wstep : 0;
         if (rc.dx != last_dx) {
             lds_barrier();
             last_dx = rc.dx;
         }
-        if (act) {
+        if (CONTIG ? act : px.any) {
             const int ob = lb + rc.dx * L::PITCH;
             int oi[VEC];
 #pragma unroll
-            for (int k = 0; k < VEC; ++k) oi[k] = ob + L::col(HALO + k + rc.dy);
+            for (int k = 0; k < VEC; ++k) oi[k] = ob + lcol(k, rc.dy);
             A xf[VEC], up_[VEC], zp_[VEC], g[VEC];
 #pragma unroll
             for (int k = 0; k < VEC; ++k) {
@@ -870,10 +912,10 @@ __global__ __launch_bounds__(TPR * ROWS) void accumulate_uz_bwd_scatter_kernel(
             const bool rok = rc.inv && (rc.per || in_range(hr + rc.dx, bd.Hg));
 #pragma unroll
             for (int k = 0; k < VEC; ++k) {
-                const bool okp = rok && (rc.per || in_range(wq + k + rc.dy, W));
+                const bool okp = rok && (rc.per || in_range(pcol(k) + rc.dy, W));
                 // forward box: a dropped w_s[q] has no gradient and adds no
                 // x-gradient term (its mirror is dropped too)
-                const bool kept = fwd_kept(rc, hr, wq + k, bd.Hg, W);
+                const bool kept = fwd_kept(rc, hr, pcol(k), bd.Hg, W);
                 wv[k] = kept ? wv[k] : A(0);
                 g[k] = kept ? fma_acc(xf[k], uo[k], zo[k]) : A(0);
                 if (okp) {
@@ -881,9 +923,17 @@ __global__ __launch_bounds__(TPR * ROWS) void accumulate_uz_bwd_scatter_kernel(
                     gxa[k] = fma_acc(wv[k], up_[k], gxa[k]);
                 }
             }
-            store_acc_at<T, VEC, true>(gp, own_b, g);
+            if constexpr (CONTIG) {
+                store_acc_at<T, VEC, NTS>(gp, own_b, g);
+            } else {
 #pragma unroll
-            for (int k = 0; k < VEC; ++k) mg[oi[k]] += wv[k] * uo[k];
+                for (int k = 0; k < VEC; ++k)
+                    if (px.act[k])
+                        store_elem_at<T, NTS>(gp, px.own[k] * static_cast<uint32_t>(sizeof(T)),
+                                               from_acc<T>(g[k]));
+            }
+#pragma unroll
+            for (int k = 0; k < VEC; ++k) mg[oi[k]] += pact(k) ? wv[k] * uo[k] : A(0);
         }
         gp += plane_step;
     };
@@ -896,17 +946,26 @@ __global__ __launch_bounds__(TPR * ROWS) void accumulate_uz_bwd_scatter_kernel(
     for (int d = 0; d < D; ++d)
         if (S_ring + d < S) step(S_ring + d, wb[d]);
     __syncthreads();
-    if (act) {
+    if constexpr (!CONTIG) {
 #pragma unroll
-        for (int k = 0; k < VEC; ++k) gxa[k] += mg[lb + L::col(HALO + k)];
+        for (int k = 0; k < VEC; ++k) {
+            if (!px.act[k]) continue;
+            const A v = gxa[k] + mg[lb + lcol(k, 0)];
+            if (gxp != nullptr)
+                gxp[off + px.own[k]] = v;
+            else
+                gx[off + px.own[k]] = from_acc<T>(v);
+        }
+    } else if (act) {
+#pragma unroll
+        for (int k = 0; k < VEC; ++k) gxa[k] += mg[lb + lcol(k, 0)];
         if (gxp != nullptr)
             store_out<A, VEC>(gxp + off + own, gxa);
         else
             store_acc<T, VEC>(gx + off + own, gxa, false);
     }
     if (R == 0) return;
-    const int th = min(G::TH, H - ti.h0);
-    const int tw = min(G::TW, W - ti.w0);
+    const int th = ti.th, tw = ti.tw;
     const int n = spill_count(th, tw, R);
     A* sg = spill + t * G::SPILL;
     for (int e = threadIdx.x; e < n; e += blockDim.x) {
@@ -1027,11 +1086,10 @@ constexpr size_t kScatterLdsLimit = 159 * 1024;
 //    tiles of 256 lanes, twice the workgroups: c3 fp64 forward 0.071 ->
 //    0.067 ms, backward 0.173 -> 0.154 ms; 32 x 8 leaves too short a last
 //    tile for many heights);
-//  * kVarAlt: 64 x 32 tiles (16 lanes x 4 pixels), for images too narrow or
-//    short for two tiles of the first choice;
+//  * kVarAlt: 64 x 32 tiles (16 lanes x 4 pixels), two workgroups per CU
+//    (scatter_plan_for says when);
 //  * kVarShort: wide backward tiles of half the rows (128 x 16, two
-//    workgroups per CU), for problems whose wide tiles would fill the CUs
-//    only once (c2 fp16 backward 0.155 -> 0.142 ms);
+//    workgroups per CU);
 //  * kVarHalo16: a 16-pixel border for tables of radius 9..16 (fp32-class
 //    types with VEC 4): forward 128 x 32 (151 KB of LDS at S = 1024),
 //    backward 128 x 16 (one 512-lane workgroup per CU);
@@ -1082,19 +1140,27 @@ static int64_t align256(int64_t b) { return (b + 255) / 256 * 256; }
 // Workspace layout: [header: table radius, 256 B][spill blocks][16-bit gx
 // partial sums (backward only)].
 constexpr int64_t kHeaderBytes = 256;
+// A gradient this small stays in the 256 MB Infinity Cache.
+constexpr int64_t kCachedBytes = int64_t(192) << 20;
 
 struct SPlan {
     bool ok = false;
-    int rows = 0, ntw = 0, nth = 0, spill = 0, halo = kRmax;
+    int rows = 0, spill = 0, halo = kRmax;
+    TileGrid grid{};
     int64_t tiles = 0, spill_bytes = 0, part_bytes = 0, total = 0;
     size_t lds = 0;
 };
 
 // Geometry and workspace of the scatter path for a given vector width.
-// Eligibility: at least 2 tiles in each direction and every tile at least
-// kRmax wide and high, so that a window's border reaches only adjacent tiles
-// for any radius up to kRmax (the kernels run the gather form inside the
-// launch for a table whose radius exceeds the halo or the narrowest tile).
+// Eligibility: an image of at least kScatterMinSide a side (a smaller one is
+// mostly border; the gather kernels read it from the caches) and every tile
+// at least kRmax wide and high, so that a window's border reaches only
+// adjacent tiles for any radius up to kRmax (the kernels run the gather form
+// inside the launch for a table whose radius exceeds the halo or the
+// narrowest tile).  With one tile in a direction the neighbour on either side
+// is the tile itself, as on a torus of one tile.
+constexpr int kScatterMinSide = 32;
+
 static SPlan scatter_plan(const Dims& d, int vec, int tpr, int rows, int halo, size_t tsize,
                           size_t asize, bool bwd) {
     SPlan p;
@@ -1109,11 +1175,10 @@ static SPlan scatter_plan(const Dims& d, int vec, int tpr, int rows, int halo, s
     p.lds = shift_lds_bytes(d.S) + (bwd ? 4 : 3) * tile;
     p.rows = rows;
     p.halo = halo;
-    p.ntw = static_cast<int>(nsh_host::ceil_div(d.W, TW));
-    p.nth = static_cast<int>(nsh_host::ceil_div(d.H, TH));
-    p.ok = p.lds <= kScatterLdsLimit && p.ntw >= 2 && p.nth >= 2 && TH >= halo &&
-           d.W - (p.ntw - 1) * TW >= kRmax && d.H - (p.nth - 1) * TH >= kRmax;
-    p.tiles = static_cast<int64_t>(d.B) * d.C * p.ntw * p.nth;
+    p.grid = nsh_host::tile_grid(d.H, d.W, TH, TW, std::max(kRmax, std::min(d.halo, halo)));
+    p.ok = p.lds <= kScatterLdsLimit && TH >= halo && p.grid.narrow >= kRmax &&
+           d.H >= kScatterMinSide && d.W >= kScatterMinSide;
+    p.tiles = static_cast<int64_t>(d.B) * d.C * p.grid.ntw * p.grid.nth;
     p.spill = 2 * halo * (TW + 2 * halo) + 2 * halo * TH;
     p.spill_bytes = align256((bwd ? 1 : 2) * p.tiles * p.spill * static_cast<int64_t>(asize));
     p.part_bytes = (bwd && tsize < asize)
@@ -1124,30 +1189,23 @@ static SPlan scatter_plan(const Dims& d, int vec, int tpr, int rows, int halo, s
     return p;
 }
 
-// Vector width of the scatter path from the shape alone (the workspace size
-// must not depend on pointer values): the widest vector of at most 4
-// elements (2 for fp64) that divides W and still leaves at least the pass's
-// fill-lane count.  Measured on MI355X: the c3 fp64 forward (393,216
-// pixels) runs 0.112 ms on 1-wide and 0.078 ms on 2-wide lanes, its
-// backward 0.179-0.180 ms on 1-wide and 0.173-0.174 ms on 2-wide lanes (so
-// fp64 takes the forward's fill count in both passes), the c2 fp16 backward
-// (1 M pixels) 0.179 ms on 2-wide and 0.168 ms on 4-wide lanes, the c2 fp16
-// forward 0.109 ms on 2-wide and 0.116 ms on 4-wide lanes; the c4 and c3
-// fp32 shapes are 4-wide either way.
-constexpr int64_t kScatterFillFwd = int64_t(1) << 17;
-constexpr int64_t kScatterFillFwd16 = int64_t(1) << 19;
-constexpr int64_t kScatterFillBwd = int64_t(1) << 18;
-
+// Pixels per lane of the scatter path, from the shape alone (the workspace
+// size must not depend on pointer values).  Any W: the forward's lanes are
+// strided, and the backward's are where W is no multiple.  Small problems
+// trade wide lanes for more of them; half-plane R = 5, 4 / 2 / 1 pixels per
+// lane, in us: fp32 forward 3 x 512^2 (0.79 M pixels) 49 / 48 / 73, 2 x 3 x 321 x
+// 481 (0.93 M) 69 / 75 / 98, 4 x 250^2 (0.25 M) 37 / 32 / 35, 256^2 37 / 29 / 26;
+// fp32 backward 2 x 3 x 71 x 654 (0.28 M) 52 / 54 / 60, 4 x 250^2 52 / 46 / 49;
+// 16-bit backward 2 x 3 x 320 x 480 (0.92 M) 73 / 87 / 137, 3 x 512^2 71 / 65 /
+// 107.  fp64 takes 2 from 0.26 M pixels on (c3 fp64, 0.39 M: forward 78 / 112,
+// backward 173 / 179).
 template <typename T>
 static int scatter_vec(const Dims& d, bool bwd) {
     const int64_t pixels = static_cast<int64_t>(d.B) * d.C * d.H * d.W;
-    const int64_t fill = bwd ? (sizeof(T) == 8 ? kScatterFillFwd : kScatterFillBwd)
-                             : (sizeof(T) == 2 ? kScatterFillFwd16 : kScatterFillFwd);
-    int maxv = sizeof(T) == 8 ? 2 : 4;
-    while (maxv > 1 && pixels / maxv < fill) maxv /= 2;
-    for (int v = maxv; v > 1; v /= 2)
-        if (d.W % v == 0) return v;
-    return 1;
+    if (sizeof(T) == 8) return pixels >= (int64_t(1) << 18) ? 2 : 1;
+    const int64_t four = !bwd ? (int64_t(3) << 18)
+                              : (sizeof(T) == 2 ? (int64_t(7) << 17) : (int64_t(1) << 18));
+    return pixels >= four ? 4 : (pixels >= (int64_t(3) << 16) ? 2 : 1);
 }
 
 template <typename T, int VEC, bool BWD, int VAR>
@@ -1157,48 +1215,79 @@ static SPlan scatter_plan_cfg(const Dims& d) {
                         BWD);
 }
 
-// The backward's wide tiles hold one workgroup per CU (their LDS), so a
-// problem of at most one tile per CU (c2: 256 tiles of 128 x 32) leaves each
-// CU one workgroup whose waves all meet at every barrier; half-height tiles
-// put two independent workgroups on each CU (c2 fp16 backward 0.155 ->
-// 0.142 ms; at c3 and c4, many tiles per CU, they cost 3-9% of halo and
-// spill, so those keep the full height).  One round is one tile per compute
+// Which tiles a shape takes.  One round is one 1024-lane tile per compute
 // unit of the current device (256 on MI355X, also the fallback when no device
-// can be queried, e.g. a workspace query from a process without a GPU).
+// can be queried, e.g. a workspace query from a process without a GPU), or
+// two 512-lane ones.  The wide tiles move the most per pixel of halo and
+// spill, but a last round of a few of them takes as long as a full one, and
+// fewer than one round leaves compute units idle; so, per pass (half-plane
+// R = 5, 61 rows, except where said; wide / 64-wide / half-height, in us):
+//  * forward, 16-bit: 64-wide tiles always (4096^2 R = 7 1194 / 1099 / 1174,
+//    2 x 3 x 321 x 481 100 / 68 / 62, 3 x 1100 x 1500 264 / 234 / 271);
+//  * forward, fp32: 64-wide below one round (2 x 3 x 320 x 480 54.9 / 50.2)
+//    and where the wide tiles' rounds, whole ones at 0.9 of the others' time,
+//    cost more (2 x 3 x 321 x 481, 1.03 rounds, 105 / 69; 1500^2, 2.2 rounds,
+//    159 / 131; not at 3 rounds, 16 x 3 x 256^2: 158 / 182, 4096^2 R = 7 1416 /
+//    1629);
+//  * backward: below one round 64-wide tiles (2 x 3 x 320 x 480 fp32 90 / 80 /
+//    105, 16-bit 79 / 73 / 75), except for fp32 rows of no whole vectors from
+//    half a round on (701 x 901: 102 / 121 / 108; 2 x 3 x 71 x 654, 0.4
+//    rounds: 92 / 52 / 67);
+//  * backward from one round, 16-bit: half-height tiles (two workgroups per
+//    compute unit: 4 x 512^2 R = 7 129 / 118 / 117, 16 x 3 x 256^2 230 / 226 /
+//    207, 4096^2 R = 7, 16 rounds, 2069 / 2006 / 1806; beyond 32 rounds the
+//    wide ones, with half the spill blocks); fp32: half-height where that saves
+//    rounds (2 x 3 x 321 x 481 177 / 176 / 120; not 16 x 3 x 256^2 304 / 327 /
+//    326).
 static int64_t one_round_tiles() { return nsh_host::compute_units(); }
 
-// The plan for a shape: with the wide halo asked for, the 16-pixel-border
-// tiles where they apply; else the first choice (the half-height backward
-// tiles when the full-height ones fill the CUs once), else the second
-// choice; *var says which (p.ok false if none applies).
+// The plan for a shape: with the wide halo asked for, the 16- or
+// 24-pixel-border tiles where they apply; else by the rule above; *var says
+// which (p.ok false if none applies).
 template <typename T, int VEC, bool BWD>
 static SPlan scatter_plan_for(const Dims& d, int* var) {
     if constexpr (ScatterCfg<T, VEC, BWD, kVarWide>::kWide) {
         if (d.halo > kRmax) {
-            const SPlan q = d.halo > 16 ? scatter_plan_cfg<T, VEC, BWD, kVarHalo24>(d)
-                                        : scatter_plan_cfg<T, VEC, BWD, kVarHalo16>(d);
+            // radius 9..16 on tiles that end in one shorter than 16 (the
+            // backward's 16-row tiles cannot lengthen it): the 24-pixel
+            // border's 32-row tiles
+            const SPlan q16 = scatter_plan_cfg<T, VEC, BWD, kVarHalo16>(d);
+            const SPlan q24 = scatter_plan_cfg<T, VEC, BWD, kVarHalo24>(d);
+            const bool wider = d.halo > 16 || (q16.grid.narrow < 16 && q24.grid.narrow >= 16);
+            const SPlan q = wider ? q24 : q16;
             if (q.ok) {
-                *var = d.halo > 16 ? kVarHalo24 : kVarHalo16;
+                *var = wider ? kVarHalo24 : kVarHalo16;
                 return q;
             }
         }
-    }
-    SPlan p = scatter_plan_cfg<T, VEC, BWD, kVarWide>(d);
-    *var = kVarWide;
-    if constexpr (BWD && ScatterCfg<T, VEC, true, kVarWide>::kWide) {
-        if (p.ok && p.tiles <= one_round_tiles()) {
-            const SPlan q = scatter_plan_cfg<T, VEC, true, kVarShort>(d);
-            if (q.ok) {
-                *var = kVarShort;
-                return q;
-            }
-        }
-    }
-    if (!p.ok) {
-        p = scatter_plan_cfg<T, VEC, BWD, kVarAlt>(d);
+        const SPlan wide = scatter_plan_cfg<T, VEC, BWD, kVarWide>(d);
+        const SPlan alt = scatter_plan_cfg<T, VEC, BWD, kVarAlt>(d);
         *var = kVarAlt;
+        // one 128-wide column of tiles would idle lanes that 64-wide ones use
+        if (!wide.ok || wide.grid.ntw < 2 || wide.grid.nth < 2) return alt;
+        const int64_t cu = one_round_tiles();
+        const double rounds = 0.9 * static_cast<double>(nsh_host::ceil_div(wide.tiles, cu));
+        if constexpr (!BWD) {
+            if (sizeof(T) == 2 || wide.tiles < cu ||
+                (wide.tiles > cu && rounds > static_cast<double>(alt.tiles) / (2 * cu)))
+                return alt;
+        } else {
+            const SPlan half = scatter_plan_cfg<T, VEC, BWD, kVarShort>(d);
+            if (wide.tiles < cu) {
+                if (sizeof(T) == 2 || d.W % VEC == 0 || 2 * wide.tiles < cu) return alt;
+            } else if (half.ok &&
+                       ((sizeof(T) == 2 && wide.tiles <= 32 * cu) ||
+                        rounds > static_cast<double>(nsh_host::ceil_div(half.tiles, 2 * cu)))) {
+                *var = kVarShort;
+                return half;
+            }
+        }
+        *var = kVarWide;
+        return wide;
+    } else {
+        *var = kVarWide;  // one geometry per type for the narrower lanes
+        return scatter_plan_cfg<T, VEC, BWD, kVarWide>(d);
     }
-    return p;
 }
 
 template <typename T, bool BWD>
@@ -1240,8 +1329,8 @@ static int launch_fwd_scatter(const void* x, const void* w, const int64_t* sh, c
     auto launch = [&](auto kernel) {
         hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(p.tiles)),
                            dim3(Cfg::TPR * Cfg::ROWS), p.lds, st, static_cast<const T*>(x),
-                           static_cast<const T*>(w), sh, d.S, d.codes, d.C, d.H, d.W, p.ntw,
-                           p.nth, step, static_cast<A*>(U), static_cast<A*>(Z), hdr, spill,
+                           static_cast<const T*>(w), sh, d.S, d.codes, d.C, d.H, d.W, p.grid,
+                           step, static_cast<A*>(U), static_cast<A*>(Z), hdr, spill,
                            p.tiles, d.band);
     };
     if constexpr (Cfg::kSgpr80)
@@ -1253,7 +1342,7 @@ static int launch_fwd_scatter(const void* x, const void* w, const int64_t* sh, c
     if (int rc = nsh_host::check_launch("accumulate_uz_forward")) return rc;
     hipLaunchKernelGGL((spill_fixup_kernel<A, A, 2, false>),
                        dim3(static_cast<unsigned>(p.tiles)), dim3(256), 0, st, d.H, d.W,
-                       Cfg::ROWS, Cfg::TPR * VEC, p.ntw, p.nth, p.spill,
+                       Cfg::ROWS, Cfg::TPR * VEC, p.grid, p.spill,
                        static_cast<const int*>(hdr), static_cast<const A*>(spill), p.tiles,
                        static_cast<const A*>(nullptr), static_cast<A*>(U), static_cast<A*>(Z));
     return nsh_host::check_launch("accumulate_uz_forward (fix-up)");
@@ -1270,18 +1359,43 @@ static int launch_bwd_scatter(const void* x, const void* w, const void* gU, cons
     int* hdr = reinterpret_cast<int*>(base);
     A* spill = reinterpret_cast<A*>(base + kHeaderBytes);
     A* part = p.part_bytes ? reinterpret_cast<A*>(base + kHeaderBytes + p.spill_bytes) : nullptr;
-    hipLaunchKernelGGL((accumulate_uz_bwd_scatter_kernel<T, VEC, Cfg::TPR, Cfg::ROWS, Cfg::D,
-                                                         Cfg::NTL, Cfg::HALO>),
-                       dim3(static_cast<unsigned>(p.tiles)), dim3(Cfg::TPR * Cfg::ROWS), p.lds,
-                       st, static_cast<const T*>(x), static_cast<const T*>(w),
-                       static_cast<const A*>(gU), static_cast<const A*>(gZ), sh, d.S, d.codes,
-                       d.C, d.H, d.W, p.ntw, p.nth, step, static_cast<T*>(gx), part,
-                       static_cast<T*>(gw), hdr, spill, p.tiles, d.band);
+    auto launch = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(p.tiles)),
+                           dim3(Cfg::TPR * Cfg::ROWS), p.lds, st, static_cast<const T*>(x),
+                           static_cast<const T*>(w), static_cast<const A*>(gU),
+                           static_cast<const A*>(gZ), sh, d.S, d.codes, d.C, d.H, d.W, p.grid,
+                           step, static_cast<T*>(gx), part, static_cast<T*>(gw), hdr, spill,
+                           p.tiles, d.band);
+    };
+    // gw is written once and not read back: streaming stores, but only where
+    // whole rows of 128-byte lines make a tile's row segments whole lines.
+    // Otherwise two tiles share a line at every seam and the streamed parts
+    // reach memory one by one (R = 5, streaming -> plain stores: 2 x 3 x 321 x
+    // 481 fp32 161 -> 123 us, 8 x 3 x 250^2 fp64 450 -> 351 us, 3 x 1100 x 1500
+    // fp16 434 -> 381 us); the fp32 vector stores' longer segments lose less
+    // there than plain ones (1500^2 290 -> 307 us, 700 x 900 74 -> 109 us), and
+    // a gw that stays in the Infinity Cache joins the parts there (4 x 250^2
+    // fp64 R = 6 81 -> 95 us).
+    const bool contig = VEC == 1 || (d.codes & kCodesVec);
+    const bool lines = static_cast<int64_t>(d.W) * sizeof(T) % 128 == 0;
+    const bool small = step * d.S * static_cast<int64_t>(sizeof(T)) < kCachedBytes;
+    const bool stream = lines || (contig && (sizeof(T) == 4 || small));
+    auto go = [&](auto contig, auto nts) {
+        launch(accumulate_uz_bwd_scatter_kernel<T, VEC, Cfg::TPR, Cfg::ROWS, Cfg::D, Cfg::NTL,
+                                                decltype(contig)::value, decltype(nts)::value,
+                                                Cfg::HALO>);
+    };
+    if (contig && stream)
+        go(std::true_type{}, std::true_type{});
+    else if (contig)
+        go(std::true_type{}, std::false_type{});
+    else if constexpr (VEC > 1)
+        go(std::false_type{}, std::false_type{});
     if (int rc = nsh_host::check_launch("accumulate_uz_backward")) return rc;
     constexpr bool kPart = sizeof(T) < sizeof(A);
     hipLaunchKernelGGL((spill_fixup_kernel<T, A, 1, kPart>),
                        dim3(static_cast<unsigned>(p.tiles)), dim3(256), 0, st, d.H, d.W,
-                       Cfg::ROWS, Cfg::TPR * VEC, p.ntw, p.nth, p.spill,
+                       Cfg::ROWS, Cfg::TPR * VEC, p.grid, p.spill,
                        static_cast<const int*>(hdr), static_cast<const A*>(spill), p.tiles,
                        static_cast<const A*>(part), static_cast<T*>(gx), static_cast<T*>(nullptr));
     return nsh_host::check_launch("accumulate_uz_backward (fix-up)");
@@ -1312,22 +1426,20 @@ static int launch_scatter_var(int var, const void* x, const void* w, const void*
 // kernels run).
 template <typename T, bool BWD>
 static int try_scatter(const void* x, const void* w, const void* gU, const void* gZ,
-                       const int64_t* sh, const Dims& d, void* o0, void* o1, void* ws,
+                       const int64_t* sh, Dims d, void* o0, void* o1, void* ws,
                        int64_t ws_bytes, hipStream_t st) {
     if (ws == nullptr || scatter_disabled()) return -1;
     const int v = scatter_vec<T>(d, BWD);
     int var = kVarWide;
     const SPlan p = scatter_plan_any<T, BWD>(d, v, &var);
     if (!p.ok || ws_bytes < p.total || !nsh_host::aligned(ws, 256)) return -1;
+    // whether the lanes' vectors fit the rows and buffers; both forms exist
     const size_t vb = static_cast<size_t>(v) * sizeof(T);
-    for (const void* q : {x, w, static_cast<const void*>(o0), static_cast<const void*>(o1)})
-        if (!nsh_host::aligned(q, vb)) return -1;
-    if (BWD && (!nsh_host::aligned(gU, v * sizeof(acc_t<T>)) ||
-                !nsh_host::aligned(gZ, v * sizeof(acc_t<T>))))
-        return -1;
-    if (!BWD && (!nsh_host::aligned(o0, v * sizeof(acc_t<T>)) ||
-                 !nsh_host::aligned(o1, v * sizeof(acc_t<T>))))
-        return -1;
+    const size_t ab = std::min<size_t>(16, static_cast<size_t>(v) * sizeof(acc_t<T>));
+    bool vec = d.W % v == 0 && nsh_host::aligned(x, vb) && nsh_host::aligned(w, vb) &&
+               nsh_host::aligned(o0, BWD ? vb : ab) && nsh_host::aligned(o1, BWD ? vb : ab);
+    if (BWD) vec = vec && nsh_host::aligned(gU, ab) && nsh_host::aligned(gZ, ab);
+    d.codes |= vec ? kCodesVec : 0;
     switch (v) {
         case 4:
             if constexpr (sizeof(T) <= 4)

@@ -628,14 +628,14 @@ __global__ __launch_bounds__(TPR * ROWS, WPE) void metropolis_aggregate_scatter_
 // plus the neighbouring tiles' spills, then Wx = x - d_hat x + K_hat x.
 template <typename T>
 __global__ __launch_bounds__(256) void metropolis_fixup_kernel(
-    int H, int W, int TH, int TW, int ntw, int nth, int spill_stride, int ring_stride,
+    int H, int W, int TH, int TW, TileGrid tg, int spill_stride, int ring_stride,
     const int* __restrict__ hdr, const acc_t<T>* __restrict__ spill,
     const acc_t<T>* __restrict__ part, int64_t ntiles, const T* __restrict__ img,
     T* __restrict__ Wx, T* __restrict__ dhat) {
     using A = acc_t<T>;
     const int R = __builtin_amdgcn_readfirstlane(hdr[0]);
     if (R == 0) return;
-    const FixTile f = fix_tile(blockIdx.x, H, W, TH, TW, ntw, nth);
+    const FixTile f = fix_tile(blockIdx.x, H, W, TH, TW, tg);
     const int64_t HW = static_cast<int64_t>(H) * W;
     const A* pk = part + 2 * static_cast<int64_t>(blockIdx.x) * ring_stride;
     const A* ph = pk + ring_stride;
@@ -1361,6 +1361,8 @@ static int m_scatter(const void* wh, const void* img, const int64_t* sh, int B, 
     A* spill = reinterpret_cast<A*>(base + kMHeader);
     A* part = reinterpret_cast<A*>(base + kMHeader + p.spill_bytes);
     constexpr int V = Cfg::VEC, T1 = Cfg::TPR1, T2 = Cfg::TPR2, R1 = Cfg::ROWS1, R2 = Cfg::ROWS2;
+    const TileGrid grid1 = nsh_host::tile_grid(H, W, R1, T1 * V);
+    const TileGrid grid2 = nsh_host::tile_grid(H, W, R2, T2 * V);
     if (use_box)
         hipLaunchKernelGGL((metropolis_degree_scatter_kernel<T, V, T1, R1, Cfg::D1, true>),
                            dim3(static_cast<unsigned>(p.tiles1)), dim3(T1 * R1), p.lds1, st,
@@ -1373,7 +1375,7 @@ static int m_scatter(const void* wh, const void* img, const int64_t* sh, int B, 
                            static_cast<A*>(deg), hdr, spill);
     if (int rc = nsh_host::check_launch("metropolis_aggregate (degree)")) return rc;
     hipLaunchKernelGGL((spill_fixup_kernel<A, A, 1, false>), dim3(static_cast<unsigned>(p.tiles1)),
-                       dim3(256), 0, st, H, W, R1, T1 * V, p.ntw1, p.nth1, p.spill1,
+                       dim3(256), 0, st, H, W, R1, T1 * V, grid1, p.spill1,
                        static_cast<const int*>(hdr), static_cast<const A*>(spill), p.tiles1,
                        static_cast<const A*>(nullptr), static_cast<A*>(deg),
                        static_cast<A*>(nullptr));
@@ -1394,7 +1396,7 @@ static int m_scatter(const void* wh, const void* img, const int64_t* sh, int B, 
                            spill, part, p.ring, p.tiles2);
     if (int rc = nsh_host::check_launch("metropolis_aggregate (aggregate)")) return rc;
     hipLaunchKernelGGL((metropolis_fixup_kernel<T>), dim3(static_cast<unsigned>(p.tiles2)),
-                       dim3(256), 0, st, H, W, R2, T2 * V, p.ntw2, p.nth2, p.spill2, p.ring,
+                       dim3(256), 0, st, H, W, R2, T2 * V, grid2, p.spill2, p.ring,
                        static_cast<const int*>(hdr), static_cast<const A*>(spill),
                        static_cast<const A*>(part), p.tiles2, static_cast<const T*>(img),
                        static_cast<T*>(Wx), static_cast<T*>(dhat));
@@ -1510,6 +1512,7 @@ static int mb_launch(const void* wh, const void* img, const int64_t* sh, int B, 
     using Cfg = MBwdCfg<T>;
     using A = acc_t<T>;
     constexpr int V = Cfg::VEC, TPR = Cfg::TPR, R1 = Cfg::ROWS1, R2 = Cfg::ROWS2;
+    const TileGrid grid1 = nsh_host::tile_grid(H, W, R1, TPR * V);
     char* base = static_cast<char*>(ws);
     int* hdr = reinterpret_cast<int*>(base);
     A* spill = reinterpret_cast<A*>(base + kMHeader);
@@ -1532,7 +1535,7 @@ static int mb_launch(const void* wh, const void* img, const int64_t* sh, int B, 
     }
     if (int rc = nsh_host::check_launch("metropolis_aggregate_backward (edges)")) return rc;
     hipLaunchKernelGGL((spill_fixup_kernel<A, A, 2, false>), dim3(static_cast<unsigned>(p.tiles1)),
-                       dim3(256), 0, st, H, W, R1, TPR * V, p.ntw1, p.nth1, p.spill,
+                       dim3(256), 0, st, H, W, R1, TPR * V, grid1, p.spill,
                        static_cast<const int*>(hdr), static_cast<const A*>(spill), p.tiles1,
                        static_cast<const A*>(nullptr), gd, gxp);
     if (int rc = nsh_host::check_launch("metropolis_aggregate_backward (fix-up)")) return rc;

@@ -24,9 +24,9 @@
 //   gw_s[q] = 0 for a masked weight, else
 //             F(L[q]) score(q, x[(q+s) mod]) + [inv, box(q+s)] F(L[q+s]) score(q+s, x[q])
 //   score(o, v) = gD[o] (v - D[o]) + gLogC[o];  F = f (log mode) or exp(-L).
+#include <algorithm>
 #include <cstdlib>
 #include <initializer_list>
-
 #include <type_traits>
 
 #include "nsh_common.hpp"
@@ -639,10 +639,10 @@ __device__ __forceinline__ int near_radius(const int4* shl, int S, bool only_inv
 // tiles 13% slower: c3 0.326 -> 0.368 ms); the 16-bit forward 2% slower,
 // the fp16 and fp64 backwards within the run-to-run spread (+-2%).  So:
 // nontemporal in the fp32 and fp64 forwards and the fp32 backward.
-template <typename T>
-constexpr bool kNormFwdNT = sizeof(T) >= 4;
-template <typename T>
-constexpr bool kNormBwdNT = sizeof(T) == 4;
+template <typename T, int TPR>
+constexpr bool kNormFwdNT = sizeof(T) == 8 || (sizeof(T) == 4 && TPR == 32);
+template <typename T, int TPR>
+constexpr bool kNormBwdNT = sizeof(T) == 4 && TPR == 32;
 // The weight of pixel p for channel c from NH head planes: NH = 1 reads the
 // plane as it is; NH > 1 forms sum_j mix[c][j] w_j[p] (the head-mixing
 // product of the attention installers, applied where the weights are
@@ -671,7 +671,7 @@ template <typename T, int VEC, int TPR, int ROWS, int D, bool LOGW,
 __global__ __launch_bounds__(TPR * ROWS, WPE) void
 normalized_fwd_scatter_kernel(const T* __restrict__ x, const T* __restrict__ w,
                               const int64_t* __restrict__ shifts, int S, int codes, int C, int H,
-                              int W, int ntw, int nth, int64_t plane_step, acc_t<T>* __restrict__ Dout,
+                              int W, TileGrid tg, int64_t plane_step, acc_t<T>* __restrict__ Dout,
                               acc_t<T>* __restrict__ Lout, int* __restrict__ hdr,
                               acc_t<T>* __restrict__ spill, acc_t<T>* __restrict__ part,
                               int ring_stride, int64_t ntiles,
@@ -686,7 +686,7 @@ normalized_fwd_scatter_kernel(const T* __restrict__ x, const T* __restrict__ w,
     A* wz = wu + G::TILE;
 
     const int64_t t = xcd_tile(blockIdx.x, gridDim.x);
-    const TileIdx ti = tile_of(t, ntw, nth, G::TH, G::TW);
+    const TileIdx ti = tile_of(t, tg, G::TH, G::TW, H, W);
     const int64_t HW = static_cast<int64_t>(H) * W;
     const int64_t off = ti.bc * HW;
     const T* xp = x + off;
@@ -706,7 +706,7 @@ normalized_fwd_scatter_kernel(const T* __restrict__ x, const T* __restrict__ w,
     const int tx = threadIdx.x % TPR;
     const int ty = threadIdx.x / TPR;
     const int h = ti.h0 + ty;
-    const LanePix<VEC, TPR> px = lane_pixels<VEC, TPR>(h, ti.w0, tx, H, W);
+    const LanePix<VEC, TPR> px = lane_pixels<VEC, TPR>(ti, ty, tx, W);
     const int lc = (ty + kRmax) * G::PITCH + tx + kRmax;  // pixel k at lc + k*TPR
     const int64_t b = ti.bc / C;
     const int64_t ch = ti.bc - b * C;
@@ -734,7 +734,7 @@ normalized_fwd_scatter_kernel(const T* __restrict__ x, const T* __restrict__ w,
     for (int d = 0; d < D; ++d)
 #pragma unroll
         for (int j = 0; j < NH; ++j)
-            slot_load_pixels<T, VEC, TPR, kNormFwdNT<T>>(
+            slot_load_pixels<T, VEC, TPR, kNormFwdNT<T, TPR>>(
                 w_bc + j * HW + static_cast<int64_t>(min(d, S - 1)) * wstep, px, wb[d][j]);
     const T* wr = w_bc + static_cast<int64_t>(min(D, S - 1)) * wstep;
     ShiftRec rn = read_shift(shl, 0);
@@ -743,7 +743,7 @@ normalized_fwd_scatter_kernel(const T* __restrict__ x, const T* __restrict__ w,
     // it for all rows of the table) need no forward-box test and no mirror
     // mask: they run a select-free copy of the loop.
     const int R_all = table_radius(shl, S, false);
-    const bool interior = ti.h0 >= R_all && ti.h0 + G::TH + R_all <= H && ti.w0 >= R_all &&
+    const bool interior = ti.th == G::TH && ti.tw == G::TW && ti.h0 >= R_all && ti.h0 + G::TH + R_all <= H && ti.w0 >= R_all &&
                           ti.w0 + G::TW + R_all <= W;
     int last_dx = kClamp;
     // MODE 0: interior tile; 1: masks; 2: masks and forward-box rows
@@ -755,7 +755,7 @@ normalized_fwd_scatter_kernel(const T* __restrict__ x, const T* __restrict__ w,
         mixed_pixels<T, VEC, NH, A>(slot, mixc, wv);
 #pragma unroll
         for (int j = 0; j < NH; ++j)
-            slot_load_pixels<T, VEC, TPR, kNormFwdNT<T>>(wr + j * HW, px, slot[j]);
+            slot_load_pixels<T, VEC, TPR, kNormFwdNT<T, TPR>>(wr + j * HW, px, slot[j]);
         wr += s + D + 1 < S ? wstep : 0;
         if (shift_in_lds(rc)) {
             const int op = lc + rc.dx * G::PITCH + rc.dy;  // window index of q + s
@@ -909,8 +909,7 @@ normalized_fwd_scatter_kernel(const T* __restrict__ x, const T* __restrict__ w,
         if (bad) *weights_ok = 0;
     }
     __syncthreads();
-    const int th = min(G::TH, H - ti.h0);
-    const int tw = min(G::TW, W - ti.w0);
+    const int th = ti.th, tw = ti.tw;
     A* pm = part + 3 * t * ring_stride;
 #pragma unroll
     for (int k = 0; k < VEC; ++k) {
@@ -951,12 +950,12 @@ normalized_fwd_scatter_kernel(const T* __restrict__ x, const T* __restrict__ w,
 // log_C.
 template <typename A, bool LOGW>
 __global__ __launch_bounds__(256) void normalized_fixup_kernel(
-    int H, int W, int TH, int TW, int ntw, int nth, int spill_stride, int ring_stride,
+    int H, int W, int TH, int TW, TileGrid tg, int spill_stride, int ring_stride,
     const int* __restrict__ hdr, const A* __restrict__ spill, const A* __restrict__ part,
     int64_t ntiles, A* __restrict__ Dout, A* __restrict__ Lout) {
     const int R = __builtin_amdgcn_readfirstlane(hdr[0]);
     if (R == 0) return;
-    const FixTile f = fix_tile(blockIdx.x, H, W, TH, TW, ntw, nth);
+    const FixTile f = fix_tile(blockIdx.x, H, W, TH, TW, tg);
     const int64_t HW = static_cast<int64_t>(H) * W;
     const A* pm = part + 3 * static_cast<int64_t>(blockIdx.x) * ring_stride;
     int lg;
@@ -1068,14 +1067,18 @@ struct NTileGeo : SGeo<VEC, ROWS, TPR, true, HALO> {
 // 16-byte load or store per shift, and the LDS tiles use the de-interleaved
 // columns of BwdLayout (conflict-free for these lanes).  Otherwise the lanes
 // are strided (pixels tx, tx + TPR, ...) with row-major tiles.
-template <typename T, int VEC, int TPR, int ROWS, int D, bool LOGW, bool CONTIG,
+// NTS: streaming stores of gw, where whole rows are whole 128-byte lines or the
+// lanes store fp32 vectors, as in accumulate_uz's backward (R = 5, streaming ->
+// plain elsewhere: 3 x 1100 x 1500 fp16 551 -> 443 us, 8 x 3 x 250^2 fp32 267 ->
+// 237 us, 1500^2 fp64 687 -> 583 us; kept streaming: 1500^2 fp32 315 against 336).
+template <typename T, int VEC, int TPR, int ROWS, int D, bool LOGW, bool CONTIG, bool NTS,
           int WPE = kScatterWavesPerEU<TPR * ROWS>, int HALO = kRmax>
 __global__ __launch_bounds__(TPR * ROWS, WPE) void
 normalized_bwd_scatter_kernel(const T* __restrict__ x, const T* __restrict__ w,
                               const acc_t<T>* __restrict__ Dg, const acc_t<T>* __restrict__ Lg,
                               const acc_t<T>* __restrict__ gDg, const acc_t<T>* __restrict__ gLg,
                               const int64_t* __restrict__ shifts, int S, int codes, int C, int H,
-                              int W, int ntw, int nth, int64_t plane_step, T* __restrict__ gx,
+                              int W, TileGrid tg, int64_t plane_step, T* __restrict__ gx,
                               acc_t<T>* __restrict__ gxp, T* __restrict__ gw,
                               int* __restrict__ hdr, acc_t<T>* __restrict__ spill) {
     using A = acc_t<T>;
@@ -1096,7 +1099,7 @@ normalized_bwd_scatter_kernel(const T* __restrict__ x, const T* __restrict__ w,
     A* mg = bt + G::TILE;
 
     const int64_t t = xcd_tile(blockIdx.x, gridDim.x);
-    const TileIdx ti = tile_of(t, ntw, nth, G::TH, G::TW);
+    const TileIdx ti = tile_of(t, tg, G::TH, G::TW, H, W);
     const int64_t HW = static_cast<int64_t>(H) * W;
     const int64_t off = ti.bc * HW;
     const T* xp = x + off;
@@ -1139,9 +1142,9 @@ normalized_bwd_scatter_kernel(const T* __restrict__ x, const T* __restrict__ w,
     const int h = ti.h0 + ty;
     // The lane's pixels: column, activity and in-plane offset of pixel k,
     // and its LDS index displaced by (dx, dy).
-    const LanePix<VEC, TPR> px = lane_pixels<VEC, TPR>(h, ti.w0, tx, H, W);  // strided form
+    const LanePix<VEC, TPR> px = lane_pixels<VEC, TPR>(ti, ty, tx, W);  // strided form
     const int wq0 = ti.w0 + tx * VEC;                                          // contiguous form
-    const bool cact = h < H && wq0 < W;
+    const bool cact = ty < ti.th && tx * VEC < ti.tw;
     const uint32_t cown = static_cast<uint32_t>(cact ? h : 0) * static_cast<uint32_t>(W) +
                           static_cast<uint32_t>(cact ? wq0 : 0);
     auto pcol = [&](int k) { return CONTIG ? wq0 + k : ti.w0 + tx + k * TPR; };
@@ -1161,10 +1164,10 @@ normalized_bwd_scatter_kernel(const T* __restrict__ x, const T* __restrict__ w,
     using Slot = std::conditional_t<CONTIG, SlotRaw<T, VEC>, PixSlot<T, VEC>>;
     auto slot_fill = [&](const T* wp, Slot& sl) {
         if constexpr (CONTIG)
-            slot_load_at<T, VEC, kNormBwdNT<T>>(wp, cown * static_cast<uint32_t>(sizeof(T)),
+            slot_load_at<T, VEC, kNormBwdNT<T, TPR>>(wp, cown * static_cast<uint32_t>(sizeof(T)),
                                                        sl);
         else
-            slot_load_pixels<T, VEC, TPR, kNormBwdNT<T>>(wp, px, sl);
+            slot_load_pixels<T, VEC, TPR, kNormBwdNT<T, TPR>>(wp, px, sl);
     };
     auto slot_take = [&](const Slot& sl, A (&wv)[VEC]) {
         if constexpr (CONTIG)
@@ -1219,7 +1222,7 @@ normalized_bwd_scatter_kernel(const T* __restrict__ x, const T* __restrict__ w,
     // Interior tiles (every pixel and every q + s inside the image for all
     // rows of the table): no forward-box test and no mirror mask.
     const int R_all = table_radius(shl, S, false);
-    const bool interior = ti.h0 >= R_all && ti.h0 + G::TH + R_all <= H && ti.w0 >= R_all &&
+    const bool interior = ti.th == G::TH && ti.tw == G::TW && ti.h0 >= R_all && ti.h0 + G::TH + R_all <= H && ti.w0 >= R_all &&
                           ti.w0 + G::TW + R_all <= W;
     int last_dx = kClamp;
     auto step = [&](int s, Slot& slot, auto fast_tag) {
@@ -1244,7 +1247,7 @@ normalized_bwd_scatter_kernel(const T* __restrict__ x, const T* __restrict__ w,
                 if constexpr (FAST) {
                     gv[k] = grad_w(k, wv[k], xt[i], lt[i], at[i], bt[i], rc.inv, fo);
                     if constexpr (!CONTIG)
-                        store_elem_at<T, true>(gs, px.own[k] * static_cast<uint32_t>(sizeof(T)),
+                        store_elem_at<T, NTS>(gs, px.own[k] * static_cast<uint32_t>(sizeof(T)),
                                                from_acc<T>(gv[k]));
                     mg[i] += fo * ao[k];
                 } else {
@@ -1253,7 +1256,7 @@ normalized_bwd_scatter_kernel(const T* __restrict__ x, const T* __restrict__ w,
                     gv[k] = grad_w(k, wk, xt[i], lt[i], at[i], bt[i], okp, fo);
                     if constexpr (!CONTIG)
                         if (px.act[k])
-                            store_elem_at<T, true>(
+                            store_elem_at<T, NTS>(
                                 gs, px.own[k] * static_cast<uint32_t>(sizeof(T)), from_acc<T>(gv[k]));
                     // x-gradient term of q + s: f(w_s[q], L[q]) gD[q]
                     mg[i] += pact(k) ? fo * ao[k] : A(0);
@@ -1261,7 +1264,7 @@ normalized_bwd_scatter_kernel(const T* __restrict__ x, const T* __restrict__ w,
             }
             if constexpr (CONTIG)
                 if (FAST || cact)
-                    store_acc_at<T, VEC, true>(gs, cown * static_cast<uint32_t>(sizeof(T)), gv);
+                    store_acc_at<T, VEC, NTS>(gs, cown * static_cast<uint32_t>(sizeof(T)), gv);
         }
         gs += plane_step;
     };
@@ -1325,8 +1328,7 @@ normalized_bwd_scatter_kernel(const T* __restrict__ x, const T* __restrict__ w,
             gx[off + pown(k)] = from_acc<T>(v);
     }
     if (R == 0) return;
-    const int th = min(G::TH, H - ti.h0);
-    const int tw = min(G::TW, W - ti.w0);
+    const int th = ti.th, tw = ti.tw;
     const int n = spill_count(th, tw, R);
     A* sg = spill + t * G::SPILL;
     for (int e = threadIdx.x; e < n; e += blockDim.x) {
@@ -1424,12 +1426,16 @@ static int n_launch_bwd(const void* x, const void* w, const void* D, const void*
 // nontemporal).  fp32 backward: 32 lanes per row (128 x 32 tiles, one
 // workgroup per CU): c3 positive 0.690 -> 0.666 ms; the 16-bit backward
 // stays at 16 (c2 logits 0.236 ms against 0.254 ms on the wide tiles).
-template <typename T, bool BWD, bool NARROW = false>
+// Images of at most 64 columns take the fp32 passes on 64 x 32 tiles (SLIM):
+// half the lanes of a 128-wide tile would idle.
+constexpr int kNSlimWidth = 64;
+template <typename T, bool BWD, bool NARROW = false, bool SLIM = false>
 struct NScatterCfg {
+    static_assert(!SLIM || sizeof(T) == 4, "the other types' tiles are 64 wide or less");
     static_assert(!NARROW || (BWD && sizeof(T) == 8), "the narrow border serves the fp64 backward");
     static constexpr bool kWide = sizeof(T) != 8;
     static constexpr int VEC = sizeof(T) == 8 ? 2 : 4;
-    static constexpr int TPR = (kWide && sizeof(T) == 4) ? 32 : kTPR;
+    static constexpr int TPR = (kWide && sizeof(T) == 4 && !SLIM) ? 32 : kTPR;
     // fp64 forward: 32 x 16 tiles (twice the workgroups; c3 0.083 -> 0.080
     // ms).  fp64 backward: 32 x 32 tiles, or on the narrow border 32 x 16
     // (three 256-lane workgroups per CU: the c3 fp64 shape's 768 tiles in one
@@ -1451,34 +1457,44 @@ struct NScatterCfg {
 
 constexpr size_t kNScatterLds = 160 * 1024 - 1024;
 constexpr int64_t kNHeader = 256;
+// A gradient this small stays in the 256 MB Infinity Cache, which joins the
+// streamed parts of a line (4 x 250^2 fp64 R = 6 backward 84 us, plain 100).
+constexpr int64_t kNCachedBytes = int64_t(192) << 20;
+// Smaller images are mostly border; the gather kernels read them from the
+// caches.  From here on every tile is at least kRmax wide and high
+// (nsh_host::tile_grid), so a window's border reaches only adjacent tiles
+// (with one tile in a direction, the tile itself, as on a torus).
+constexpr int kNScatterMinSide = 32;
 
 struct NPlan {
     bool ok = false;
     bool narrow = false;  // the backward on the narrow border (NScatterCfg<T, true, true>)
-    int ntw = 0, nth = 0, spill = 0, ring = 0;
+    bool slim = false;    // 64-wide fp32 tiles (NScatterCfg<T, BWD, false, true>)
+    int spill = 0, ring = 0;
+    TileGrid grid{};
     int64_t tiles = 0, spill_bytes = 0, part_bytes = 0, total = 0;
     size_t lds = 0;
 };
 
 static int64_t n_align256(int64_t b) { return (b + 255) / 256 * 256; }
 
-template <typename T, bool BWD, bool NARROW = false>
+template <typename T, bool BWD, bool NARROW = false, bool SLIM = false>
 static NPlan n_plan_cfg(const NDims& d) {
-    using Cfg = NScatterCfg<T, BWD, NARROW>;
+    using Cfg = NScatterCfg<T, BWD, NARROW, SLIM>;
     using G = typename Cfg::G;
     constexpr bool bwd = BWD;
     const int64_t ab = sizeof(acc_t<T>);
     NPlan p;
     p.narrow = NARROW;
-    p.ntw = static_cast<int>(nsh_host::ceil_div(d.W, G::TW));
-    p.nth = static_cast<int>(nsh_host::ceil_div(d.H, G::TH));
-    p.tiles = static_cast<int64_t>(d.B) * d.C * p.ntw * p.nth;
+    p.slim = SLIM;
+    p.grid = nsh_host::tile_grid(d.H, d.W, G::TH, G::TW);
+    p.tiles = static_cast<int64_t>(d.B) * d.C * p.grid.ntw * p.grid.nth;
     p.lds = shift_lds_bytes(d.S) +
             (bwd ? 5 : 4) * static_cast<size_t>(G::TILE) * ab;
     p.spill = G::SPILL;
     p.ring = G::RING;
-    p.ok = p.ntw >= 2 && p.nth >= 2 && d.W - (p.ntw - 1) * G::TW >= kRmax &&
-           d.H - (p.nth - 1) * G::TH >= kRmax && p.lds <= kNScatterLds;
+    p.ok = p.grid.narrow >= kRmax && d.H >= kNScatterMinSide && d.W >= kNScatterMinSide &&
+           p.lds <= kNScatterLds;
     p.spill_bytes = n_align256((bwd ? 1 : 3) * p.tiles * p.spill * ab);
     if (bwd)
         p.part_bytes = sizeof(T) < sizeof(acc_t<T>)
@@ -1493,13 +1509,16 @@ static NPlan n_plan_cfg(const NDims& d) {
 // The plan; the fp64 backward on the narrow border when the caller's hint
 // asks for it (d.narrow) and `narrow` allows it.
 template <typename T>
-static NPlan n_plan(const NDims& d, bool bwd, bool narrow = true) {
+static NPlan n_plan(const NDims& d, bool bwd, bool narrow = true, bool slim = true) {
     if constexpr (sizeof(T) == 8) {
         if (bwd && narrow && d.narrow) {
             const NPlan p = n_plan_cfg<T, true, true>(d);
             if (p.ok) return p;
         }
     }
+    if constexpr (sizeof(T) == 4)
+        if (slim && d.W <= kNSlimWidth)
+            return bwd ? n_plan_cfg<T, true, false, true>(d) : n_plan_cfg<T, false, false, true>(d);
     return bwd ? n_plan_cfg<T, true>(d) : n_plan_cfg<T, false>(d);
 }
 
@@ -1519,11 +1538,11 @@ static bool n_use_scatter(const NPlan& p, void* ws, int64_t ws_bytes) {
 
 // NH > 1: w is a head stack (S*B, NH, H, W) mixed by mix (C, NH) in the
 // kernel's weight load.
-template <typename T, bool LOGW, int NH = 1>
-static int n_scatter_fwd(const void* x, const void* w, const int64_t* sh, NDims d, void* D,
+template <typename T, bool LOGW, int NH = 1, bool SLIM = false>
+static int n_scatter_fwd_cfg(const void* x, const void* w, const int64_t* sh, NDims d, void* D,
                          void* L, const NPlan& p, void* ws, int* weights_ok, hipStream_t st,
                          const acc_t<T>* mix = nullptr) {
-    using Cfg = NScatterCfg<T, false>;
+    using Cfg = NScatterCfg<T, false, false, SLIM>;
     using A = acc_t<T>;
     constexpr int V = Cfg::VEC, TPR = Cfg::TPR, RW = Cfg::ROWS;
     char* base = static_cast<char*>(ws);
@@ -1534,22 +1553,32 @@ static int n_scatter_fwd(const void* x, const void* w, const int64_t* sh, NDims 
     hipLaunchKernelGGL((normalized_fwd_scatter_kernel<T, V, TPR, RW, Cfg::D, LOGW, Cfg::WPE, NH>),
                        dim3(static_cast<unsigned>(p.tiles)), dim3(TPR * RW), p.lds, st,
                        static_cast<const T*>(x), static_cast<const T*>(w), sh, d.S, d.codes, d.C, d.H, d.W,
-                       p.ntw, p.nth, step, static_cast<A*>(D), static_cast<A*>(L), hdr, spill, part,
+                       p.grid, step, static_cast<A*>(D), static_cast<A*>(L), hdr, spill, part,
                        p.ring, p.tiles, mix, weights_ok);
     if (int rc = nsh_host::check_launch("normalized_accumulate_uz_forward")) return rc;
     hipLaunchKernelGGL((normalized_fixup_kernel<A, LOGW>), dim3(static_cast<unsigned>(p.tiles)),
-                       dim3(256), 0, st, d.H, d.W, RW, TPR * V, p.ntw, p.nth, p.spill, p.ring,
+                       dim3(256), 0, st, d.H, d.W, RW, TPR * V, p.grid, p.spill, p.ring,
                        static_cast<const int*>(hdr), static_cast<const A*>(spill),
                        static_cast<const A*>(part), p.tiles, static_cast<A*>(D),
                        static_cast<A*>(L));
     return nsh_host::check_launch("normalized_accumulate_uz_forward (fix-up)");
 }
 
-template <typename T, bool LOGW, bool NARROW>
+template <typename T, bool LOGW, int NH = 1>
+static int n_scatter_fwd(const void* x, const void* w, const int64_t* sh, NDims d, void* D,
+                         void* L, const NPlan& p, void* ws, int* weights_ok, hipStream_t st,
+                         const acc_t<T>* mix = nullptr) {
+    if constexpr (sizeof(T) == 4 && NH == 1)
+        if (p.slim)
+            return n_scatter_fwd_cfg<T, LOGW, 1, true>(x, w, sh, d, D, L, p, ws, weights_ok, st);
+    return n_scatter_fwd_cfg<T, LOGW, NH>(x, w, sh, d, D, L, p, ws, weights_ok, st, mix);
+}
+
+template <typename T, bool LOGW, bool NARROW, bool SLIM = false>
 static int n_scatter_bwd_cfg(const void* x, const void* w, const void* D, const void* L,
                              const void* gD, const void* gL, const int64_t* sh, NDims d, void* gx,
                              void* gw, const NPlan& p, void* ws, hipStream_t st) {
-    using Cfg = NScatterCfg<T, true, NARROW>;
+    using Cfg = NScatterCfg<T, true, NARROW, SLIM>;
     using A = acc_t<T>;
     constexpr int V = Cfg::VEC, TPR = Cfg::TPR, RW = Cfg::ROWS;
     char* base = static_cast<char*>(ws);
@@ -1561,29 +1590,38 @@ static int n_scatter_bwd_cfg(const void* x, const void* w, const void* D, const 
     const size_t vb = static_cast<size_t>(V) * sizeof(T);
     const bool contig = V == 4 && d.W % V == 0 && nsh_host::aligned(x, vb) &&
                         nsh_host::aligned(w, vb) && nsh_host::aligned(gw, vb);
-#define NSH_NBWD_LAUNCH(CT_)                                                                    \
-    hipLaunchKernelGGL((normalized_bwd_scatter_kernel<T, V, TPR, RW, Cfg::D, LOGW, CT_,      \
-                                                      Cfg::WPE, Cfg::HALO>),                    \
-                       dim3(static_cast<unsigned>(p.tiles)), dim3(TPR * RW), p.lds, st,         \
-                       static_cast<const T*>(x), static_cast<const T*>(w),                      \
-                       static_cast<const A*>(D), static_cast<const A*>(L),                      \
-                       static_cast<const A*>(gD), static_cast<const A*>(gL), sh, d.S, d.codes,  \
-                       d.C, d.H, d.W, p.ntw, p.nth, step, static_cast<T*>(gx), part,            \
-                       static_cast<T*>(gw),                                                     \
-                       hdr, spill)
+    const bool lines = static_cast<int64_t>(d.W) * sizeof(T) % 128 == 0;
+    const bool small = step * d.S * static_cast<int64_t>(sizeof(T)) < kNCachedBytes;
+    const bool stream = lines || (contig && (sizeof(T) == 4 || small)) || (V == 2 && small);
+    auto go = [&](auto contig_tag, auto nts_tag) {
+        hipLaunchKernelGGL((normalized_bwd_scatter_kernel<T, V, TPR, RW, Cfg::D, LOGW,
+                                                          decltype(contig_tag)::value,
+                                                          decltype(nts_tag)::value, Cfg::WPE,
+                                                          Cfg::HALO>),
+                           dim3(static_cast<unsigned>(p.tiles)), dim3(TPR * RW), p.lds, st,
+                           static_cast<const T*>(x), static_cast<const T*>(w),
+                           static_cast<const A*>(D), static_cast<const A*>(L),
+                           static_cast<const A*>(gD), static_cast<const A*>(gL), sh, d.S, d.codes,
+                           d.C, d.H, d.W, p.grid, step, static_cast<T*>(gx), part,
+                           static_cast<T*>(gw), hdr, spill);
+    };
     if constexpr (V == 4) {
-        if (contig)
-            NSH_NBWD_LAUNCH(true);
+        if (contig && stream)
+            go(std::true_type{}, std::true_type{});
+        else if (contig)
+            go(std::true_type{}, std::false_type{});
         else
-            NSH_NBWD_LAUNCH(false);
+            go(std::false_type{}, std::false_type{});
     } else {
-        NSH_NBWD_LAUNCH(false);
+        if (stream)
+            go(std::false_type{}, std::true_type{});
+        else
+            go(std::false_type{}, std::false_type{});
     }
-#undef NSH_NBWD_LAUNCH
     if (int rc = nsh_host::check_launch("normalized_accumulate_uz_backward")) return rc;
     constexpr bool kPart = sizeof(T) < sizeof(A);
     hipLaunchKernelGGL((spill_fixup_kernel<T, A, 1, kPart>), dim3(static_cast<unsigned>(p.tiles)),
-                       dim3(256), 0, st, d.H, d.W, RW, TPR * V, p.ntw, p.nth, p.spill,
+                       dim3(256), 0, st, d.H, d.W, RW, TPR * V, p.grid, p.spill,
                        static_cast<const int*>(hdr), static_cast<const A*>(spill), p.tiles,
                        static_cast<const A*>(part), static_cast<T*>(gx), static_cast<T*>(nullptr));
     return nsh_host::check_launch("normalized_accumulate_uz_backward (fix-up)");
@@ -1597,16 +1635,23 @@ static int n_scatter_bwd(const void* x, const void* w, const void* D, const void
         if (p.narrow)
             return n_scatter_bwd_cfg<T, LOGW, true>(x, w, D, L, gD, gL, sh, d, gx, gw, p, ws, st);
     }
+    if constexpr (sizeof(T) == 4) {
+        if (p.slim)
+            return n_scatter_bwd_cfg<T, LOGW, false, true>(x, w, D, L, gD, gL, sh, d, gx, gw, p,
+                                                           ws, st);
+    }
     return n_scatter_bwd_cfg<T, LOGW, false>(x, w, D, L, gD, gL, sh, d, gx, gw, p, ws, st);
 }
 
-// Either plan may run (n_run_bwd takes the 8-pixel border when the workspace
-// is too small for the narrow one): the larger of the two.
+// Any of the plans may run (n_run_bwd takes the 8-pixel border when the
+// workspace is too small for the narrow one, the head-mixed forward the wide
+// tiles): the largest.
 template <typename T>
 static int64_t n_workspace(const NDims& d, bool bwd) {
     const NPlan p = n_plan<T>(d, bwd, false);
     const NPlan q = n_plan<T>(d, bwd);
-    return std::max(p.ok ? p.total : 0, q.ok ? q.total : 0);
+    const NPlan r = n_plan<T>(d, bwd, false, false);
+    return std::max({p.ok ? p.total : 0, q.ok ? q.total : 0, r.ok ? r.total : 0});
 }
 
 template <typename T, bool LOGW>
@@ -1720,7 +1765,7 @@ static int n_run_fwd_mixed(const void* x, const void* hw, const void* mix, const
                            nsh::NDims d, int heads, void* D, void* L, void* ws, int64_t nws,
                            hipStream_t st) {
     using A = nsh::acc_t<T>;
-    const nsh::NPlan p = nsh::n_plan<T>(d, false);
+    const nsh::NPlan p = nsh::n_plan<T>(d, false, true, false);
     if (!nsh::n_use_scatter<T>(p, ws, nws))
         return fail(NSH_ERR_UNSUPPORTED,
                     "normalized_accumulate_uz_forward_mixed: shape or workspace not served by "

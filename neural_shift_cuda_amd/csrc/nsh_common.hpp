@@ -277,6 +277,9 @@ constexpr int kCodesRows = 1;
 constexpr int kCodesSharedW = 2;
 constexpr int kCodesPeriodic = 4;
 constexpr int kCodesBox = 8;
+// accumulate_uz's scatter forward: rows and buffers fit the lanes' vectors
+// (set by the launcher; only its gather form inside the launch asks).
+constexpr int kCodesVec = 16;
 
 // The kernels' `codes` from the flags a call ORs into its dtype argument.
 __host__ __forceinline__ int dtype_codes(int dtype) {
@@ -402,6 +405,16 @@ __device__ __forceinline__ int64_t xcd_tile(int64_t bid, int64_t nblocks) {
 struct TileIdx {
     int64_t bc;  // plane index b*C + c
     int h0, w0;  // top-left pixel of the tile
+    int th, tw;  // its extent inside the image (scatter grids only)
+};
+
+// The tiles of a scatter launch.  Tile row r starts at r * TH, except that
+// the last one starts at hl, and columns likewise at wl: a last row of tiles
+// that would be narrower than the tables' radius takes rows from the one
+// before (tile_grid), so that a window's border still reaches only adjacent
+// tiles.  `narrow` is the smallest extent of any tile in the grid.
+struct TileGrid {
+    int ntw, nth, wl, hl, narrow;
 };
 
 // Tile t of the launch.  order 0: the tiles of a plane row-major; order 2:
@@ -429,6 +442,21 @@ __device__ __forceinline__ TileIdx tile_of(int64_t t, int ntw, int nth, int TH, 
     }
     r.h0 = tr * TH;
     r.w0 = tc * TW;
+    return r;
+}
+
+__device__ __forceinline__ TileIdx tile_of(int64_t t, const TileGrid& g, int TH, int TW, int H,
+                                           int W) {
+    const int64_t per_plane = static_cast<int64_t>(g.ntw) * g.nth;
+    TileIdx r;
+    r.bc = t / per_plane;
+    const int rem = static_cast<int>(t - r.bc * per_plane);
+    const int tr = rem / g.ntw, tc = rem - tr * g.ntw;
+    const bool lr = tr == g.nth - 1, lc = tc == g.ntw - 1;
+    r.h0 = lr ? g.hl : tr * TH;
+    r.w0 = lc ? g.wl : tc * TW;
+    r.th = min(lr ? H - g.hl : TH, (tr == g.nth - 2 ? g.hl : H) - r.h0);
+    r.tw = min(lc ? W - g.wl : TW, (tc == g.ntw - 2 ? g.wl : W) - r.w0);
     return r;
 }
 
