@@ -86,7 +86,7 @@ extern "C" {
  * device, so any table gives the same results with or without it (a table
  * of radius <= 8 runs on the wider border, one above 16 in the gather
  * form).  An extension with no counterpart in the reference. */
-#define NSH_WIDE_HALO 0x400
+#define NSH_WIDE_HALO 0x400 /* also taken by the normalized_accumulate_uz calls */
 /* The same hint for a radius in 17..24 (a 24-pixel border; the half-plane
  * tables up to R = 22, S = 1013, the largest the 1 <= S <= 1024 contract
  * admits).  NSH_WIDE_HALO is ignored when both are set. */

@@ -322,6 +322,19 @@ def _halo_flag(shifts: torch.Tensor) -> int:
     return NSH_WIDER_HALO if 16 < r <= 24 else 0
 
 
+# The normalized passes take the wide border too (fp32 and 16-bit), but ask
+# for the radius, a device read on a table's first use, only where it can
+# matter: half-plane tables of up to 8 pixels have at most 145 rows.
+_HALO8_HALF_ROWS = 2 * 8 * 8 + 2 * 8 + 1
+
+
+def _norm_halo_flag(shifts: torch.Tensor, dtype: torch.dtype) -> int:
+    """NSH_WIDE_HALO for the normalized passes, as _halo_flag."""
+    if dtype == torch.float64 or shifts.size(0) <= _HALO8_HALF_ROWS:
+        return 0
+    return _halo_flag(shifts) & NSH_WIDE_HALO
+
+
 def _band_args(band) -> tuple:
     """(row_origin, image_height) of a band call, checked."""
     org, hg = (int(v) for v in band)
@@ -415,7 +428,8 @@ def normalized_accumulate_uz_forward(x: torch.Tensor, weights: torch.Tensor, shi
                                     "normalized_accumulate_uz: weights must be (S*B, C, H, W)",
                                     shared_weights)
     acc = _acc_dtype(x.dtype)
-    code = _code(x, "normalized_accumulate_uz_fwd") | _flags(row_codes, shared_weights, rules)
+    code = (_code(x, "normalized_accumulate_uz_fwd") | _flags(row_codes, shared_weights, rules)
+            | _norm_halo_flag(shifts, x.dtype))
     if weights_ok is not None:
         _check(weights_ok.device == x.device and weights_ok.dtype == torch.int32
                and weights_ok.numel() == 1,
@@ -459,7 +473,8 @@ def normalized_accumulate_uz_forward_mixed(x: torch.Tensor, head_weights: torch.
            f"{op}: head_mix must be (C, heads)")
     acc = _acc_dtype(x.dtype)
     mix = head_mix.detach().to(device=x.device, dtype=acc).contiguous()
-    code = _code(x, op) | _flags(row_codes, False, rules)
+    code = (_code(x, op) | _flags(row_codes, False, rules)
+            | _norm_halo_flag(shifts, x.dtype))
     D = torch.empty(x.shape, dtype=acc, device=x.device)
     L = torch.empty(x.shape, dtype=acc, device=x.device)
     ws, nws = _norm_workspace(S, B, C, H, W, code, False, x.device)
@@ -555,7 +570,8 @@ def normalized_accumulate_uz_backward(x: torch.Tensor, weights: torch.Tensor, D:
     gL = _grad_in(grad_log_C, x, acc, "grad_log_C")
     gx = torch.empty_like(x)
     gw = torch.empty((S * B, C, H, W), dtype=weights.dtype, device=weights.device)
-    code = _code(x, "normalized_accumulate_uz_bwd") | _flags(row_codes, shared_weights, rules)
+    code = (_code(x, "normalized_accumulate_uz_bwd") | _flags(row_codes, shared_weights, rules)
+            | _norm_halo_flag(shifts, x.dtype))
     if x.dtype == torch.float64:
         code |= _narrow_halo_flag(sh)
     ws, nws = _norm_workspace(S, B, C, H, W, code, True, x.device)

@@ -664,10 +664,22 @@ __device__ __forceinline__ void mixed_pixels(PixSlot<T, VEC> (&slot)[NH], const 
     }
 }
 
+// Tile geometry with a HALO border: SGeo's, or rows at the plain LW pitch for
+// the other borders where a row of lanes covers every bank at any pitch: the
+// narrow one (fp64, 16 lanes of 8 bytes; the NSH_NARROW_HALO hint), so that
+// three 256-lane workgroups share a CU, and the forward's wide one (32 lanes
+// of 4 bytes; NSH_WIDE_HALO), whose four arrays would not fit otherwise.
+template <int VEC, int ROWS, int TPR, int HALO, bool PLAIN = HALO != kRmax>
+struct NTileGeo : SGeo<VEC, ROWS, TPR, true, HALO> {
+    using Base = SGeo<VEC, ROWS, TPR, true, HALO>;
+    static constexpr int PITCH = PLAIN ? Base::LW : Base::PITCH;
+    static constexpr int TILE = Base::LH * PITCH;
+};
+
 // NH > 1: w is the head stack (S*B, NH, H, W), plane_step = B * NH * H * W,
 // and mix the (C, NH) mixing matrix in the accumulator type.
 template <typename T, int VEC, int TPR, int ROWS, int D, bool LOGW,
-          int WPE = kScatterWavesPerEU<TPR * ROWS>, int NH = 1>
+          int WPE = kScatterWavesPerEU<TPR * ROWS>, int NH = 1, int HALO = kRmax>
 __global__ __launch_bounds__(TPR * ROWS, WPE) void
 normalized_fwd_scatter_kernel(const T* __restrict__ x, const T* __restrict__ w,
                               const int64_t* __restrict__ shifts, int S, int codes, int C, int H,
@@ -677,7 +689,7 @@ normalized_fwd_scatter_kernel(const T* __restrict__ x, const T* __restrict__ w,
                               int ring_stride, int64_t ntiles,
                               const acc_t<T>* __restrict__ mix, int* __restrict__ weights_ok) {
     using A = acc_t<T>;
-    using G = SGeo<VEC, ROWS, TPR>;
+    using G = NTileGeo<VEC, ROWS, TPR, HALO>;
     extern __shared__ __align__(16) unsigned char smem[];
     int4* shl = reinterpret_cast<int4*>(smem);
     A* xt = reinterpret_cast<A*>(smem + shift_lds_bytes(S));
@@ -691,8 +703,8 @@ normalized_fwd_scatter_kernel(const T* __restrict__ x, const T* __restrict__ w,
     const int64_t off = ti.bc * HW;
     const T* xp = x + off;
     stage_shifts(shl, shifts, S, 3, H, W, codes);
-    stage_tile<T, A>(xt, xp, H, W, ti.h0, ti.w0, G::LH, G::LW, G::PITCH);
-    const int R = near_radius(shl, S, true);
+    stage_tile<T, A>(xt, xp, H, W, ti.h0, ti.w0, G::LH, G::LW, G::PITCH, HALO);
+    const int R = near_radius<HALO>(shl, S, true);
     if (blockIdx.x == 0 && threadIdx.x == 0) hdr[0] = R;  // for the fix-up
     const A m0 = empty_m<A, LOGW>();
     // the window is also used at R = 0 by a (0, 0) mirror row
@@ -707,7 +719,7 @@ normalized_fwd_scatter_kernel(const T* __restrict__ x, const T* __restrict__ w,
     const int ty = threadIdx.x / TPR;
     const int h = ti.h0 + ty;
     const LanePix<VEC, TPR> px = lane_pixels<VEC, TPR>(ti, ty, tx, W);
-    const int lc = (ty + kRmax) * G::PITCH + tx + kRmax;  // pixel k at lc + k*TPR
+    const int lc = (ty + HALO) * G::PITCH + tx + HALO;  // pixel k at lc + k*TPR
     const int64_t b = ti.bc / C;
     const int64_t ch = ti.bc - b * C;
     const bool wsh = (codes & kCodesSharedW) != 0;
@@ -757,7 +769,7 @@ normalized_fwd_scatter_kernel(const T* __restrict__ x, const T* __restrict__ w,
         for (int j = 0; j < NH; ++j)
             slot_load_pixels<T, VEC, TPR, kNormFwdNT<T, TPR>>(wr + j * HW, px, slot[j]);
         wr += s + D + 1 < S ? wstep : 0;
-        if (shift_in_lds(rc)) {
+        if (shift_in_lds<HALO>(rc)) {
             const int op = lc + rc.dx * G::PITCH + rc.dy;  // window index of q + s
             if constexpr (MODE == 2) {
                 // Forward box: a w_s[q] whose q + s leaves the image is a
@@ -850,7 +862,7 @@ normalized_fwd_scatter_kernel(const T* __restrict__ x, const T* __restrict__ w,
     };
     for (int s = 0; s < S && px.any; ++s) {
         const ShiftRec rc = read_shift(shl, s);
-        if (shift_in_lds(rc)) continue;
+        if (shift_in_lds<HALO>(rc)) continue;
         const T* wp = w_bc + static_cast<int64_t>(s) * wstep;
         int hp = h + rc.dxm;
         hp -= hp >= H ? H : 0;
@@ -938,7 +950,7 @@ normalized_fwd_scatter_kernel(const T* __restrict__ x, const T* __restrict__ w,
     for (int e = threadIdx.x; e < n; e += blockDim.x) {
         int i, j;
         spill_coords(e, th, tw, R, i, j);
-        const int li = (i + kRmax) * G::PITCH + j + kRmax;
+        const int li = (i + HALO) * G::PITCH + j + HALO;
         s0p[e] = wm[li];
         s1p[e] = wu[li];
         s2p[e] = wz[li];
@@ -1050,21 +1062,9 @@ __device__ __forceinline__ A frac_log(A kw, A key) {
     return Lim<A>::ex(kw - key);
 }
 
-// Tile geometry of the backward with a HALO border: SGeo's, or for the
-// narrow border (fp64, tables within it: the NSH_NARROW_HALO hint) rows at the
-// plain LW pitch -- its 8-byte elements are read as 16-lane rows of 128 bytes,
-// which cover every bank at any pitch -- so that three 256-lane workgroups
-// share a CU.
-template <int VEC, int ROWS, int TPR, int HALO>
-struct NTileGeo : SGeo<VEC, ROWS, TPR, true, HALO> {
-    using Base = SGeo<VEC, ROWS, TPR, true, HALO>;
-    static constexpr int PITCH = HALO == kRmax ? Base::PITCH : Base::LW;
-    static constexpr int TILE = Base::LH * PITCH;
-};
-
-// CONTIG (VEC = 4, W a multiple of 4, 16-byte aligned tensors): lane tx owns
-// the four consecutive pixels 4 tx .. 4 tx + 3 of its row, moved with one
-// 16-byte load or store per shift, and the LDS tiles use the de-interleaved
+// CONTIG (W a multiple of VEC = 4, or 2 on the wide border, and tensors aligned
+// for it): lane tx owns VEC consecutive pixels of its row, moved with one
+// vector load or store per shift, and the LDS tiles use the de-interleaved
 // columns of BwdLayout (conflict-free for these lanes).  Otherwise the lanes
 // are strided (pixels tx, tx + TPR, ...) with row-major tiles.
 // NTS: streaming stores of gw, where whole rows are whole 128-byte lines or the
@@ -1082,9 +1082,9 @@ normalized_bwd_scatter_kernel(const T* __restrict__ x, const T* __restrict__ w,
                               acc_t<T>* __restrict__ gxp, T* __restrict__ gw,
                               int* __restrict__ hdr, acc_t<T>* __restrict__ spill) {
     using A = acc_t<T>;
-    using G = NTileGeo<VEC, ROWS, TPR, HALO>;
-    static_assert(HALO == kRmax || !CONTIG, "the narrow border is built for strided lanes");
-    static_assert(!CONTIG || VEC == 4, "the contiguous form moves 4-pixel vectors");
+    using G = NTileGeo<VEC, ROWS, TPR, HALO, (HALO < kRmax)>;
+    static_assert(HALO >= kRmax || !CONTIG, "the narrow border is built for strided lanes");
+    static_assert(!CONTIG || VEC == 4 || VEC == 2, "the contiguous form moves vectors");
     // Column offset within a row: de-interleaved for the contiguous lanes
     // (the strided SGeo pitch is the BwdLayout pitch), row-major otherwise.
     using L = BwdLayout<VEC, G::LW, G::PITCH>;
@@ -1378,6 +1378,7 @@ struct NDims {
     int S, B, C, H, W;
     int codes = 0;  // kCodesRows / kCodesSharedW (from NSH_SHIFT_CODES, NSH_SHARED_WEIGHTS)
     bool narrow = false;  // NSH_NARROW_HALO: every row within 6 pixels (a hint)
+    bool wide = false;    // NSH_WIDE_HALO: the radius lies in 9..16 (a hint)
 };
 
 template <typename T, int VEC, bool LOGW>
@@ -1426,33 +1427,47 @@ static int n_launch_bwd(const void* x, const void* w, const void* D, const void*
 // nontemporal).  fp32 backward: 32 lanes per row (128 x 32 tiles, one
 // workgroup per CU): c3 positive 0.690 -> 0.666 ms; the 16-bit backward
 // stays at 16 (c2 logits 0.236 ms against 0.254 ms on the wide tiles).
-// Images of at most 64 columns take the fp32 passes on 64 x 32 tiles (SLIM):
-// half the lanes of a 128-wide tile would idle.
+// Variants:
+//  * kNNarrow: the fp64 backward on a 6-pixel border (NSH_NARROW_HALO): 32 x 16
+//    tiles, three 256-lane workgroups per CU (the c3 fp64 shape's 768 tiles in
+//    one round; 32 x 16 on the 8-pixel border, two workgroups per CU and 1.5
+//    rounds, measured no faster than 32 x 32; 1-pixel lanes on the narrow
+//    border, 24 waves per CU: no faster);
+//  * kNSlim: fp32 on 64 x 32 tiles for images of at most 64 columns, where half
+//    the lanes of a 128-wide tile would idle;
+//  * kNWide: a 16-pixel border for tables of radius 9..16 (NSH_WIDE_HALO; fp32
+//    and 16-bit): 64 x 32 tiles of 1024 lanes, 2 pixels each (one workgroup per
+//    CU: forward 98 KB of LDS plus the table, backward 143 KB).  On the 8-pixel
+//    border such tables' far rows take the gather loop, one row's loads at a
+//    time (half-plane R = 10, 221 rows, fp32: 1024^2 forward 524 -> 350 us,
+//    backward 1115 -> 471 us; 3 x 792^2 1308 -> 647 and 2886 -> 1108).  Bound by
+//    the loop's instructions and LDS latency at 16 waves per CU, not by the
+//    stream (fp16 takes as long): 4-pixel lanes, half the waves, 396 and 538 us.
+enum { kNBase = 0, kNNarrow = 1, kNSlim = 2, kNWide = 3 };
 constexpr int kNSlimWidth = 64;
-template <typename T, bool BWD, bool NARROW = false, bool SLIM = false>
+template <typename T, bool BWD, int VAR = kNBase>
 struct NScatterCfg {
+    static constexpr bool NARROW = VAR == kNNarrow, SLIM = VAR == kNSlim, WIDE = VAR == kNWide;
     static_assert(!SLIM || sizeof(T) == 4, "the other types' tiles are 64 wide or less");
     static_assert(!NARROW || (BWD && sizeof(T) == 8), "the narrow border serves the fp64 backward");
-    static constexpr bool kWide = sizeof(T) != 8;
-    static constexpr int VEC = sizeof(T) == 8 ? 2 : 4;
-    static constexpr int TPR = (kWide && sizeof(T) == 4 && !SLIM) ? 32 : kTPR;
-    // fp64 forward: 32 x 16 tiles (twice the workgroups; c3 0.083 -> 0.080
-    // ms).  fp64 backward: 32 x 32 tiles, or on the narrow border 32 x 16
-    // (three 256-lane workgroups per CU: the c3 fp64 shape's 768 tiles in one
-    // round); 32 x 16 on the 8-pixel border (two workgroups per CU, 1.5
-    // rounds) measured no faster.
+    static_assert(!WIDE || sizeof(T) <= 4, "fp64 tiles do not fit a 16-pixel border");
+    static constexpr int VEC = (sizeof(T) == 8 || WIDE) ? 2 : 4;
+    static constexpr int TPR = ((sizeof(T) == 4 && !SLIM) || WIDE) ? 32 : kTPR;
+    // fp64 forward: 32 x 16 tiles (twice the workgroups; c3 0.083 -> 0.080 ms)
     static constexpr int ROWS = ((!BWD || NARROW) && sizeof(T) == 8) ? 16 : 32;
-    static constexpr int HALO = NARROW ? 6 : kRmax;
+    static constexpr int HALO = NARROW ? 6 : (WIDE ? 16 : kRmax);
     // prefetch depth: 4 for the fp64 backward on the 8-pixel border, 2 on
-    // the narrow one (c3 fp64 0.189 ms at 4, 0.181 at 2, 0.191 at 6)
-    static constexpr int D = (BWD && sizeof(T) == 8 && !NARROW) ? 4 : 2;
+    // the narrow one (c3 fp64 0.189 ms at 4, 0.181 at 2, 0.191 at 6); on the
+    // wide one 2 forward and 4 backward (1024^2 R = 10 fp32: forward 350 us at
+    // 2, 373 at 4, backward 496 and 471, 460 at 8)
+    static constexpr int D = (BWD && (WIDE || (sizeof(T) == 8 && !NARROW))) ? 4 : 2;
     // register budget: a 1024-lane workgroup holds a CU alone (its LDS), so
     // four waves per SIMD; smaller ones two workgroups per CU, the narrow
-    // border's three (1-pixel lanes there, 32 per row and 24 waves per CU:
-    // no faster)
+    // border's three
     static constexpr int WPE = NARROW ? 3
                                       : (TPR * ROWS >= 1024 ? 4 : kScatterWavesPerEU<TPR * ROWS>);
-    using G = NTileGeo<VEC, ROWS, TPR, HALO>;
+    using G = std::conditional_t<BWD, NTileGeo<VEC, ROWS, TPR, HALO, (HALO < kRmax)>,
+                                 NTileGeo<VEC, ROWS, TPR, HALO>>;
 };
 
 constexpr size_t kNScatterLds = 160 * 1024 - 1024;
@@ -1468,8 +1483,7 @@ constexpr int kNScatterMinSide = 32;
 
 struct NPlan {
     bool ok = false;
-    bool narrow = false;  // the backward on the narrow border (NScatterCfg<T, true, true>)
-    bool slim = false;    // 64-wide fp32 tiles (NScatterCfg<T, BWD, false, true>)
+    int var = kNBase;
     int spill = 0, ring = 0;
     TileGrid grid{};
     int64_t tiles = 0, spill_bytes = 0, part_bytes = 0, total = 0;
@@ -1478,22 +1492,22 @@ struct NPlan {
 
 static int64_t n_align256(int64_t b) { return (b + 255) / 256 * 256; }
 
-template <typename T, bool BWD, bool NARROW = false, bool SLIM = false>
+template <typename T, bool BWD, int VAR = kNBase>
 static NPlan n_plan_cfg(const NDims& d) {
-    using Cfg = NScatterCfg<T, BWD, NARROW, SLIM>;
+    using Cfg = NScatterCfg<T, BWD, VAR>;
     using G = typename Cfg::G;
     constexpr bool bwd = BWD;
     const int64_t ab = sizeof(acc_t<T>);
     NPlan p;
-    p.narrow = NARROW;
-    p.slim = SLIM;
-    p.grid = nsh_host::tile_grid(d.H, d.W, G::TH, G::TW);
+    p.var = VAR;
+    constexpr int kReach = VAR == kNWide ? 16 : kRmax;  // the tables' largest radius
+    p.grid = nsh_host::tile_grid(d.H, d.W, G::TH, G::TW, kReach);
     p.tiles = static_cast<int64_t>(d.B) * d.C * p.grid.ntw * p.grid.nth;
     p.lds = shift_lds_bytes(d.S) +
             (bwd ? 5 : 4) * static_cast<size_t>(G::TILE) * ab;
     p.spill = G::SPILL;
     p.ring = G::RING;
-    p.ok = p.grid.narrow >= kRmax && d.H >= kNScatterMinSide && d.W >= kNScatterMinSide &&
+    p.ok = p.grid.narrow >= kReach && d.H >= kNScatterMinSide && d.W >= kNScatterMinSide &&
            p.lds <= kNScatterLds;
     p.spill_bytes = n_align256((bwd ? 1 : 3) * p.tiles * p.spill * ab);
     if (bwd)
@@ -1506,20 +1520,27 @@ static NPlan n_plan_cfg(const NDims& d) {
     return p;
 }
 
-// The plan; the fp64 backward on the narrow border when the caller's hint
-// asks for it (d.narrow) and `narrow` allows it.
-template <typename T>
-static NPlan n_plan(const NDims& d, bool bwd, bool narrow = true, bool slim = true) {
-    if constexpr (sizeof(T) == 8) {
-        if (bwd && narrow && d.narrow) {
-            const NPlan p = n_plan_cfg<T, true, true>(d);
-            if (p.ok) return p;
+// The plan: the variant that the caller's hint or the width asks for, where
+// it applies and `hints` allows it, else the base one.
+template <typename T, bool BWD>
+static NPlan n_plan(const NDims& d, bool hints = true) {
+    if (hints) {
+        if constexpr (sizeof(T) == 8 && BWD) {
+            if (d.narrow) {
+                const NPlan p = n_plan_cfg<T, true, kNNarrow>(d);
+                if (p.ok) return p;
+            }
+        }
+        if constexpr (sizeof(T) <= 4) {
+            if (d.wide) {
+                const NPlan p = n_plan_cfg<T, BWD, kNWide>(d);
+                if (p.ok) return p;
+            }
         }
     }
     if constexpr (sizeof(T) == 4)
-        if (slim && d.W <= kNSlimWidth)
-            return bwd ? n_plan_cfg<T, true, false, true>(d) : n_plan_cfg<T, false, false, true>(d);
-    return bwd ? n_plan_cfg<T, true>(d) : n_plan_cfg<T, false>(d);
+        if (d.W <= kNSlimWidth) return n_plan_cfg<T, BWD, kNSlim>(d);
+    return n_plan_cfg<T, BWD>(d);
 }
 
 static bool n_scatter_disabled() {
@@ -1538,11 +1559,11 @@ static bool n_use_scatter(const NPlan& p, void* ws, int64_t ws_bytes) {
 
 // NH > 1: w is a head stack (S*B, NH, H, W) mixed by mix (C, NH) in the
 // kernel's weight load.
-template <typename T, bool LOGW, int NH = 1, bool SLIM = false>
+template <typename T, bool LOGW, int NH, int VAR>
 static int n_scatter_fwd_cfg(const void* x, const void* w, const int64_t* sh, NDims d, void* D,
                          void* L, const NPlan& p, void* ws, int* weights_ok, hipStream_t st,
                          const acc_t<T>* mix = nullptr) {
-    using Cfg = NScatterCfg<T, false, false, SLIM>;
+    using Cfg = NScatterCfg<T, false, VAR>;
     using A = acc_t<T>;
     constexpr int V = Cfg::VEC, TPR = Cfg::TPR, RW = Cfg::ROWS;
     char* base = static_cast<char*>(ws);
@@ -1550,7 +1571,8 @@ static int n_scatter_fwd_cfg(const void* x, const void* w, const int64_t* sh, ND
     A* spill = reinterpret_cast<A*>(base + kNHeader);
     A* part = reinterpret_cast<A*>(base + kNHeader + p.spill_bytes);
     const int64_t step = static_cast<int64_t>(d.B) * (NH > 1 ? NH : d.C) * d.H * d.W;
-    hipLaunchKernelGGL((normalized_fwd_scatter_kernel<T, V, TPR, RW, Cfg::D, LOGW, Cfg::WPE, NH>),
+    hipLaunchKernelGGL((normalized_fwd_scatter_kernel<T, V, TPR, RW, Cfg::D, LOGW, Cfg::WPE, NH,
+                                                      Cfg::HALO>),
                        dim3(static_cast<unsigned>(p.tiles)), dim3(TPR * RW), p.lds, st,
                        static_cast<const T*>(x), static_cast<const T*>(w), sh, d.S, d.codes, d.C, d.H, d.W,
                        p.grid, step, static_cast<A*>(D), static_cast<A*>(L), hdr, spill, part,
@@ -1568,17 +1590,22 @@ template <typename T, bool LOGW, int NH = 1>
 static int n_scatter_fwd(const void* x, const void* w, const int64_t* sh, NDims d, void* D,
                          void* L, const NPlan& p, void* ws, int* weights_ok, hipStream_t st,
                          const acc_t<T>* mix = nullptr) {
-    if constexpr (sizeof(T) == 4 && NH == 1)
-        if (p.slim)
-            return n_scatter_fwd_cfg<T, LOGW, 1, true>(x, w, sh, d, D, L, p, ws, weights_ok, st);
-    return n_scatter_fwd_cfg<T, LOGW, NH>(x, w, sh, d, D, L, p, ws, weights_ok, st, mix);
+    if constexpr (sizeof(T) == 4)
+        if (p.var == kNSlim)
+            return n_scatter_fwd_cfg<T, LOGW, NH, kNSlim>(x, w, sh, d, D, L, p, ws, weights_ok,
+                                                          st, mix);
+    if constexpr (sizeof(T) <= 4)
+        if (p.var == kNWide)
+            return n_scatter_fwd_cfg<T, LOGW, NH, kNWide>(x, w, sh, d, D, L, p, ws, weights_ok,
+                                                          st, mix);
+    return n_scatter_fwd_cfg<T, LOGW, NH, kNBase>(x, w, sh, d, D, L, p, ws, weights_ok, st, mix);
 }
 
-template <typename T, bool LOGW, bool NARROW, bool SLIM = false>
+template <typename T, bool LOGW, int VAR>
 static int n_scatter_bwd_cfg(const void* x, const void* w, const void* D, const void* L,
                              const void* gD, const void* gL, const int64_t* sh, NDims d, void* gx,
                              void* gw, const NPlan& p, void* ws, hipStream_t st) {
-    using Cfg = NScatterCfg<T, true, NARROW, SLIM>;
+    using Cfg = NScatterCfg<T, true, VAR>;
     using A = acc_t<T>;
     constexpr int V = Cfg::VEC, TPR = Cfg::TPR, RW = Cfg::ROWS;
     char* base = static_cast<char*>(ws);
@@ -1588,11 +1615,12 @@ static int n_scatter_bwd_cfg(const void* x, const void* w, const void* D, const 
     const int64_t step = static_cast<int64_t>(d.B) * d.C * d.H * d.W;
     // Contiguous 16-byte lanes where the row length and the pointers allow.
     const size_t vb = static_cast<size_t>(V) * sizeof(T);
-    const bool contig = V == 4 && d.W % V == 0 && nsh_host::aligned(x, vb) &&
+    constexpr bool kContig = V == 4 || VAR == kNWide;
+    const bool contig = kContig && d.W % V == 0 && nsh_host::aligned(x, vb) &&
                         nsh_host::aligned(w, vb) && nsh_host::aligned(gw, vb);
     const bool lines = static_cast<int64_t>(d.W) * sizeof(T) % 128 == 0;
     const bool small = step * d.S * static_cast<int64_t>(sizeof(T)) < kNCachedBytes;
-    const bool stream = lines || (contig && (sizeof(T) == 4 || small)) || (V == 2 && small);
+    const bool stream = lines || (contig && (sizeof(T) == 4 || small)) || (!kContig && small);
     auto go = [&](auto contig_tag, auto nts_tag) {
         hipLaunchKernelGGL((normalized_bwd_scatter_kernel<T, V, TPR, RW, Cfg::D, LOGW,
                                                           decltype(contig_tag)::value,
@@ -1605,7 +1633,7 @@ static int n_scatter_bwd_cfg(const void* x, const void* w, const void* D, const 
                            d.C, d.H, d.W, p.grid, step, static_cast<T*>(gx), part,
                            static_cast<T*>(gw), hdr, spill);
     };
-    if constexpr (V == 4) {
+    if constexpr (kContig) {
         if (contig && stream)
             go(std::true_type{}, std::true_type{});
         else if (contig)
@@ -1631,34 +1659,46 @@ template <typename T, bool LOGW>
 static int n_scatter_bwd(const void* x, const void* w, const void* D, const void* L,
                          const void* gD, const void* gL, const int64_t* sh, NDims d, void* gx,
                          void* gw, const NPlan& p, void* ws, hipStream_t st) {
-    if constexpr (sizeof(T) == 8) {
-        if (p.narrow)
-            return n_scatter_bwd_cfg<T, LOGW, true>(x, w, D, L, gD, gL, sh, d, gx, gw, p, ws, st);
-    }
-    if constexpr (sizeof(T) == 4) {
-        if (p.slim)
-            return n_scatter_bwd_cfg<T, LOGW, false, true>(x, w, D, L, gD, gL, sh, d, gx, gw, p,
-                                                           ws, st);
-    }
-    return n_scatter_bwd_cfg<T, LOGW, false>(x, w, D, L, gD, gL, sh, d, gx, gw, p, ws, st);
+    if constexpr (sizeof(T) == 8)
+        if (p.var == kNNarrow)
+            return n_scatter_bwd_cfg<T, LOGW, kNNarrow>(x, w, D, L, gD, gL, sh, d, gx, gw, p, ws,
+                                                        st);
+    if constexpr (sizeof(T) == 4)
+        if (p.var == kNSlim)
+            return n_scatter_bwd_cfg<T, LOGW, kNSlim>(x, w, D, L, gD, gL, sh, d, gx, gw, p, ws, st);
+    if constexpr (sizeof(T) <= 4)
+        if (p.var == kNWide)
+            return n_scatter_bwd_cfg<T, LOGW, kNWide>(x, w, D, L, gD, gL, sh, d, gx, gw, p, ws, st);
+    return n_scatter_bwd_cfg<T, LOGW, kNBase>(x, w, D, L, gD, gL, sh, d, gx, gw, p, ws, st);
 }
 
-// Any of the plans may run (n_run_bwd takes the 8-pixel border when the
-// workspace is too small for the narrow one, the head-mixed forward the wide
-// tiles): the largest.
+// Either plan may run (the base one when the workspace is too small for the
+// hinted one): the larger of the two.
+template <typename T, bool BWD>
+static int64_t n_workspace(const NDims& d) {
+    const NPlan p = n_plan<T, BWD>(d, false);
+    const NPlan q = n_plan<T, BWD>(d);
+    return std::max(p.ok ? p.total : 0, q.ok ? q.total : 0);
+}
 template <typename T>
 static int64_t n_workspace(const NDims& d, bool bwd) {
-    const NPlan p = n_plan<T>(d, bwd, false);
-    const NPlan q = n_plan<T>(d, bwd);
-    const NPlan r = n_plan<T>(d, bwd, false, false);
-    return std::max({p.ok ? p.total : 0, q.ok ? q.total : 0, r.ok ? r.total : 0});
+    return bwd ? n_workspace<T, true>(d) : n_workspace<T, false>(d);
+}
+
+// The plan that a call's workspace allows (p.ok is false if none).
+template <typename T, bool BWD>
+static NPlan n_usable_plan(const NDims& d, void* ws, int64_t ws_bytes) {
+    NPlan p = n_plan<T, BWD>(d);
+    if (!n_use_scatter<T>(p, ws, ws_bytes)) p = n_plan<T, BWD>(d, false);
+    p.ok = n_use_scatter<T>(p, ws, ws_bytes);
+    return p;
 }
 
 template <typename T, bool LOGW>
 static int n_run_fwd(const void* x, const void* w, const int64_t* sh, NDims d, void* D, void* L,
                      void* ws, int64_t ws_bytes, int* weights_ok, hipStream_t st) {
-    const NPlan p = n_plan<T>(d, false);
-    if (n_use_scatter<T>(p, ws, ws_bytes))
+    const NPlan p = n_usable_plan<T, false>(d, ws, ws_bytes);
+    if (p.ok)
         return n_scatter_fwd<T, LOGW>(x, w, sh, d, D, L, p, ws, weights_ok, st);
     switch (n_pick_vec<T>(d.W, {x, w, D, L}, d.S, false)) {
         case 8: if constexpr (sizeof(T) == 2) return n_launch_fwd<T, 8, LOGW>(x, w, sh, d, D, L, weights_ok, st); break;
@@ -1673,9 +1713,8 @@ template <typename T, bool LOGW>
 static int n_run_bwd(const void* x, const void* w, const void* D, const void* L, const void* gD,
                      const void* gL, const int64_t* sh, NDims d, void* gx, void* gw, void* ws,
                      int64_t ws_bytes, hipStream_t st) {
-    NPlan p = n_plan<T>(d, true);
-    if (p.narrow && !n_use_scatter<T>(p, ws, ws_bytes)) p = n_plan<T>(d, true, false);
-    if (n_use_scatter<T>(p, ws, ws_bytes))
+    const NPlan p = n_usable_plan<T, true>(d, ws, ws_bytes);
+    if (p.ok)
         return n_scatter_bwd<T, LOGW>(x, w, D, L, gD, gL, sh, d, gx, gw, p, ws, st);
     switch (n_pick_vec<T>(d.W, {x, w, D, L, gD, gL, gx, gw}, d.S, true)) {
         case 8: if constexpr (sizeof(T) == 2) return n_launch_bwd<T, 8, LOGW>(x, w, D, L, gD, gL, sh, d, gx, gw, st); break;
@@ -1694,6 +1733,7 @@ static int n_check(const char* op, int64_t S, int64_t B, int64_t C, int64_t H, i
                    nsh::NDims* d) {
     const int codes = nsh::dtype_codes(dtype);
     const bool narrow = (dtype & NSH_NARROW_HALO) != 0;
+    const bool wide = (dtype & NSH_WIDE_HALO) != 0 && (dtype & NSH_WIDER_HALO) == 0;
     dtype &= ~NSH_DTYPE_FLAGS;
     if (S < 1 || S > 1024)
         return fail(NSH_ERR_INVALID, "%s: tree reduction requires 1 <= S <= 1024", op);
@@ -1706,7 +1746,7 @@ static int n_check(const char* op, int64_t S, int64_t B, int64_t C, int64_t H, i
         return fail(NSH_ERR_INVALID, "%s: one (b, c) plane must stay below 2^31 bytes", op);
     if (B * C > (int64_t(1) << 24)) return fail(NSH_ERR_INVALID, "%s: B*C too large", op);
     *d = nsh::NDims{static_cast<int>(S), static_cast<int>(B), static_cast<int>(C),
-                    static_cast<int>(H), static_cast<int>(W), codes, narrow};
+                    static_cast<int>(H), static_cast<int>(W), codes, narrow, wide};
     return NSH_OK;
 }
 
@@ -1765,8 +1805,8 @@ static int n_run_fwd_mixed(const void* x, const void* hw, const void* mix, const
                            nsh::NDims d, int heads, void* D, void* L, void* ws, int64_t nws,
                            hipStream_t st) {
     using A = nsh::acc_t<T>;
-    const nsh::NPlan p = nsh::n_plan<T>(d, false, true, false);
-    if (!nsh::n_use_scatter<T>(p, ws, nws))
+    const nsh::NPlan p = nsh::n_usable_plan<T, false>(d, ws, nws);
+    if (!p.ok)
         return fail(NSH_ERR_UNSUPPORTED,
                     "normalized_accumulate_uz_forward_mixed: shape or workspace not served by "
                     "the scatter path");

@@ -523,7 +523,8 @@ class _NormalizedAccumulateUZFn(torch.autograd.Function):
     def forward(ctx, x, weights, shifts, log_weights, rules=0, shared=False, weights_ok=None):
         if shifts.dim() != 2 or shifts.size(1) != 3:
             raise ValueError("normalized_accumulate_uz requires shifts of shape (S, 3)")
-        shifts_i = _prep_shifts_for_cuda(shifts, x.device, radius=x.dtype == torch.float64)
+        shifts_i = _prep_shifts_for_cuda(shifts, x.device, radius=(
+            x.dtype == torch.float64 or shifts.size(0) > _C._HALO8_HALF_ROWS))
         x_c, w_c = x.contiguous(), weights.contiguous()
         D, log_C = _C.normalized_accumulate_uz_forward(x_c, w_c, shifts_i, bool(log_weights),
                                                        rules=rules, shared_weights=shared,
