@@ -30,6 +30,7 @@ reports it when a GPU tensor reaches an op, instead of falling back.
 from __future__ import annotations
 
 import ctypes
+import functools
 import os
 import weakref
 from typing import List, Optional, Sequence
@@ -129,25 +130,41 @@ def _check(ok: bool, msg: str) -> None:
 
 
 def _cuda(t: torch.Tensor, name: str) -> None:
-    _check(t.is_cuda, f"{name} must be a CUDA tensor")
+    if not t.is_cuda:
+        raise RuntimeError(f"{name} must be a CUDA tensor")
 
 
 def _contig(t: torch.Tensor, name: str) -> None:
-    _check(t.is_contiguous(), f"{name} must be contiguous")
+    if not t.is_contiguous():
+        raise RuntimeError(f"{name} must be contiguous")
 
 
 def _nchw(t: torch.Tensor, name: str) -> None:
-    _check(t.dim() == 4, f"{name} must have 4 dims (N,C,H,W)")
+    if t.dim() != 4:
+        raise RuntimeError(f"{name} must have 4 dims (N,C,H,W)")
 
 
 def _prep_shifts(shifts: torch.Tensor, device: torch.device) -> torch.Tensor:
     """(S, 2|3) int64 contiguous table on `device` (shift_ops.cpp:65-75)."""
     _check(shifts.dim() == 2, "shifts must be 2-D (S, 2 or 3)")
     _check(shifts.size(1) in (2, 3), "shifts must have 2 or 3 columns")
+    if (shifts.dtype == torch.int64 and shifts.device == device and shifts.is_contiguous()):
+        return shifts
     return shifts.to(device=device, dtype=torch.int64).contiguous()
 
 
+# The host side of a call is most of a small call's time (a 32 x 32 forward
+# took 17 us here, 24 with the op above it; in the autograd thread, whose
+# caches it shares with nothing, about twice that), so the calls below take the
+# stream as a handle, enter a device only when it is not the current one,
+# format messages only for a check that fails, and keep the workspace sizes of
+# the shapes they have seen.
+_RAW_STREAM = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def _stream(t: torch.Tensor) -> int:
+    if _RAW_STREAM is not None:
+        return _RAW_STREAM(t.get_device())
     return torch.cuda.current_stream(t.device).cuda_stream
 
 
@@ -156,6 +173,25 @@ def _call(name: str, *args) -> None:
     if rc != 0:
         msg = _lib.nsh_last_error().decode(errors="replace")
         raise RuntimeError(msg or f"{name} failed with code {rc}")
+
+
+def _call_on(t: torch.Tensor, name: str, *args) -> None:
+    """The native call `name` on t's device, t's current stream last."""
+    if t.get_device() == torch.cuda.current_device():
+        _call(name, *args, _stream(t))
+    else:
+        with torch.cuda.device(t.device):
+            _call(name, *args, _stream(t))
+
+
+@functools.lru_cache(maxsize=512)
+def _bytes_on(device: int, query: str, *args) -> int:
+    """A workspace size query, by value of its arguments (the library asks the
+    current device for its compute units)."""
+    if device == torch.cuda.current_device():
+        return int(getattr(_lib, query)(*args))
+    with torch.cuda.device(device):
+        return int(getattr(_lib, query)(*args))
 
 
 def _ptr(t) -> int:
@@ -186,9 +222,8 @@ def _gather_forward(op: str, fn: str, guide: torch.Tensor, shifts: torch.Tensor,
     mask = torch.empty((S * B, 1, H, W), dtype=guide.dtype, device=guide.device)
     if out.numel() == 0:
         return [out, mask]
-    with torch.cuda.device(guide.device):
-        _call(fn, guide.data_ptr(), sh.data_ptr(), S, sh.size(1), B, C, H, W, _code(guide, op),
-              out.data_ptr(), mask.data_ptr(), _stream(guide))
+    _call_on(guide, fn, guide.data_ptr(), sh.data_ptr(), S, sh.size(1), B, C, H, W,
+             _code(guide, op), out.data_ptr(), mask.data_ptr())
     return [out, mask]
 
 
@@ -201,9 +236,8 @@ def _gather_backward(op: str, fn: str, grad_out: torch.Tensor, shifts: torch.Ten
     grad = torch.empty((B, C, H, W), dtype=grad_out.dtype, device=grad_out.device)
     if grad.numel() == 0:
         return grad
-    with torch.cuda.device(grad_out.device):
-        _call(fn, grad_out.data_ptr(), sh.data_ptr(), sh.size(0), sh.size(1), B, C, H, W,
-              _code(grad_out, op), grad.data_ptr(), _stream(grad_out))
+    _call_on(grad_out, fn, grad_out.data_ptr(), sh.data_ptr(), sh.size(0), sh.size(1), B, C, H, W,
+             _code(grad_out, op), grad.data_ptr())
     return grad
 
 
@@ -233,6 +267,14 @@ def pair_gather_backward(grad_out: torch.Tensor, shifts: torch.Tensor, B: int, C
 
 def _check_pair(op: str, x: torch.Tensor, weights: torch.Tensor, shifts: torch.Tensor,
                 weight_shape_msg: str, shared: bool = False):
+    if (x.is_cuda and weights.is_cuda and x.is_contiguous() and weights.is_contiguous()
+            and x.dim() == 4 and weights.dim() == 4 and shifts.dim() == 2
+            and shifts.size(1) == 3 and weights.device == x.device and weights.dtype == x.dtype):
+        B, C, H, W = x.shape
+        S = shifts.size(0)
+        if 0 < S <= 1024 and weights.shape == (S * B, 1 if shared else C, H, W):
+            return _prep_shifts(shifts, x.device), B, C, H, W, S
+    # a check fails: the same ones, each with its message
     _cuda(x, "x")
     _contig(x, "x")
     _nchw(x, "x")
@@ -358,30 +400,31 @@ def accumulate_uz_forward(x: torch.Tensor, weights: torch.Tensor,
     U = torch.empty(x.shape, dtype=acc, device=x.device)
     Z = torch.empty(x.shape, dtype=acc, device=x.device)
     ws, nws = _workspace(S, B, C, H, W, code, False, x.device)
-    with torch.cuda.device(x.device):
-        if band is None:
-            _call("nsh_accumulate_uz_forward", x.data_ptr(), weights.data_ptr(), sh.data_ptr(),
-                  S, B, C, H, W, code, U.data_ptr(), Z.data_ptr(), _ptr(ws), nws, _stream(x))
-        else:
-            org, hg = _band_args(band)
-            _call("nsh_accumulate_uz_forward_band", x.data_ptr(), weights.data_ptr(),
-                  sh.data_ptr(), S, B, C, H, W, org, hg, code, U.data_ptr(), Z.data_ptr(),
-                  _ptr(ws), nws, _stream(x))
+    if band is None:
+        _call_on(x, "nsh_accumulate_uz_forward", x.data_ptr(), weights.data_ptr(), sh.data_ptr(),
+                 S, B, C, H, W, code, U.data_ptr(), Z.data_ptr(), _ptr(ws), nws)
+    else:
+        org, hg = _band_args(band)
+        _call_on(x, "nsh_accumulate_uz_forward_band", x.data_ptr(), weights.data_ptr(),
+                 sh.data_ptr(), S, B, C, H, W, org, hg, code, U.data_ptr(), Z.data_ptr(),
+                 _ptr(ws), nws)
     return [U, Z]
 
 
 def _workspace(S, B, C, H, W, code, backward, device):
     """Scratch buffer of accumulate_uz (spilled window borders of the
     once-per-element weight stream); (None, 0) when the shape needs none."""
-    n = int(_lib.nsh_accumulate_uz_workspace_bytes(S, B, C, H, W, code, int(backward)))
+    n = _bytes_on(device.index, "nsh_accumulate_uz_workspace_bytes", S, B, C, H, W, code,
+                  int(backward))
     if n <= 0:
         return None, 0
     return torch.empty(n, dtype=torch.uint8, device=device), n
 
 
 def _grad_in(g: torch.Tensor, like: torch.Tensor, acc: torch.dtype, name: str) -> torch.Tensor:
-    _cuda(g, name)
-    _check(tuple(g.shape) == tuple(like.shape), f"{name} must match the shape of x")
+    if not (g.is_cuda and g.shape == like.shape):
+        _cuda(g, name)
+        _check(False, f"{name} must match the shape of x")
     return g.to(acc).contiguous()
 
 
@@ -402,16 +445,15 @@ def accumulate_uz_backward(x: torch.Tensor, weights: torch.Tensor, grad_U: torch
     gx = torch.empty_like(x)
     gw = torch.empty((S * B, C, H, W), dtype=weights.dtype, device=weights.device)
     ws, nws = _workspace(S, B, C, H, W, code, True, x.device)
-    with torch.cuda.device(x.device):
-        if band is None:
-            _call("nsh_accumulate_uz_backward", x.data_ptr(), weights.data_ptr(), gU.data_ptr(),
-                  gZ.data_ptr(), sh.data_ptr(), S, B, C, H, W, code, gx.data_ptr(),
-                  gw.data_ptr(), _ptr(ws), nws, _stream(x))
-        else:
-            org, hg = _band_args(band)
-            _call("nsh_accumulate_uz_backward_band", x.data_ptr(), weights.data_ptr(),
-                  gU.data_ptr(), gZ.data_ptr(), sh.data_ptr(), S, B, C, H, W, org, hg, code,
-                  gx.data_ptr(), gw.data_ptr(), _ptr(ws), nws, _stream(x))
+    if band is None:
+        _call_on(x, "nsh_accumulate_uz_backward", x.data_ptr(), weights.data_ptr(),
+                 gU.data_ptr(), gZ.data_ptr(), sh.data_ptr(), S, B, C, H, W, code, gx.data_ptr(),
+                 gw.data_ptr(), _ptr(ws), nws)
+    else:
+        org, hg = _band_args(band)
+        _call_on(x, "nsh_accumulate_uz_backward_band", x.data_ptr(), weights.data_ptr(),
+                 gU.data_ptr(), gZ.data_ptr(), sh.data_ptr(), S, B, C, H, W, org, hg, code,
+                 gx.data_ptr(), gw.data_ptr(), _ptr(ws), nws)
     return [gx, gw]
 
 
@@ -437,10 +479,9 @@ def normalized_accumulate_uz_forward(x: torch.Tensor, weights: torch.Tensor, shi
     D = torch.empty(x.shape, dtype=acc, device=x.device)
     L = torch.empty(x.shape, dtype=acc, device=x.device)
     ws, nws = _norm_workspace(S, B, C, H, W, code, False, x.device)
-    with torch.cuda.device(x.device):
-        _call("nsh_normalized_accumulate_uz_forward_checked", x.data_ptr(), weights.data_ptr(),
-              sh.data_ptr(), S, B, C, H, W, code, int(bool(log_weights)), D.data_ptr(),
-              L.data_ptr(), _ptr(weights_ok), _ptr(ws), nws, _stream(x))
+    _call_on(x, "nsh_normalized_accumulate_uz_forward_checked", x.data_ptr(), weights.data_ptr(),
+             sh.data_ptr(), S, B, C, H, W, code, int(bool(log_weights)), D.data_ptr(),
+             L.data_ptr(), _ptr(weights_ok), _ptr(ws), nws)
     return [D, L]
 
 
@@ -536,9 +577,8 @@ def head_mix_backward(w: torch.Tensor, mix: torch.Tensor, grad_out: torch.Tensor
     n = int(_lib.nsh_head_mix_workspace_bytes(N, h, C, P, code))
     _check(n > 0, f"{op}: {_lib.nsh_last_error().decode(errors='replace')}")
     ws = torch.empty(n, dtype=torch.uint8, device=w.device)
-    with torch.cuda.device(w.device):
-        _call("nsh_head_mix_backward", w.data_ptr(), m.data_ptr(), g.data_ptr(), N, h, C, P,
-              code, gw.data_ptr(), gm.data_ptr(), ws.data_ptr(), n, _stream(w))
+    _call_on(w, "nsh_head_mix_backward", w.data_ptr(), m.data_ptr(), g.data_ptr(), N, h, C, P,
+             code, gw.data_ptr(), gm.data_ptr(), ws.data_ptr(), n)
     return [gw, gm]
 
 
@@ -546,7 +586,8 @@ def _norm_workspace(S, B, C, H, W, code, backward, device):
     """Scratch buffer of normalized_accumulate_uz (spilled window borders and
     the partial states of tile-edge pixels); (None, 0) when the shape needs
     none."""
-    n = int(_lib.nsh_normalized_workspace_bytes(S, B, C, H, W, code, int(backward)))
+    n = _bytes_on(device.index, "nsh_normalized_workspace_bytes", S, B, C, H, W, code,
+                  int(backward))
     if n <= 0:
         return None, 0
     return torch.empty(n, dtype=torch.uint8, device=device), n
@@ -575,15 +616,21 @@ def normalized_accumulate_uz_backward(x: torch.Tensor, weights: torch.Tensor, D:
     if x.dtype == torch.float64:
         code |= _narrow_halo_flag(sh)
     ws, nws = _norm_workspace(S, B, C, H, W, code, True, x.device)
-    with torch.cuda.device(x.device):
-        _call("nsh_normalized_accumulate_uz_backward", x.data_ptr(), weights.data_ptr(),
-              Dc.data_ptr(), Lc.data_ptr(), gD.data_ptr(), gL.data_ptr(), sh.data_ptr(), S, B, C,
-              H, W, code, int(bool(log_weights)), gx.data_ptr(), gw.data_ptr(), _ptr(ws), nws,
-              _stream(x))
+    _call_on(x, "nsh_normalized_accumulate_uz_backward", x.data_ptr(), weights.data_ptr(),
+             Dc.data_ptr(), Lc.data_ptr(), gD.data_ptr(), gL.data_ptr(), sh.data_ptr(), S, B, C,
+             H, W, code, int(bool(log_weights)), gx.data_ptr(), gw.data_ptr(), _ptr(ws), nws)
     return [gx, gw]
 
 
 def _check_scalar(x: torch.Tensor, weights: torch.Tensor, shifts: torch.Tensor):
+    if (x.is_cuda and weights.is_cuda and x.is_contiguous() and weights.is_contiguous()
+            and x.dim() == 4 and shifts.dim() == 2 and shifts.size(1) in (2, 3)
+            and weights.device == x.device and weights.dtype == x.dtype):
+        B, C, H, W = x.shape
+        S = shifts.size(0)
+        if 0 < S <= 1024 and weights.shape == (S, B, C):
+            return _prep_shifts(shifts, x.device), B, C, H, W, S
+    # a check fails: the same ones, each with its message
     _cuda(x, "x")
     _contig(x, "x")
     _nchw(x, "x")
@@ -609,10 +656,9 @@ def accumulate_uz_scalar_forward(x: torch.Tensor, weights: torch.Tensor,
     acc = _acc_dtype(x.dtype)
     U = torch.empty(x.shape, dtype=acc, device=x.device)
     Z = torch.empty(x.shape, dtype=acc, device=x.device)
-    with torch.cuda.device(x.device):
-        _call("nsh_accumulate_uz_scalar_forward", x.data_ptr(), weights.data_ptr(),
-              sh.data_ptr(), S, sh.size(1), B, C, H, W, _code(x, "accumulate_uz_scalar_fwd"),
-              U.data_ptr(), Z.data_ptr(), _stream(x))
+    _call_on(x, "nsh_accumulate_uz_scalar_forward", x.data_ptr(), weights.data_ptr(),
+             sh.data_ptr(), S, sh.size(1), B, C, H, W, _code(x, "accumulate_uz_scalar_fwd"),
+             U.data_ptr(), Z.data_ptr())
     return [U, Z]
 
 
@@ -627,11 +673,10 @@ def accumulate_uz_scalar_backward(x: torch.Tensor, weights: torch.Tensor, grad_U
     gw = torch.empty_like(weights)
     nsplit = int(_lib.nsh_scalar_backward_splits(H, W))
     part = torch.empty(S * B * C * nsplit, dtype=acc, device=x.device)
-    with torch.cuda.device(x.device):
-        _call("nsh_accumulate_uz_scalar_backward", x.data_ptr(), weights.data_ptr(),
-              gU.data_ptr(), gZ.data_ptr(), sh.data_ptr(), S, sh.size(1), B, C, H, W,
-              _code(x, "accumulate_uz_scalar_bwd"), gx.data_ptr(), gw.data_ptr(),
-              part.data_ptr(), _stream(x))
+    _call_on(x, "nsh_accumulate_uz_scalar_backward", x.data_ptr(), weights.data_ptr(),
+             gU.data_ptr(), gZ.data_ptr(), sh.data_ptr(), S, sh.size(1), B, C, H, W,
+             _code(x, "accumulate_uz_scalar_bwd"), gx.data_ptr(), gw.data_ptr(),
+             part.data_ptr())
     return [gx, gw]
 
 
@@ -672,11 +717,10 @@ def metropolis_aggregate_backward(w_half: torch.Tensor, img: torch.Tensor, shift
     ws = torch.empty(n, dtype=torch.uint8, device=img.device)
     gw = torch.empty_like(w_half)
     gx = torch.empty_like(img)
-    with torch.cuda.device(img.device):
-        _call("nsh_metropolis_aggregate_backward", w_half.data_ptr(), img.data_ptr(),
-              sh.data_ptr(), B, S, C, H, W, code | flag, int(bool(use_box)), float(eps),
-              degree.data_ptr(), d_hat.contiguous().data_ptr(), gWx.data_ptr(), gdh.data_ptr(),
-              gw.data_ptr(), gx.data_ptr(), ws.data_ptr(), n, _stream(img))
+    _call_on(img, "nsh_metropolis_aggregate_backward", w_half.data_ptr(), img.data_ptr(),
+             sh.data_ptr(), B, S, C, H, W, code | flag, int(bool(use_box)), float(eps),
+             degree.data_ptr(), d_hat.contiguous().data_ptr(), gWx.data_ptr(), gdh.data_ptr(),
+             gw.data_ptr(), gx.data_ptr(), ws.data_ptr(), n)
     return [gw, gx]
 
 
@@ -704,10 +748,9 @@ def metropolis_aggregate_with_degree(w_half: torch.Tensor, img: torch.Tensor,
     code = _code(img, "metropolis_aggregate_cuda")
     n = int(_lib.nsh_metropolis_workspace_bytes(B, S, C, H, W, code))
     ws = torch.empty(n, dtype=torch.uint8, device=img.device) if n > 0 else None
-    with torch.cuda.device(img.device):
-        _call("nsh_metropolis_aggregate", w_half.data_ptr(), img.data_ptr(), sh.data_ptr(), B, S,
-              C, H, W, code, int(bool(use_box)), float(eps), Wx.data_ptr(), d_hat.data_ptr(),
-              degree.data_ptr(), _ptr(ws), max(n, 0), _stream(img))
+    _call_on(img, "nsh_metropolis_aggregate", w_half.data_ptr(), img.data_ptr(), sh.data_ptr(), B,
+             S, C, H, W, code, int(bool(use_box)), float(eps), Wx.data_ptr(), d_hat.data_ptr(),
+             degree.data_ptr(), _ptr(ws), max(n, 0))
     return [Wx, d_hat, degree]
 
 

@@ -97,6 +97,8 @@ def _prep_shifts_for_cuda(shifts: torch.Tensor, device: torch.device,
     (reference ops.py:397-404)."""
     if shifts.dim() != 2 or shifts.size(1) not in (2, 3):
         raise ValueError(f"shifts must be (S, 2) or (S, 3); got {tuple(shifts.shape)}")
+    if (shifts.dtype == torch.int64 and shifts.device == device and shifts.is_contiguous()):
+        return shifts
     out = shifts.to(device=device, dtype=torch.int64).contiguous()
     if out is not shifts and _HAS_CUDA_EXT and (radius or not shifts.is_cuda):
         # the kernels' launch shape depends on the table's radius: record it
@@ -408,13 +410,16 @@ class _ShiftGatherFn(torch.autograd.Function):
         out, mask = _C.shift_gather_forward(guide.contiguous(), shifts_i)
         ctx.save_for_backward(shifts_i)
         ctx.guide_shape = tuple(guide.shape)
+        # the mask is no function of the guide: its gradient is not used, and
+        # not made up as zeros where the caller has none
+        ctx.set_materialize_grads(False)
         return out, mask
 
     @staticmethod
     def backward(ctx, grad_out, grad_mask):
         (shifts_i,) = ctx.saved_tensors
-        if grad_out is None:
-            return None, None
+        if grad_out is None:  # zeros where only the mask has a gradient
+            return (None if grad_mask is None else grad_mask.new_zeros(ctx.guide_shape)), None
         B, C, H, W = ctx.guide_shape
         return _C.shift_gather_backward(grad_out.contiguous(), shifts_i, B, C, H, W), None
 
@@ -426,13 +431,16 @@ class _PairGatherFn(torch.autograd.Function):
         out, mask = _C.pair_gather_forward(guide.contiguous(), shifts_i)
         ctx.save_for_backward(shifts_i)
         ctx.guide_shape = tuple(guide.shape)
+        # the mask is no function of the guide: its gradient is not used, and
+        # not made up as zeros where the caller has none
+        ctx.set_materialize_grads(False)
         return out, mask
 
     @staticmethod
     def backward(ctx, grad_out, grad_mask):
         (shifts_i,) = ctx.saved_tensors
-        if grad_out is None:
-            return None, None
+        if grad_out is None:  # zeros where only the mask has a gradient
+            return (None if grad_mask is None else grad_mask.new_zeros(ctx.guide_shape)), None
         B, C, H, W = ctx.guide_shape
         return _C.pair_gather_backward(grad_out.contiguous(), shifts_i, B, C, H, W), None
 
@@ -441,7 +449,7 @@ def _shared_grad(grad_w: torch.Tensor, shared: bool) -> torch.Tensor:
     """The kernels return the weight gradient per channel; shared weights
     (S*B, 1, H, W) receive its sum over the channels (in the accumulator
     type, rounded once)."""
-    if not shared:
+    if not shared or grad_w.size(1) == 1:
         return grad_w
     acc = torch.float64 if grad_w.dtype == torch.float64 else torch.float32
     return grad_w.sum(dim=1, keepdim=True, dtype=acc).to(grad_w.dtype)
