@@ -97,6 +97,103 @@ __global__ __launch_bounds__(kThreads) void gather_fwd_kernel(
     }
 }
 
+// Fills the vectors of one lane's chunk of a plane of HW elements at p with
+// value(h, w): aligned 16-byte vectors from the plane's first aligned element
+// on, wherever its rows begin, and single elements before the first and after
+// the last vector.
+template <typename E, int VEC, typename F>
+__device__ __forceinline__ void fill_flat(E* __restrict__ p, int64_t chunk, uint32_t HW, uint32_t W,
+                                          F&& next) {
+    const uint32_t a = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(p) / sizeof(E)) % VEC;
+    const uint32_t lead = min((VEC - a) % VEC, HW);
+    const uint32_t nv = (HW - lead) / VEC;
+    const uint32_t v0 = static_cast<uint32_t>(chunk) * (kThreads * kGIter) + threadIdx.x;
+#pragma unroll
+    for (int n = 0; n < kGIter; ++n) {
+        const uint32_t v = v0 + n * kThreads;
+        if (v >= nv) break;
+        const uint32_t o = lead + v * VEC;
+        uint32_t h = o / W, w = o - h * W;
+        Pack<E, VEC> t;
+        next(h, w, t.e);
+        store_pack_nt<E, VEC>(p + o, t);
+    }
+    if (chunk == 0) {  // fewer than VEC elements before the vectors, and after
+        const uint32_t tail = lead + nv * VEC;
+        const uint32_t o = threadIdx.x < lead ? threadIdx.x : tail + (threadIdx.x - lead);
+        if (o < HW && threadIdx.x < lead + (HW - tail)) {
+            const uint32_t h = o / W, w = o - h * W;
+            E t[1];
+            next(h, w, t);
+            p[o] = t[0];
+        }
+    }
+}
+
+// 16-bit planes whose rows take no vector (odd W): written as a flat run of
+// 16-byte vectors instead of element by element, kThreads * kGIter vectors per
+// workgroup (R = 5, bf16: 4 x 3 x 321 x 481 203 -> 116 us, pairs 355 -> 214;
+// 2 x 1 x 977^2 211 -> 123).  Where rows take vectors of 4 or 8 elements the
+// row-wise forms need less work per element (320 x 484: 66 us, flat 108), and
+// fp32 stores one by one are no slower (977^2 240, flat 249).
+template <int ES, bool PAIR>
+__global__ __launch_bounds__(kThreads) void gather_fwd_flat_kernel(
+    const typename Bits<ES>::type* __restrict__ guide, const int64_t* __restrict__ shifts,
+    int cols, int B, int C, int H, int W, int64_t chunks, typename Bits<ES>::type* __restrict__ out,
+    typename Bits<ES>::type* __restrict__ mask, typename Bits<ES>::type one) {
+    using E = typename Bits<ES>::type;
+    constexpr int VEC = 16 / ES;
+    const int Cout = PAIR ? 2 * C : C;
+    const int64_t plane = blockIdx.x / chunks;  // output plane (s*B+b)*Cout + co
+    const int64_t chunk = blockIdx.x - plane * chunks;
+    const int64_t sb = plane / Cout;
+    const int co = static_cast<int>(plane - sb * Cout);
+    const int64_t s = sb / B;
+    const int64_t b = sb - s * B;
+    const bool centre = PAIR && co < C;
+    const int c = PAIR ? (co < C ? co : co - C) : co;
+
+    const int64_t dx64 = shifts[s * cols + 0];
+    const int64_t dy64 = shifts[s * cols + 1];
+    const uint32_t sx = centre ? 0 : static_cast<uint32_t>(mod_pos(dx64, H));
+    const uint32_t sy = centre ? 0 : static_cast<uint32_t>(mod_pos(dy64, W));
+    const int64_t HW = static_cast<int64_t>(H) * W;
+    const E* __restrict__ g = guide + (b * C + c) * HW;
+    const uint32_t uH = H, uW = W;
+    fill_flat<E, VEC>(out + plane * HW, chunk, static_cast<uint32_t>(HW), uW,
+                      [&](uint32_t h, uint32_t w, auto& e) {
+        uint32_t hh = h + sx, ww = w + sy;
+        hh -= hh >= uH ? uH : 0;
+        ww -= ww >= uW ? uW : 0;
+        uint32_t row = hh * uW;
+#pragma unroll
+        for (uint32_t k = 0; k < sizeof(e) / sizeof(E); ++k) {
+            e[k] = g[row + ww];
+            ww = ww + 1 == uW ? 0 : ww + 1;
+            if (++w == uW) {  // the next row of the output
+                w = 0;
+                hh = hh + 1 == uH ? 0 : hh + 1;
+                row = hh * uW;
+                ww = sy;
+            }
+        }
+    });
+    if (mask == nullptr || co != 0) return;
+    const int dxc = clamp_shift(dx64), dyc = clamp_shift(dy64);
+    fill_flat<E, VEC>(mask + sb * HW, chunk, static_cast<uint32_t>(HW), uW,
+                      [&](uint32_t h, uint32_t w, auto& e) {
+        int hi = static_cast<int>(h), wi = static_cast<int>(w);
+#pragma unroll
+        for (uint32_t k = 0; k < sizeof(e) / sizeof(E); ++k) {
+            e[k] = (in_range(hi + dxc, H) && in_range(wi + dyc, W)) ? one : E(0);
+            if (++wi == W) {
+                wi = 0;
+                ++hi;
+            }
+        }
+    });
+}
+
 template <typename T, int VEC, bool PAIR>
 __global__ __launch_bounds__(kThreads) void gather_bwd_kernel(
     const T* __restrict__ gout, const int64_t* __restrict__ shifts, int cols, int S, int B, int C,
@@ -488,6 +585,22 @@ static int g_fwd_launch(const void* guide, const int64_t* sh, int cols, int S, i
     return nsh_host::check_launch(PAIR ? "pair_gather_forward" : "shift_gather_forward");
 }
 
+template <int ES, bool PAIR>
+static int g_fwd_flat(const void* guide, const int64_t* sh, int cols, int S, int B, int C, int H,
+                      int W, void* out, void* mask, uint64_t one_bits, hipStream_t st) {
+    using E = typename Bits<ES>::type;
+    const int64_t nvec = static_cast<int64_t>(H) * W / (16 / ES) + 1;
+    const int64_t chunks = nsh_host::ceil_div(nvec, static_cast<int64_t>(kThreads) * kGIter);
+    const int64_t planes = static_cast<int64_t>(S) * B * (PAIR ? 2 * C : C);
+    const int64_t blocks = planes * chunks;
+    if (blocks > 0x7fffffff) return nsh_host::fail(NSH_ERR_INVALID, "gather: grid too large");
+    hipLaunchKernelGGL((gather_fwd_flat_kernel<ES, PAIR>), dim3(static_cast<unsigned>(blocks)),
+                       dim3(kThreads), 0, st, static_cast<const E*>(guide), sh, cols, B, C, H, W,
+                       chunks, static_cast<E*>(out), static_cast<E*>(mask),
+                       static_cast<E>(one_bits));
+    return nsh_host::check_launch(PAIR ? "pair_gather_forward" : "shift_gather_forward");
+}
+
 // Tiled path: 16-byte vectors, W a multiple of the vector width, aligned
 // pointers, S <= 1024 (the shift table lives in LDS).
 static bool g_tile_ok(int S, int W, int vec, std::initializer_list<const void*> ptrs) {
@@ -547,7 +660,10 @@ static int g_fwd(const void* guide, const int64_t* sh, int cols, int S, int B, i
         case 2: return g_fwd_launch<ES, 2, PAIR>(guide, sh, cols, S, B, C, H, W, out, mask, one_bits, st);
         default: break;
     }
-    return g_fwd_launch<ES, 1, PAIR>(guide, sh, cols, S, B, C, H, W, out, mask, one_bits, st);
+    if constexpr (ES == 2)
+        return g_fwd_flat<ES, PAIR>(guide, sh, cols, S, B, C, H, W, out, mask, one_bits, st);
+    else
+        return g_fwd_launch<ES, 1, PAIR>(guide, sh, cols, S, B, C, H, W, out, mask, one_bits, st);
 }
 
 template <typename T, int VEC, bool PAIR>
