@@ -297,6 +297,23 @@ NSH_API int nsh_normalized_accumulate_uz_backward(const void* x, const void* wei
                                           void* grad_x, void* grad_w, void* workspace,
                                           int64_t workspace_bytes, void* stream);
 
+/* The backward of channel-shared weights with their own gradient: weights and
+ * grad_w are (S*B, 1, H, W), grad_w the sum over the C channels (accumulator
+ * type, rounded once).  log_C is that of the forward on the same weights, the
+ * same in every channel (channel 0 is read).  dtype takes the row rules and
+ * codes; shared weights are understood.  Served: C 2 or 3, fp16/bf16/fp32,
+ * images of at least 32 a side, with a workspace of
+ * nsh_normalized_shared_workspace_bytes (0: not served, -1: invalid
+ * arguments); otherwise NSH_ERR_UNSUPPORTED, nothing launched.  No counterpart
+ * in the reference. */
+NSH_API int64_t nsh_normalized_shared_workspace_bytes(int64_t S, int64_t B, int64_t C, int64_t H,
+                                                      int64_t W, int dtype);
+NSH_API int nsh_normalized_accumulate_uz_backward_shared(
+    const void* x, const void* weights, const void* D, const void* log_C, const void* grad_D,
+    const void* grad_log_C, const int64_t* shifts, int64_t S, int64_t B, int64_t C, int64_t H,
+    int64_t W, int dtype, int log_weights, void* grad_x, void* grad_w, void* workspace,
+    int64_t workspace_bytes, void* stream);
+
 /* Workspace of normalized_accumulate_uz forward (backward = 0) or backward
  * (1), in bytes; 0 when the shape does not use one, -1 on invalid arguments.
  * No counterpart in the reference (whose kernels re-read shifted weights).

@@ -83,6 +83,10 @@ _SIGS = {
                               _I),
     "nsh_normalized_accumulate_uz_backward": ([_P, _P, _P, _P, _P, _P, _P, _I64, _I64, _I64,
                                                _I64, _I64, _I, _I, _P, _P, _P, _I64, _P], _I),
+    "nsh_normalized_accumulate_uz_backward_shared": ([_P, _P, _P, _P, _P, _P, _P, _I64, _I64,
+                                                      _I64, _I64, _I64, _I, _I, _P, _P, _P, _I64,
+                                                      _P], _I),
+    "nsh_normalized_shared_workspace_bytes": ([_I64, _I64, _I64, _I64, _I64, _I], _I64),
     "nsh_normalized_workspace_bytes": ([_I64, _I64, _I64, _I64, _I64, _I, _I], _I64),
     "nsh_scalar_backward_splits": ([_I64, _I64], _I),
     "nsh_accumulate_uz_scalar_forward": ([_P, _P, _P, _I64, _I64, _I64, _I64, _I64, _I64, _I, _P,
@@ -172,7 +176,12 @@ def _call(name: str, *args) -> None:
     rc = getattr(_lib, name)(*args)
     if rc != 0:
         msg = _lib.nsh_last_error().decode(errors="replace")
-        raise RuntimeError(msg or f"{name} failed with code {rc}")
+        raise (_Unsupported if rc == NSH_ERR_UNSUPPORTED else RuntimeError)(
+            msg or f"{name} failed with code {rc}")
+
+
+class _Unsupported(RuntimeError):
+    """An entry point does not serve a valid call (nothing was launched)."""
 
 
 def _call_on(t: torch.Tensor, name: str, *args) -> None:
@@ -619,6 +628,36 @@ def normalized_accumulate_uz_backward(x: torch.Tensor, weights: torch.Tensor, D:
     _call_on(x, "nsh_normalized_accumulate_uz_backward", x.data_ptr(), weights.data_ptr(),
              Dc.data_ptr(), Lc.data_ptr(), gD.data_ptr(), gL.data_ptr(), sh.data_ptr(), S, B, C,
              H, W, code, int(bool(log_weights)), gx.data_ptr(), gw.data_ptr(), _ptr(ws), nws)
+    return [gx, gw]
+
+
+def normalized_accumulate_uz_backward_shared(
+        x: torch.Tensor, weights: torch.Tensor, D: torch.Tensor, log_C: torch.Tensor,
+        grad_D: torch.Tensor, grad_log_C: torch.Tensor, shifts: torch.Tensor, log_weights: bool, *,
+        rules: int = 0) -> Optional[List[torch.Tensor]]:
+    """[grad_x, grad_w] for shared weights (S*B, 1, H, W), grad_w their own
+    gradient (the sum over the channels), in one pass
+    (nsh_normalized_accumulate_uz_backward_shared); None for a shape or type
+    it does not serve."""
+    sh, B, C, H, W, S = _check_pair("normalized_accumulate_uz", x, weights, shifts,
+                                    "normalized_accumulate_uz: weights must be (S*B, C, H, W)",
+                                    True)
+    code = _code(x, "normalized_accumulate_uz_bwd") | _flags(False, True, rules)
+    n = _bytes_on(x.device.index, "nsh_normalized_shared_workspace_bytes", S, B, C, H, W, code)
+    if n <= 0:
+        return None
+    acc = _acc_dtype(x.dtype)
+    Dc, Lc = _grad_in(D, x, acc, "D"), _grad_in(log_C, x, acc, "log_C")
+    gD, gL = _grad_in(grad_D, x, acc, "grad_D"), _grad_in(grad_log_C, x, acc, "grad_log_C")
+    gx, gw = torch.empty_like(x), torch.empty_like(weights)
+    ws = torch.empty(n, dtype=torch.uint8, device=x.device)
+    try:
+        _call_on(x, "nsh_normalized_accumulate_uz_backward_shared", x.data_ptr(),
+                 weights.data_ptr(), Dc.data_ptr(), Lc.data_ptr(), gD.data_ptr(), gL.data_ptr(),
+                 sh.data_ptr(), S, B, C, H, W, code, int(bool(log_weights)), gx.data_ptr(),
+                 gw.data_ptr(), ws.data_ptr(), n)
+    except _Unsupported:
+        return None
     return [gx, gw]
 
 

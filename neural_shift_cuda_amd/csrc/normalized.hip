@@ -1338,6 +1338,243 @@ normalized_bwd_scatter_kernel(const T* __restrict__ x, const T* __restrict__ w,
     }
 }
 
+// Backward of channel-shared weights, the weights' own gradient (the sum over
+// the channels) formed here.  The per-channel kernel above runs one workgroup
+// per channel: each reads the weights and forms the fractions f(w, L) again
+// (the degree of shared weights is the same for every channel, so L is read
+// from channel 0), writes a gradient plane of its own, and the C planes per
+// shift are read back and summed.  Here a workgroup takes the NC channels of
+// its tile: one key array, and x, alpha, beta and the gx window per channel,
+// 4 NC + 1 LDS arrays, on 64 x 16 tiles of 1024 lanes, one pixel each (133 KB
+// at NC = 3; four channels would not fit).  Per channel with the sum, and
+// here: 8 x 3 x 250^2 R = 5 fp32 330 and 112 us (3.1 TB/s of weights and their
+// gradient), fp16 207 and 104; 1024^2 C = 3 R = 6 fp32 690 and 283; 2 channels
+// of 321 x 481 R = 6 256 and 113.  Rows beyond the border take the gather form
+// here too, and that is still the faster side of the two for tables that the
+// per-channel kernels serve on the 16-pixel border (R = 10, 221 rows, fp32:
+// 1230 and 494 us; 69 rows of radius 16, 832 and 215).  Bound by the loop's
+// LDS accesses (13 reads and 3 writes per pixel and row) at 16 waves per CU:
+// fp16 takes 0.93 of fp32's time.
+// beta stays per channel, so that each score is formed as above: with the
+// channels' beta summed at the load the scores' error against 64 bits grew by
+// 4% (x of mean 5, C = 3) to 22% (maximum, C = 4).
+constexpr int kNShRows = 16, kNShTpr = 64, kNShDepth = 4;
+
+template <typename T, int NC, bool LOGW>
+__global__ __launch_bounds__(kNShTpr * kNShRows, 4) void normalized_bwd_shared_kernel(
+    const T* __restrict__ x, const T* __restrict__ w, const acc_t<T>* __restrict__ Dg,
+    const acc_t<T>* __restrict__ Lg, const acc_t<T>* __restrict__ gDg,
+    const acc_t<T>* __restrict__ gLg, const int64_t* __restrict__ shifts, int S, int codes, int H,
+    int W, TileGrid tg, int64_t wstep, T* __restrict__ gx, acc_t<T>* __restrict__ gxp,
+    T* __restrict__ gw, int* __restrict__ hdr, acc_t<T>* __restrict__ spill) {
+    using A = acc_t<T>;
+    using G = SGeo<1, kNShRows, kNShTpr>;
+    constexpr int D = kNShDepth, HALO = kRmax;
+    extern __shared__ __align__(16) unsigned char smem[];
+    int4* shl = reinterpret_cast<int4*>(smem);
+    A* lt = reinterpret_cast<A*>(smem + shift_lds_bytes(S));  // L key or E
+    A* xt = lt + G::TILE;                                      // NC tiles each
+    A* at = xt + NC * G::TILE;
+    A* bt = at + NC * G::TILE;
+    A* mg = bt + NC * G::TILE;
+
+    const int64_t t = xcd_tile(blockIdx.x, gridDim.x);
+    const TileIdx ti = tile_of(t, tg, G::TH, G::TW, H, W);  // ti.bc: the batch entry
+    const int64_t HW = static_cast<int64_t>(H) * W;
+    const int64_t off = ti.bc * NC * HW;  // channel 0 of this batch entry
+    stage_shifts(shl, shifts, S, 3, H, W, codes);
+    {
+        const bool cheap = H >= G::LH && W >= G::LW;
+        for (int i = threadIdx.x; i < G::LH * G::LW; i += blockDim.x) {
+            const int64_t g = off + halo_offset(i, G::LW, ti.h0, ti.w0, H, W, cheap);
+            const int r = i / G::LW;
+            const int li = r * G::PITCH + (i - r * G::LW);
+            A d[NC], gd[NC], gl[NC];
+            T xv[NC];
+            const A L = Lg[g];
+#pragma unroll
+            for (int c = 0; c < NC; ++c) {
+                xv[c] = x[g + c * HW];
+                gd[c] = gDg[g + c * HW];
+                gl[c] = gLg[g + c * HW];
+                d[c] = Dg[g + c * HW];
+            }
+#pragma unroll
+            for (int c = 0; c < NC; ++c) {
+                xt[c * G::TILE + li] = to_acc(xv[c]);
+                at[c * G::TILE + li] = gd[c];
+                bt[c * G::TILE + li] = gl[c] - gd[c] * d[c];
+            }
+            lt[li] = LOGW ? log_key<A>(L) : Lim<A>::ex(-L);
+        }
+    }
+    const int R = near_radius(shl, S, false);
+    if (blockIdx.x == 0 && threadIdx.x == 0) hdr[0] = R;  // for the fix-up
+    lds_zero(mg, NC * G::TILE);
+    __syncthreads();
+
+    const int tx = threadIdx.x % kNShTpr;
+    const int ty = threadIdx.x / kNShTpr;
+    const int h = ti.h0 + ty, wq = ti.w0 + tx;
+    const bool act = ty < ti.th && tx < ti.tw;
+    const uint32_t own = act ? static_cast<uint32_t>(h) * static_cast<uint32_t>(W) + wq : 0u;
+    const uint32_t own_b = own * static_cast<uint32_t>(sizeof(T));
+    const int li = (ty + HALO) * G::PITCH + tx + HALO;
+    const T* w_b = w + ti.bc * HW;
+    T* g_b = gw + ti.bc * HW;
+
+    A xo[NC], ao[NC], bo[NC], gxa[NC];
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+        xo[c] = xt[c * G::TILE + li];
+        ao[c] = at[c * G::TILE + li];
+        bo[c] = bt[c * G::TILE + li];
+        gxa[c] = A(0);
+    }
+    const A lo = lt[li];
+    SlotRaw<T, 1> wb[D];  // weight prefetch ring, as in the kernels above
+#pragma unroll
+    for (int d = 0; d < D; ++d)
+        slot_load_at<T, 1>(w_b + static_cast<int64_t>(min(d, S - 1)) * wstep, own_b, wb[d]);
+    const T* wr = w_b + static_cast<int64_t>(min(D, S - 1)) * wstep;
+    ShiftRec rn = read_shift(shl, 0);
+    T* gs = g_b;
+
+    // The terms of one weight: its gradient, summed over the channels, from
+    // the neighbour's values; the mirror's x gradient; fo = f(w, L[q]).
+    auto terms = [&](A wv, const A (&xf)[NC], A lp, const A (&ap)[NC], const A (&bp)[NC],
+                     bool okp, A& fo) -> A {
+        const bool masked = LOGW ? wv == -Lim<A>::inf() : wv == A(0);
+        A Ff, Fi, fi;
+        if constexpr (LOGW) {
+            const A kw = log_scale<A>(wv);
+            fo = masked ? A(0) : frac_log<A>(kw, lo);
+            fi = masked ? A(0) : frac_log<A>(kw, lp);
+            Ff = fo;
+            Fi = fi;
+        } else {
+            fo = frac_tile<A, false>(wv, lo);
+            fi = frac_tile<A, false>(wv, lp);
+            Ff = lo;
+            Fi = lp;
+        }
+        A sf = A(0), si = A(0);
+#pragma unroll
+        for (int c = 0; c < NC; ++c) {
+            sf += fma_acc(ao[c], xf[c], bo[c]);
+            si += fma_acc(ap[c], xo[c], bp[c]);
+            if (okp) gxa[c] = fma_acc(fi, ap[c], gxa[c]);
+        }
+        const A gv = fma_acc(Ff, sf, okp ? Fi * si : A(0));
+        return masked ? A(0) : gv;
+    };
+    const int R_all = table_radius(shl, S, false);
+    const bool interior = ti.th == G::TH && ti.tw == G::TW && ti.h0 >= R_all &&
+                          ti.h0 + G::TH + R_all <= H && ti.w0 >= R_all &&
+                          ti.w0 + G::TW + R_all <= W;
+    int last_dx = kClamp;
+    auto step = [&](int s, SlotRaw<T, 1>& slot, auto fast_tag) {
+        constexpr bool FAST = decltype(fast_tag)::value;
+        const ShiftRec rc = rn;
+        rn = read_shift(shl, min(s + 1, S - 1));
+        A w1[1];
+        slot_get<T, 1>(slot, w1);
+        slot_load_at<T, 1>(wr, own_b, slot);
+        wr += s + D + 1 < S ? wstep : 0;
+        if (shift_in_lds(rc)) {
+            if (rc.dx != last_dx) {
+                lds_barrier();
+                last_dx = rc.dx;
+            }
+            const int i = li + rc.dx * G::PITCH + rc.dy;
+            const bool okp = rc.inv && (FAST || rc.per ||
+                                        (in_range(h + rc.dx, H) && in_range(wq + rc.dy, W)));
+            const A wv = FAST || fwd_kept(rc, h, wq, H, W) ? w1[0] : masked_key<A, LOGW>();
+            A xf[NC], ap[NC], bp[NC], m[NC], fo;
+#pragma unroll
+            for (int c = 0; c < NC; ++c) {
+                xf[c] = xt[c * G::TILE + i];
+                ap[c] = at[c * G::TILE + i];
+                bp[c] = bt[c * G::TILE + i];
+                m[c] = mg[c * G::TILE + i];
+            }
+            const A g = terms(wv, xf, lt[i], ap, bp, okp, fo);
+            if (FAST || act) store_elem_at<T, false>(gs, own_b, from_acc<T>(g));
+#pragma unroll
+            for (int c = 0; c < NC; ++c)
+                mg[c * G::TILE + i] = m[c] + (FAST || act ? fo * ao[c] : A(0));
+        }
+        gs += wstep;
+    };
+    auto ring = [&](auto fast_tag) {
+        const int S_ring = S - S % D;
+        for (int s0 = 0; s0 < S_ring; s0 += D) {
+#pragma unroll
+            for (int d = 0; d < D; ++d) step(s0 + d, wb[d], fast_tag);
+        }
+#pragma unroll
+        for (int d = 0; d < D; ++d)
+            if (S_ring + d < S) step(S_ring + d, wb[d], fast_tag);
+    };
+    if (interior)
+        ring(std::true_type{});
+    else
+        ring(std::false_type{});
+    // Shifts beyond the halo: gather form, neighbour values from HBM.
+    for (int s = 0; s < S && act; ++s) {
+        const ShiftRec rc = read_shift(shl, s);
+        if (shift_in_lds(rc)) continue;
+        const T* wp = w_b + static_cast<int64_t>(s) * wstep;
+        const int hp = wrap1(h + rc.dxm, H), hm = wrap1(h - rc.dxm, H);
+        const int wp_ = wrap1(wq + rc.dym, W), wm_ = wrap1(wq - rc.dym, W);
+        const uint32_t jp = static_cast<uint32_t>(hp) * W + wp_;
+        const uint32_t jm = static_cast<uint32_t>(hm) * W + wm_;
+        const int64_t ip = off + jp, im = off + jm;
+        const bool okp = rc.inv && (rc.per || (in_range(h + rc.dx, H) && in_range(wq + rc.dy, W)));
+        A xf[NC], ap[NC], bp[NC], fo;
+#pragma unroll
+        for (int c = 0; c < NC; ++c) {
+            xf[c] = to_acc(x[ip + c * HW]);
+            ap[c] = gDg[ip + c * HW];
+            bp[c] = gLg[ip + c * HW] - ap[c] * Dg[ip + c * HW];
+        }
+        const A lp = LOGW ? log_key<A>(Lg[ip]) : Lim<A>::ex(-Lg[ip]);
+        const A wv = fwd_kept(rc, h, wq, H, W) ? to_acc(wp[own]) : masked_key<A, LOGW>();
+        const A g = terms(wv, xf, lp, ap, bp, okp, fo);
+        g_b[static_cast<int64_t>(s) * wstep + own] = from_acc<T>(g);
+        // x-gradient term from o = (q - s) mod: f(w_s[o], L[o]) gD[o]
+        const A lm = LOGW ? Lg[im] : Lim<A>::ex(-Lg[im]);
+        const A wo = fwd_kept_src(rc, h, wq, H, W) ? to_acc(wp[jm]) : masked_key<A, LOGW>();
+        const A f = frac_tile<A, LOGW>(wo, lm);
+#pragma unroll
+        for (int c = 0; c < NC; ++c) gxa[c] = fma_acc(f, gDg[im + c * HW], gxa[c]);
+    }
+    __syncthreads();
+    if (act) {
+#pragma unroll
+        for (int c = 0; c < NC; ++c) {
+            const A v = gxa[c] + mg[c * G::TILE + li];
+            const int64_t o = off + c * HW + own;
+            if (gxp != nullptr)
+                gxp[o] = v;
+            else
+                gx[o] = from_acc<T>(v);
+        }
+    }
+    if (R == 0) return;
+    const int n = spill_count(ti.th, ti.tw, R);
+    const int64_t per_plane = static_cast<int64_t>(tg.ntw) * tg.nth;
+    const int64_t tile = t - ti.bc * per_plane;
+    for (int e = threadIdx.x; e < n; e += blockDim.x) {
+        int i, j;
+        spill_coords(e, ti.th, ti.tw, R, i, j);
+        const int l = (i + HALO) * G::PITCH + j + HALO;
+#pragma unroll
+        for (int c = 0; c < NC; ++c)
+            spill[((ti.bc * NC + c) * per_plane + tile) * G::SPILL + e] = mg[c * G::TILE + l];
+    }
+}
+
 // ---------------------------------------------------------------------------
 // Host side
 // ---------------------------------------------------------------------------
@@ -1725,6 +1962,73 @@ static int n_run_bwd(const void* x, const void* w, const void* D, const void* L,
     return n_launch_bwd<T, 1, LOGW>(x, w, D, L, gD, gL, sh, d, gx, gw, st);
 }
 
+// The shared-weight backward with the summed gradient: two or three channels
+// of fp32 or 16-bit type on images the tiles serve.
+struct NShPlan {
+    bool ok = false;
+    TileGrid grid{};
+    int64_t tiles = 0, spill_bytes = 0, part_bytes = 0, total = 0;
+    size_t lds = 0;
+};
+
+template <typename T>
+static NShPlan n_shared_plan(const NDims& d) {
+    using G = SGeo<1, kNShRows, kNShTpr>;
+    const int64_t ab = sizeof(acc_t<T>);
+    NShPlan p;
+    p.grid = nsh_host::tile_grid(d.H, d.W, G::TH, G::TW);
+    p.tiles = static_cast<int64_t>(d.B) * p.grid.ntw * p.grid.nth;  // per channel
+    p.lds = shift_lds_bytes(d.S) + (4 * d.C + 1) * static_cast<size_t>(G::TILE) * ab;
+    p.ok = sizeof(T) <= 4 && (d.C == 2 || d.C == 3) && p.grid.narrow >= kRmax &&
+           d.H >= kNScatterMinSide && d.W >= kNScatterMinSide && p.lds <= kNScatterLds;
+    p.spill_bytes = n_align256(p.tiles * d.C * G::SPILL * ab);
+    p.part_bytes = sizeof(T) < sizeof(acc_t<T>)
+                       ? n_align256(static_cast<int64_t>(d.B) * d.C * d.H * d.W * ab)
+                       : 0;
+    p.total = kNHeader + p.spill_bytes + p.part_bytes;
+    return p;
+}
+
+template <typename T, bool LOGW>
+static int n_run_bwd_shared(const void* x, const void* w, const void* D, const void* L,
+                            const void* gD, const void* gL, const int64_t* sh, NDims d, void* gx,
+                            void* gw, void* ws, int64_t ws_bytes, hipStream_t st) {
+    using A = acc_t<T>;
+    using G = SGeo<1, kNShRows, kNShTpr>;
+    const NShPlan p = n_shared_plan<T>(d);
+    if (!p.ok || n_scatter_disabled() || ws == nullptr || ws_bytes < p.total ||
+        !nsh_host::aligned(ws, 256))
+        return nsh_host::fail(NSH_ERR_UNSUPPORTED,
+                              "normalized_accumulate_uz_backward_shared: shape or workspace not "
+                              "served");
+    char* base = static_cast<char*>(ws);
+    int* hdr = reinterpret_cast<int*>(base);
+    A* spill = reinterpret_cast<A*>(base + kNHeader);
+    A* part = p.part_bytes ? reinterpret_cast<A*>(base + kNHeader + p.spill_bytes) : nullptr;
+    const int64_t wstep = static_cast<int64_t>(d.B) * d.H * d.W;
+    auto go = [&](auto nc) {
+        hipLaunchKernelGGL((normalized_bwd_shared_kernel<T, decltype(nc)::value, LOGW>),
+                           dim3(static_cast<unsigned>(p.tiles)), dim3(G::THREADS), p.lds, st,
+                           static_cast<const T*>(x), static_cast<const T*>(w),
+                           static_cast<const A*>(D), static_cast<const A*>(L),
+                           static_cast<const A*>(gD), static_cast<const A*>(gL), sh, d.S, d.codes,
+                           d.H, d.W, p.grid, wstep, static_cast<T*>(gx), part,
+                           static_cast<T*>(gw), hdr, spill);
+    };
+    if (d.C == 2)
+        go(std::integral_constant<int, 2>{});
+    else
+        go(std::integral_constant<int, 3>{});
+    if (int rc = nsh_host::check_launch("normalized_accumulate_uz_backward_shared")) return rc;
+    constexpr bool kPart = sizeof(T) < sizeof(A);
+    hipLaunchKernelGGL((spill_fixup_kernel<T, A, 1, kPart>),
+                       dim3(static_cast<unsigned>(p.tiles * d.C)), dim3(256), 0, st, d.H, d.W,
+                       G::TH, G::TW, p.grid, G::SPILL, static_cast<const int*>(hdr),
+                       static_cast<const A*>(spill), p.tiles * d.C, static_cast<const A*>(part),
+                       static_cast<T*>(gx), static_cast<T*>(nullptr));
+    return nsh_host::check_launch("normalized_accumulate_uz_backward_shared (fix-up)");
+}
+
 }  // namespace nsh
 
 using nsh_host::fail;
@@ -1874,5 +2178,50 @@ extern "C" int nsh_normalized_accumulate_uz_backward(const void* x, const void* 
             return NSH_DISPATCH_LOGW(float, n_run_bwd, x, weights, D, log_C, grad_D, grad_log_C, shifts, d, grad_x, grad_w, ws, nws, st);
         default:
             return NSH_DISPATCH_LOGW(double, n_run_bwd, x, weights, D, log_C, grad_D, grad_log_C, shifts, d, grad_x, grad_w, ws, nws, st);
+    }
+}
+
+extern "C" int64_t nsh_normalized_shared_workspace_bytes(int64_t S, int64_t B, int64_t C, int64_t H,
+                                                         int64_t W, int dtype) {
+    nsh::NDims d;
+    if (n_check("normalized_accumulate_uz_backward_shared", S, B, C, H, W, dtype, &d)) return -1;
+    switch (dtype & ~NSH_DTYPE_FLAGS) {
+        case NSH_DTYPE_FLOAT16:
+        case NSH_DTYPE_BFLOAT16: {
+            const nsh::NShPlan p = nsh::n_shared_plan<nsh::f16>(d);
+            return p.ok ? p.total : 0;
+        }
+        case NSH_DTYPE_FLOAT32: {
+            const nsh::NShPlan p = nsh::n_shared_plan<float>(d);
+            return p.ok ? p.total : 0;
+        }
+        default: return 0;
+    }
+}
+
+extern "C" int nsh_normalized_accumulate_uz_backward_shared(
+    const void* x, const void* weights, const void* D, const void* log_C, const void* grad_D,
+    const void* grad_log_C, const int64_t* shifts, int64_t S, int64_t B, int64_t C, int64_t H,
+    int64_t W, int dtype, int log_weights, void* grad_x, void* grad_w, void* workspace,
+    int64_t workspace_bytes, void* stream) {
+    nsh::NDims d;
+    if (int rc = n_check("normalized_accumulate_uz_backward_shared", S, B, C, H, W, dtype, &d))
+        return rc;
+    dtype &= ~NSH_DTYPE_FLAGS;
+    if (!x || !weights || !D || !log_C || !grad_D || !grad_log_C || !shifts || !grad_x || !grad_w)
+        return fail(NSH_ERR_INVALID,
+                    "normalized_accumulate_uz_backward_shared: null pointer argument");
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    const int64_t nws = workspace ? workspace_bytes : 0;
+    switch (dtype) {
+        case NSH_DTYPE_FLOAT16:
+            return NSH_DISPATCH_LOGW(nsh::f16, n_run_bwd_shared, x, weights, D, log_C, grad_D, grad_log_C, shifts, d, grad_x, grad_w, workspace, nws, st);
+        case NSH_DTYPE_BFLOAT16:
+            return NSH_DISPATCH_LOGW(nsh::bf16, n_run_bwd_shared, x, weights, D, log_C, grad_D, grad_log_C, shifts, d, grad_x, grad_w, workspace, nws, st);
+        case NSH_DTYPE_FLOAT32:
+            return NSH_DISPATCH_LOGW(float, n_run_bwd_shared, x, weights, D, log_C, grad_D, grad_log_C, shifts, d, grad_x, grad_w, workspace, nws, st);
+        default:
+            return fail(NSH_ERR_UNSUPPORTED,
+                        "normalized_accumulate_uz_backward_shared: fp64 is not served");
     }
 }

@@ -526,6 +526,15 @@ def mix_head_planes(w: torch.Tensor, mix: torch.Tensor) -> torch.Tensor:
     return (mix.to(w.dtype).view(1, C, h, 1) * w.reshape(N, 1, h, P)).sum(2)
 
 
+# Shared weights' own gradient is formed in one pass from this many pixels
+# (B * H * W) on.  Below, a forward and backward take the host longer (~150 us)
+# than the kernels either way (1x3x72x200 R = 3: 50 us per channel, 27 in one
+# pass), and the per-channel kernels' x gradient is the broadcast weights' bit
+# for bit; above, 8x3x250^2 R = 5 fp32 takes 330 us per channel
+# (two kernels and the sum) and 112 in one pass.
+_ONE_PASS_PIXELS = 1 << 15
+
+
 class _NormalizedAccumulateUZFn(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x, weights, shifts, log_weights, rules=0, shared=False, weights_ok=None):
@@ -551,6 +560,13 @@ class _NormalizedAccumulateUZFn(torch.autograd.Function):
             grad_D = torch.zeros_like(D)
         if grad_log_C is None:
             grad_log_C = torch.zeros_like(log_C)
+        if ctx.shared and x.numel() // x.size(1) >= _ONE_PASS_PIXELS:
+            # their own gradient in one pass, where that is served
+            grads = _C.normalized_accumulate_uz_backward_shared(
+                x, weights, D, log_C, grad_D.contiguous(), grad_log_C.contiguous(), shifts_i,
+                ctx.log_weights, rules=ctx.rules)
+            if grads is not None:
+                return grads[0], grads[1], None, None, None, None, None
         grad_x, grad_w = _C.normalized_accumulate_uz_backward(
             x, weights, D, log_C, grad_D.contiguous(), grad_log_C.contiguous(), shifts_i,
             ctx.log_weights, rules=ctx.rules, shared_weights=ctx.shared)
