@@ -249,9 +249,9 @@ NSH_API int64_t nsh_accumulate_uz_workspace_bytes(int64_t S, int64_t B, int64_t 
  * array of NSH_NOALLOC_SCRATCH_BYTES that every GPU the library runs on
  * holds until the process ends (the current device's copy is used; a
  * non-null stream of another device is rejected with NSH_ERR_INVALID).  A
- * shape whose workspace (nsh_accumulate_uz_workspace_bytes) exceeds it is
- * rejected with NSH_ERR_INVALID; shapes that need none run the gather
- * kernels.  Every call on one GPU shares that GPU's array: calls that
+ * shape whose tiles need more than it is rejected with NSH_ERR_INVALID,
+ * except images ending 1..7 pixels past whole 16s, which then run the gather
+ * kernels, as shapes that need none do.  Every call on one GPU shares that GPU's array: calls that
  * overlap on one GPU (other streams or threads) race, so the caller must
  * serialize them. */
 #define NSH_NOALLOC_SCRATCH_BYTES (32ll << 20)

@@ -17,6 +17,7 @@
 // cross-lane traffic at all.  The mirror term re-reads w_s at p-s: the
 // same cache lines the tile (or its neighbour on the same XCD) has just
 // streamed, so that read is served by L1/L2 rather than HBM.
+#include <limits>
 #include <algorithm>
 #include <cstdio>
 #include <cstdlib>
@@ -1243,9 +1244,11 @@ static int64_t one_round_tiles() { return nsh_host::compute_units(); }
 
 // The plan for a shape: with the wide halo asked for, the 16- or
 // 24-pixel-border tiles where they apply; else by the rule above; *var says
-// which (p.ok false if none applies).
+// which (p.ok false if none applies).  A forward whose workspace holds
+// `room` bytes, too few for the 64-wide tiles but enough for the wide ones
+// (7 and 5.5 bytes a pixel), takes those.
 template <typename T, int VEC, bool BWD>
-static SPlan scatter_plan_for(const Dims& d, int* var) {
+static SPlan scatter_plan_for(const Dims& d, int64_t room, int* var) {
     if constexpr (ScatterCfg<T, VEC, BWD, kVarWide>::kWide) {
         if (d.halo > kRmax) {
             // radius 9..16 on tiles that end in one shorter than 16 (the
@@ -1268,9 +1271,10 @@ static SPlan scatter_plan_for(const Dims& d, int* var) {
         const int64_t cu = one_round_tiles();
         const double rounds = 0.9 * static_cast<double>(nsh_host::ceil_div(wide.tiles, cu));
         if constexpr (!BWD) {
-            if (sizeof(T) == 2 || wide.tiles < cu ||
-                (wide.tiles > cu && rounds > static_cast<double>(alt.tiles) / (2 * cu)))
-                return alt;
+            const bool narrow =
+                sizeof(T) == 2 || wide.tiles < cu ||
+                (wide.tiles > cu && rounds > static_cast<double>(alt.tiles) / (2 * cu));
+            if (narrow && (alt.total <= room || wide.total > room)) return alt;
         } else {
             const SPlan half = scatter_plan_cfg<T, VEC, BWD, kVarShort>(d);
             if (wide.tiles < cu) {
@@ -1291,20 +1295,22 @@ static SPlan scatter_plan_for(const Dims& d, int* var) {
 }
 
 template <typename T, bool BWD>
-static SPlan scatter_plan_any(const Dims& d, int vec, int* var) {
+static SPlan scatter_plan_any(const Dims& d, int vec, int64_t room, int* var) {
     switch (vec) {
-        case 4: if constexpr (sizeof(T) <= 4) return scatter_plan_for<T, 4, BWD>(d, var); break;
-        case 2: return scatter_plan_for<T, 2, BWD>(d, var);
+        case 4: if constexpr (sizeof(T) <= 4) return scatter_plan_for<T, 4, BWD>(d, room, var); break;
+        case 2: return scatter_plan_for<T, 2, BWD>(d, room, var);
         default: break;
     }
-    return scatter_plan_for<T, 1, BWD>(d, var);
+    return scatter_plan_for<T, 1, BWD>(d, room, var);
 }
 
+// Workspace of a pass, of the tiles it takes where the caller has `room`.
 template <typename T>
-static int64_t scatter_workspace(const Dims& d, bool bwd) {
+static int64_t scatter_workspace(const Dims& d, bool bwd,
+                                 int64_t room = std::numeric_limits<int64_t>::max()) {
     int var;
-    const SPlan p = bwd ? scatter_plan_any<T, true>(d, scatter_vec<T>(d, true), &var)
-                        : scatter_plan_any<T, false>(d, scatter_vec<T>(d, false), &var);
+    const SPlan p = bwd ? scatter_plan_any<T, true>(d, scatter_vec<T>(d, true), room, &var)
+                        : scatter_plan_any<T, false>(d, scatter_vec<T>(d, false), room, &var);
     return p.ok ? p.total : 0;
 }
 
@@ -1418,7 +1424,8 @@ static int launch_scatter_var(int var, const void* x, const void* w, const void*
         if constexpr (BWD)
             if (var == kVarShort) return go(std::integral_constant<int, kVarShort>{});
     }
-    if (var == kVarAlt) return go(std::integral_constant<int, kVarAlt>{});
+    if constexpr (ScatterCfg<T, VEC, BWD, kVarWide>::kWide)
+        if (var == kVarAlt) return go(std::integral_constant<int, kVarAlt>{});
     return go(std::integral_constant<int, kVarWide>{});
 }
 
@@ -1431,7 +1438,7 @@ static int try_scatter(const void* x, const void* w, const void* gU, const void*
     if (ws == nullptr || scatter_disabled()) return -1;
     const int v = scatter_vec<T>(d, BWD);
     int var = kVarWide;
-    const SPlan p = scatter_plan_any<T, BWD>(d, v, &var);
+    const SPlan p = scatter_plan_any<T, BWD>(d, v, ws_bytes, &var);
     if (!p.ok || ws_bytes < p.total || !nsh_host::aligned(ws, 256)) return -1;
     // whether the lanes' vectors fit the rows and buffers; both forms exist
     const size_t vb = static_cast<size_t>(v) * sizeof(T);
@@ -1501,18 +1508,27 @@ static int check_acc_dims(const char* op, int64_t S, int64_t B, int64_t C, int64
     return NSH_OK;
 }
 
-extern "C" int64_t nsh_accumulate_uz_workspace_bytes(int64_t S, int64_t B, int64_t C, int64_t H,
-                                                     int64_t W, int dtype, int backward) {
+static int64_t acc_workspace(int64_t S, int64_t B, int64_t C, int64_t H, int64_t W, int dtype,
+                             bool bwd, int64_t room) {
     nsh::Dims d;
     if (check_acc_dims("accumulate_uz_workspace_bytes", S, B, C, H, W, dtype, &d)) return -1;
-    dtype &= ~NSH_DTYPE_FLAGS;
-    const bool bwd = backward != 0;
-    switch (dtype) {
-        case NSH_DTYPE_FLOAT16: return nsh::scatter_workspace<nsh::f16>(d, bwd);
-        case NSH_DTYPE_BFLOAT16: return nsh::scatter_workspace<nsh::bf16>(d, bwd);
-        case NSH_DTYPE_FLOAT32: return nsh::scatter_workspace<float>(d, bwd);
-        default: return nsh::scatter_workspace<double>(d, bwd);
+    switch (dtype & ~NSH_DTYPE_FLAGS) {
+        case NSH_DTYPE_FLOAT16: return nsh::scatter_workspace<nsh::f16>(d, bwd, room);
+        case NSH_DTYPE_BFLOAT16: return nsh::scatter_workspace<nsh::bf16>(d, bwd, room);
+        case NSH_DTYPE_FLOAT32: return nsh::scatter_workspace<float>(d, bwd, room);
+        default: return nsh::scatter_workspace<double>(d, bwd, room);
     }
+}
+
+int64_t nsh_host::accumulate_forward_workspace(int64_t S, int64_t B, int64_t C, int64_t H,
+                                               int64_t W, int dtype, int64_t room) {
+    return acc_workspace(S, B, C, H, W, dtype, false, room);
+}
+
+extern "C" int64_t nsh_accumulate_uz_workspace_bytes(int64_t S, int64_t B, int64_t C, int64_t H,
+                                                     int64_t W, int dtype, int backward) {
+    return acc_workspace(S, B, C, H, W, dtype, backward != 0,
+                         std::numeric_limits<int64_t>::max());
 }
 
 // Optional band: local row h is image row (row_origin + h) mod image_height

@@ -84,13 +84,19 @@ extern "C" int nsh_accumulate_uz_forward_noalloc(const void* x, const void* weig
         return nsh_accumulate_uz_forward(x, weights, shifts, S, B, C, H, W, dtype, U, Z, nullptr,
                                          0, stream);
     }
-    if (need > NSH_NOALLOC_SCRATCH_BYTES)
+    // The preferred tiles may need more than the scratch where others fit it.
+    const int64_t fits = nsh_host::accumulate_forward_workspace(S, B, C, H, W, dtype,
+                                                                NSH_NOALLOC_SCRATCH_BYTES);
+    // An image that ends 1..7 pixels past whole 16s does not depend on tiles:
+    // the gather kernels, which use no workspace, serve it at any size.
+    const bool ragged = (H % 16 != 0 && H % 16 < 8) || (W % 16 != 0 && W % 16 < 8);
+    if (fits > NSH_NOALLOC_SCRATCH_BYTES && !ragged)
         return nsh_host::fail(NSH_ERR_INVALID,
                               "accumulate_uz_forward_noalloc: this shape needs a %lld-byte "
                               "workspace, above the %lld-byte static scratch; use "
                               "nsh_accumulate_uz_forward with a caller workspace",
                               (long long)need, (long long)NSH_NOALLOC_SCRATCH_BYTES);
-    if (need == 0)  // the shape takes the gather kernels, which use no workspace
+    if (need == 0 || fits > NSH_NOALLOC_SCRATCH_BYTES)  // the gather kernels
         return nsh_accumulate_uz_forward(x, weights, shifts, S, B, C, H, W, dtype, U, Z, nullptr,
                                          0, stream);
     void* ws = nullptr;

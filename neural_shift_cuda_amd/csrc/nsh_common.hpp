@@ -603,6 +603,13 @@ __device__ __forceinline__ bool shift_in_lds(const ShiftRec& r) {
 // Host side: error channel and launch helpers (defined in nsh_capi.cpp).
 // ---------------------------------------------------------------------------
 namespace nsh_host {
+
+// Workspace of the accumulate_uz forward on the tiles it takes where the
+// caller has `room` bytes (above `room` if none fit, 0 if it needs none, -1
+// for invalid arguments).
+int64_t accumulate_forward_workspace(int64_t S, int64_t B, int64_t C, int64_t H, int64_t W,
+                                     int dtype, int64_t room);
+
 int fail(int code, const char* fmt, ...);
 int check_launch(const char* what);
 bool aligned(const void* p, size_t bytes);
