@@ -250,10 +250,12 @@ NSH_API int64_t nsh_accumulate_uz_workspace_bytes(int64_t S, int64_t B, int64_t 
  * holds until the process ends (the current device's copy is used; a
  * non-null stream of another device is rejected with NSH_ERR_INVALID).  A
  * shape whose tiles need more than it is rejected with NSH_ERR_INVALID,
- * except images ending 1..7 pixels past whole 16s, which then run the gather
- * kernels, as shapes that need none do.  Every call on one GPU shares that GPU's array: calls that
- * overlap on one GPU (other streams or threads) race, so the caller must
- * serialize them. */
+ * except images of one tile row or column (at most 32 rows, 16 for fp64; at
+ * most 16 v columns, v the widest of 4 (2 for fp64), 2 and 1 that divides W)
+ * and images ending 1..7 pixels past whole 16s: at any batch size these then
+ * run the gather kernels, as shapes that need none do.  Every call on one GPU
+ * shares that GPU's array: calls that overlap on one GPU (other streams or
+ * threads) race, so the caller must serialize them. */
 #define NSH_NOALLOC_SCRATCH_BYTES (32ll << 20)
 NSH_API int nsh_accumulate_uz_forward_noalloc(const void* x, const void* weights,
                                               const int64_t* shifts, int64_t S, int64_t B,

@@ -1244,9 +1244,11 @@ static int64_t one_round_tiles() { return nsh_host::compute_units(); }
 
 // The plan for a shape: with the wide halo asked for, the 16- or
 // 24-pixel-border tiles where they apply; else by the rule above; *var says
-// which (p.ok false if none applies).  A forward whose workspace holds
-// `room` bytes, too few for the 64-wide tiles but enough for the wide ones
-// (7 and 5.5 bytes a pixel), takes those.
+// which (p.ok false if none applies).  A pass whose workspace holds `room`
+// bytes, too few for the wider border's tiles, takes those of the 8-pixel
+// border (such a table's rows then run the gather form inside the launch), and
+// a forward with too few for the 64-wide tiles but enough for the wide ones
+// (7 and 5.5 bytes a pixel) takes those.
 template <typename T, int VEC, bool BWD>
 static SPlan scatter_plan_for(const Dims& d, int64_t room, int* var) {
     if constexpr (ScatterCfg<T, VEC, BWD, kVarWide>::kWide) {
@@ -1258,7 +1260,7 @@ static SPlan scatter_plan_for(const Dims& d, int64_t room, int* var) {
             const SPlan q24 = scatter_plan_cfg<T, VEC, BWD, kVarHalo24>(d);
             const bool wider = d.halo > 16 || (q16.grid.narrow < 16 && q24.grid.narrow >= 16);
             const SPlan q = wider ? q24 : q16;
-            if (q.ok) {
+            if (q.ok && q.total <= room) {
                 *var = wider ? kVarHalo24 : kVarHalo16;
                 return q;
             }

@@ -72,6 +72,18 @@ int device_scratch(hipStream_t stream, void** out) {
     return NSH_OK;
 }
 
+// Whether a shape whose tiles all need more than the scratch runs on the
+// gather kernels, which use none: an image of a single tile row or column
+// (16 lanes of the widest vector that divides W, 32 rows, 16 for fp64), or
+// one that ends 1..7 pixels past whole 16s, at any batch size.  Larger images
+// are refused: the caller finds out that a workspace pays there.
+bool gather_serves(int64_t H, int64_t W, int dtype) {
+    const bool f64 = dtype == NSH_DTYPE_FLOAT64;
+    const int64_t vec = W % 4 == 0 && !f64 ? 4 : (W % 2 == 0 ? 2 : 1);
+    const auto ragged = [](int64_t n) { return n % 16 != 0 && n % 16 < 8; };
+    return W <= 16 * vec || H <= (f64 ? 16 : 32) || ragged(H) || ragged(W);
+}
+
 }  // namespace
 
 extern "C" int nsh_accumulate_uz_forward_noalloc(const void* x, const void* weights,
@@ -87,16 +99,13 @@ extern "C" int nsh_accumulate_uz_forward_noalloc(const void* x, const void* weig
     // The preferred tiles may need more than the scratch where others fit it.
     const int64_t fits = nsh_host::accumulate_forward_workspace(S, B, C, H, W, dtype,
                                                                 NSH_NOALLOC_SCRATCH_BYTES);
-    // An image that ends 1..7 pixels past whole 16s does not depend on tiles:
-    // the gather kernels, which use no workspace, serve it at any size.
-    const bool ragged = (H % 16 != 0 && H % 16 < 8) || (W % 16 != 0 && W % 16 < 8);
-    if (fits > NSH_NOALLOC_SCRATCH_BYTES && !ragged)
+    if (fits > NSH_NOALLOC_SCRATCH_BYTES && !gather_serves(H, W, dtype & ~NSH_DTYPE_FLAGS))
         return nsh_host::fail(NSH_ERR_INVALID,
                               "accumulate_uz_forward_noalloc: this shape needs a %lld-byte "
                               "workspace, above the %lld-byte static scratch; use "
                               "nsh_accumulate_uz_forward with a caller workspace",
                               (long long)need, (long long)NSH_NOALLOC_SCRATCH_BYTES);
-    if (need == 0 || fits > NSH_NOALLOC_SCRATCH_BYTES)  // the gather kernels
+    if (fits == 0 || fits > NSH_NOALLOC_SCRATCH_BYTES)  // the gather kernels
         return nsh_accumulate_uz_forward(x, weights, shifts, S, B, C, H, W, dtype, U, Z, nullptr,
                                          0, stream);
     void* ws = nullptr;
