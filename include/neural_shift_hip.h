@@ -252,8 +252,9 @@ NSH_API int64_t nsh_accumulate_uz_workspace_bytes(int64_t S, int64_t B, int64_t 
  * shape whose tiles need more than it is rejected with NSH_ERR_INVALID,
  * except images of one tile row or column (at most 32 rows, 16 for fp64; at
  * most 16 v columns, v the widest of 4 (2 for fp64), 2 and 1 that divides W)
- * and images ending 1..7 pixels past whole 16s: at any batch size these then
- * run the gather kernels, as shapes that need none do.  Every call on one GPU
+ * and images ending 1..7 pixels past whole 16s, and except under the wide
+ * border hints: these then run the gather kernels at any batch size, as shapes
+ * that need none do.  Every call on one GPU
  * shares that GPU's array: calls that overlap on one GPU (other streams or
  * threads) race, so the caller must serialize them. */
 #define NSH_NOALLOC_SCRATCH_BYTES (32ll << 20)

@@ -408,7 +408,7 @@ def accumulate_uz_forward(x: torch.Tensor, weights: torch.Tensor,
             | _halo_flag(shifts))
     U = torch.empty(x.shape, dtype=acc, device=x.device)
     Z = torch.empty(x.shape, dtype=acc, device=x.device)
-    ws, nws = _workspace(S, B, C, H, W, code, False, x.device)
+    ws, nws = _workspace(S, B, C, H, W, code, False, x.device, shifts)
     if band is None:
         _call_on(x, "nsh_accumulate_uz_forward", x.data_ptr(), weights.data_ptr(), sh.data_ptr(),
                  S, B, C, H, W, code, U.data_ptr(), Z.data_ptr(), _ptr(ws), nws)
@@ -420,13 +420,20 @@ def accumulate_uz_forward(x: torch.Tensor, weights: torch.Tensor,
     return [U, Z]
 
 
-def _workspace(S, B, C, H, W, code, backward, device):
+def _workspace(S, B, C, H, W, code, backward, device, shifts):
     """Scratch buffer of accumulate_uz (spilled window borders of the
-    once-per-element weight stream); (None, 0) when the shape needs none."""
+    once-per-element weight stream); (None, 0) when the shape needs none, and
+    for a table beyond every border (24 pixels), all of whose rows would run
+    the gather form at the tiles' occupancy, which only a backward on whole
+    vectors of whole tiles does as fast as the gather kernels."""
     n = _bytes_on(device.index, "nsh_accumulate_uz_workspace_bytes", S, B, C, H, W, code,
                   int(backward))
     if n <= 0:
         return None, 0
+    if not code & (NSH_WIDE_HALO | NSH_WIDER_HALO) and not (backward and W % 16 == H % 16 == 0):
+        r = table_radius(shifts)
+        if r is not None and r > 24:
+            return None, 0
     return torch.empty(n, dtype=torch.uint8, device=device), n
 
 
@@ -453,7 +460,7 @@ def accumulate_uz_backward(x: torch.Tensor, weights: torch.Tensor, grad_U: torch
             | _halo_flag(shifts))
     gx = torch.empty_like(x)
     gw = torch.empty((S * B, C, H, W), dtype=weights.dtype, device=weights.device)
-    ws, nws = _workspace(S, B, C, H, W, code, True, x.device)
+    ws, nws = _workspace(S, B, C, H, W, code, True, x.device, shifts)
     if band is None:
         _call_on(x, "nsh_accumulate_uz_backward", x.data_ptr(), weights.data_ptr(),
                  gU.data_ptr(), gZ.data_ptr(), sh.data_ptr(), S, B, C, H, W, code, gx.data_ptr(),

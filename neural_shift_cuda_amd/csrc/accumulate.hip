@@ -1146,8 +1146,10 @@ constexpr int64_t kCachedBytes = int64_t(192) << 20;
 
 struct SPlan {
     bool ok = false;
+    bool even = false;  // whole vectors, two tiles each way, none of them shifted
     int rows = 0, spill = 0, halo = kRmax;
     TileGrid grid{};
+    double padded = 1;  // lanes' pixels over the image's
     int64_t tiles = 0, spill_bytes = 0, part_bytes = 0, total = 0;
     size_t lds = 0;
 };
@@ -1179,6 +1181,10 @@ static SPlan scatter_plan(const Dims& d, int vec, int tpr, int rows, int halo, s
     p.grid = nsh_host::tile_grid(d.H, d.W, TH, TW, std::max(kRmax, std::min(d.halo, halo)));
     p.ok = p.lds <= kScatterLdsLimit && TH >= halo && p.grid.narrow >= kRmax &&
            d.H >= kScatterMinSide && d.W >= kScatterMinSide;
+    p.even = d.W % vec == 0 && p.grid.ntw >= 2 && p.grid.nth >= 2 &&
+             p.grid.wl == (p.grid.ntw - 1) * TW && p.grid.hl == (p.grid.nth - 1) * TH;
+    p.padded = static_cast<double>(p.grid.ntw) * TW * p.grid.nth * TH /
+               (static_cast<double>(d.H) * d.W);
     p.tiles = static_cast<int64_t>(d.B) * d.C * p.grid.ntw * p.grid.nth;
     p.spill = 2 * halo * (TW + 2 * halo) + 2 * halo * TH;
     p.spill_bytes = align256((bwd ? 1 : 2) * p.tiles * p.spill * static_cast<int64_t>(asize));
@@ -1296,14 +1302,48 @@ static SPlan scatter_plan_for(const Dims& d, int64_t room, int* var) {
     }
 }
 
+// Whether the gather kernels beat a plan that fits (scatter -> gather, in us):
+//  * tables known to reach beyond the plan's border, whose rows would all run
+//    the gather form inside the launch, on rows that the lanes' vectors do not
+//    divide (fp64 4 x 280 x 391 R = 9 forward 524 -> 286, backward 1121 -> 615;
+//    fp16 3 x 953 x 97 R = 10 433 -> 267 and 472 -> 272), in fp64 forwards (1183 x
+//    212 R = 10 501 -> 305) and in backwards on shifted tiles of fewer than two
+//    fp64 values a lane (fp32 773 x 276 230 -> 206, bf16 3 x 187 x 680 398 -> 354).
+//    Otherwise, and on small images, it is level or ahead (fp32 8 x 51 x 1118
+//    forward 252, gather 318; fp64 592^2 backward 348, 398, 24 x 118^2 462, 540,
+//    55^2 128, 176, 16 x 32^2 forward 87, 100);
+//  * tables of a few rows on many images that fill their tiles badly, for the
+//    spilled borders and the fix-up cost as much as the rows, if their rows
+//    are whole 16-byte vectors of the gather kernels (R = 1: fp32 154 x 259 x
+//    100 forward 58 -> 37, bf16 1082 x 66 x 56 67 -> 52; others and fewer or
+//    fuller ones keep the tiles: fp32 R = 1 100 x 100^2 forward 28, gather 27,
+//    1443 x 66 x 42 backward 100, gather 154, fp16 window R = 1 192 x 67 x 805
+//    115, gather 292), and in fp64 forwards on shifted or strided tiles (3 x
+//    660^2 46 -> 20).
+static bool gather_instead(const SPlan& p, const Dims& d, int vec, size_t tsize, bool bwd) {
+    const int64_t pixels = static_cast<int64_t>(d.B) * d.C * d.H * d.W;
+    if (d.halo > p.halo) {
+        if (d.W % vec != 0) return true;
+        return bwd ? !p.even && !(tsize == 8 && vec == 2) && pixels >= (int64_t(1) << 17)
+                   : tsize == 8 && pixels >= (int64_t(3) << 13);
+    }
+    if (d.S > 9 || p.even) return false;
+    if (tsize == 8) return !bwd && pixels >= (int64_t(1) << 18);
+    return p.padded >= 1.4 && d.W * tsize % 16 == 0 && pixels >= (int64_t(3) << 19);
+}
+
 template <typename T, bool BWD>
 static SPlan scatter_plan_any(const Dims& d, int vec, int64_t room, int* var) {
-    switch (vec) {
-        case 4: if constexpr (sizeof(T) <= 4) return scatter_plan_for<T, 4, BWD>(d, room, var); break;
-        case 2: return scatter_plan_for<T, 2, BWD>(d, room, var);
-        default: break;
+    SPlan p;
+    if (vec == 4) {
+        if constexpr (sizeof(T) <= 4) p = scatter_plan_for<T, 4, BWD>(d, room, var);
+    } else if (vec == 2) {
+        p = scatter_plan_for<T, 2, BWD>(d, room, var);
+    } else {
+        p = scatter_plan_for<T, 1, BWD>(d, room, var);
     }
-    return scatter_plan_for<T, 1, BWD>(d, room, var);
+    p.ok = p.ok && !gather_instead(p, d, vec, sizeof(T), BWD);
+    return p;
 }
 
 // Workspace of a pass, of the tiles it takes where the caller has `room`.

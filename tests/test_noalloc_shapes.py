@@ -1,7 +1,7 @@
 """Which shapes nsh_accumulate_uz_forward_noalloc takes: those whose tiles fit
 its static scratch, images of one tile row or column and images ending 1..7
-pixels past whole 16s at any batch size (gather kernels), and, under the
-wide-border hints, whatever the 8-pixel border's tiles would serve."""
+pixels past whole 16s at any batch size (gather kernels), and tables
+hinted beyond 8 pixels whose wider border's tiles do not fit."""
 from __future__ import annotations
 
 import ctypes
@@ -31,6 +31,8 @@ SERVED = [
     (225, 1, 3, 1280, 768, BF16 | WIDE),
     (225, 2, 1, 2856, 458, F16 | WIDE),
     (225, 4, 1, 681, 555, F32 | WIDER),
+    (85, 235, 1, 60, 268, F16 | _C.NSH_NARROW_HALO),
+    (113, 7, 2, 1088, 304, F32),
     (85, 1, 1, 8191, 8193, F32),
 ]
 REFUSED = [
@@ -38,7 +40,6 @@ REFUSED = [
     (113, 8, 1, 2048, 2048, F16),
     (5, 600, 3, 96, 128, F32),
     (225, 16, 1, 1024, 1024, F64),
-    (225, 4, 3, 1024, 1024, F32 | WIDE),
 ]
 
 
