@@ -1198,21 +1198,67 @@ static SPlan scatter_plan(const Dims& d, int vec, int tpr, int rows, int halo, s
 
 // Pixels per lane of the scatter path, from the shape alone (the workspace
 // size must not depend on pointer values).  Any W: the forward's lanes are
-// strided, and the backward's are where W is no multiple.  Small problems
-// trade wide lanes for more of them; half-plane R = 5, 4 / 2 / 1 pixels per
-// lane, in us: fp32 forward 3 x 512^2 (0.79 M pixels) 49 / 48 / 73, 2 x 3 x 321 x
-// 481 (0.93 M) 69 / 75 / 98, 4 x 250^2 (0.25 M) 37 / 32 / 35, 256^2 37 / 29 / 26;
-// fp32 backward 2 x 3 x 71 x 654 (0.28 M) 52 / 54 / 60, 4 x 250^2 52 / 46 / 49;
-// 16-bit backward 2 x 3 x 320 x 480 (0.92 M) 73 / 87 / 137, 3 x 512^2 71 / 65 /
-// 107.  fp64 takes 2 from 0.26 M pixels on (c3 fp64, 0.39 M: forward 78 / 112,
-// backward 173 / 179).
+// strided, and the backward's are where W is no multiple.  A tile of wider
+// lanes takes longer, so narrow lanes win while their tiles (16 v x 32 pixels;
+// 16 v x 16 for fp64) all run at once: three workgroups per compute unit in the
+// backward, four of fp64, and one more tile starts another round.  Half-plane
+// R = 5 except where said, 4 / 2 / 1 pixels per lane, in us:
+//  * forward: fp32 256^2 37 / 29 / 26, 4 x 250^2 (0.25 M pixels) 37 / 32 / 35,
+//    768^2 (0.59 M) 47 / 43 / 58, R = 7 656^2 (0.43 M) 59 / 55 / 78, R = 3 894^2
+//    (0.80 M) 30 / 34 / 51; 16-bit 576^2 (0.33 M) 37 / 36 / 39, R = 6 864^2 (0.75
+//    M) 61 / 54 / -, 2 x 633 x 663 (0.84 M) 63 / 67 / 94, R = 7 1520 x 524 (0.80 M)
+//    78 / 83 / 114 (without mirror rows 4 pixels win from 0.6 M on: window R = 4
+//    8 x 304^2 fp32 41 / 46 / 58, 16-bit 32 / 42 / 55);
+//  * backward, rows of whole 16s: fp32 R = 3 512^2 (512 tiles of 1-pixel
+//    lanes) 30 / 24 / 23, window R = 4 16 x 144^2 (720) 71 / 64 / 57, 16 x 160^2
+//    (800; 400 of 2-pixel lanes) 71 / 65 / 77, 4 x 384^2 (576) 88 / 78 / 92,
+//    8 x 304^2 (800) 92 / 116 / 152; 16-bit, two per compute unit, 512^2 R = 6
+//    (512) 77 / 53 / 52, window R = 7 592^2 (703) 2 and 1 pixels 153 / 177, 96 x
+//    64^2 (768) 138 / 214, window R = 4 8 x 304^2 95 / 108 / 138;
+//  * backward, other rows, whose narrow tiles' rows are parts of lines: fp32
+//    R = 6 447 x 481 (0.22 M) 69 / 53 / 65, 2 x 367 x 389 (0.29 M) 69 / 63 / 90,
+//    519 x 518 R = 4 window (0.27 M) 62 / 65 / 79, 6 x 273 x 305 (0.50 M) 81 / 80 /
+//    110 (wide tiles 100), R = 3 774^2 (0.60 M) 36 / 42 / 55; 16-bit window R = 5
+//    504^2 (0.25 M) - / 64 / 78, 2 x 317 x 337 (0.21 M) 97 / 68 / 73;
+//  * backward, 2.0 to 2.5 tiles of 4-pixel lanes per compute unit, where two
+//    run at once: 8 x 352^2 16-bit 116 / 88 / 138, fp32 window R = 5 280 / 246 /
+//    307; and where 64-wide tiles idle a fifth of their lanes that 32-wide ones
+//    use, below 1.3 M pixels: 16-bit R = 6 192 x 48 x 96 142 / 119, R = 3 105 x 128 x
+//    74 70 / 56, fp32 window R = 5 34 x 361 x 80 327 / 286 (179 x 259 x 86, 4 M
+//    pixels, 597 / 715);
+//  * tables hinted beyond 8 pixels: only the 4-pixel lanes have the wider
+//    borders, and the others run the gather form in the launch (fp32 R = 9 4 x
+//    368 x 384 forward 137 / 276, 2 x 1251 x 148 backward 158 / - / 273; 16-bit
+//    backward 8 x 256^2 - / 332 / 428; forward 464^2 R = 10 - / 226 / 193);
+//  * fp64, 2 / 1: R = 3 17 x 100 x 140 (1071 tiles) forward 29 / 40, window R = 4
+//    8 x 176^2 (968) forward 40 / 39, backward 62 / 61, 512^2 (1024) 63 / 68.
 template <typename T>
 static int scatter_vec(const Dims& d, bool bwd) {
-    const int64_t pixels = static_cast<int64_t>(d.B) * d.C * d.H * d.W;
-    if (sizeof(T) == 8) return pixels >= (int64_t(1) << 18) ? 2 : 1;
-    const int64_t four = !bwd ? (int64_t(3) << 18)
-                              : (sizeof(T) == 2 ? (int64_t(7) << 17) : (int64_t(1) << 18));
-    return pixels >= four ? 4 : (pixels >= (int64_t(3) << 16) ? 2 : 1);
+    const int64_t planes = static_cast<int64_t>(d.B) * d.C;
+    const int64_t pixels = planes * d.H * d.W;
+    const int64_t cu = nsh_host::compute_units();
+    auto tiles = [&](int v, int rows) {
+        return planes * nsh_host::ceil_div(d.H, rows) * nsh_host::ceil_div(d.W, kTPR * v);
+    };
+    if (sizeof(T) == 8) return tiles(1, 16) < 4 * cu ? 1 : 2;
+    if (d.halo > kRmax) {
+        if (pixels >= (bwd && sizeof(T) == 2 ? int64_t(7) << 17 : int64_t(1) << 18) && d.W >= 64)
+            return 4;
+        return pixels >= (bwd ? int64_t(3) << 16 : int64_t(3) << 17) ? 2 : 1;
+    }
+    if (!bwd)
+        return pixels >= (int64_t(3) << 18) ? 4 : (pixels >= (int64_t(3) << 16) ? 2 : 1);
+    const bool whole = d.W % 16 == 0;
+    if (whole ? tiles(1, 32) <= (sizeof(T) == 4 ? 3 : 2) * cu : pixels < (int64_t(3) << 16))
+        return 1;
+    if (sizeof(T) == 2 || whole ? tiles(2, 32) <= 3 * cu
+                                : pixels < (d.W > 64 ? int64_t(1) << 19 : int64_t(1) << 18))
+        return 2;
+    const int64_t four = tiles(4, 32);
+    if (whole && four > 2 * cu && 2 * four <= 5 * cu) return 2;
+    // columns of the 64-wide tiles a fifth wider than the image's 32s
+    const bool idle = 10 * nsh_host::ceil_div(d.W, 64) >= 6 * nsh_host::ceil_div(d.W, 32);
+    return idle && (sizeof(T) == 2 || whole) && pixels < (int64_t(5) << 18) ? 2 : 4;
 }
 
 template <typename T, int VEC, bool BWD, int VAR>
@@ -1224,9 +1270,10 @@ static SPlan scatter_plan_cfg(const Dims& d) {
 
 // Which tiles a shape takes.  One round is one 1024-lane tile per compute
 // unit of the current device (256 on MI355X, also the fallback when no device
-// can be queried, e.g. a workspace query from a process without a GPU), or
-// two 512-lane ones.  The wide tiles move the most per pixel of halo and
-// spill, but a last round of a few of them takes as long as a full one, and
+// can be queried, e.g. a workspace query from a process without a GPU); two
+// 64-wide or half-height tiles hold its pixels, so they are counted at two per
+// compute unit, though a third fits by registers and LDS (74 and 46 KB of the
+// 64-wide forward).  The wide tiles have the least halo and spill per pixel, but a last round of a few of them takes as long as a full one, and
 // fewer than one round leaves compute units idle; so, per pass (half-plane
 // R = 5, 61 rows, except where said; wide / 64-wide / half-height, in us):
 //  * forward, 16-bit: 64-wide tiles always (4096^2 R = 7 1194 / 1099 / 1174,
@@ -1240,21 +1287,20 @@ static SPlan scatter_plan_cfg(const Dims& d) {
 //    105, 16-bit 79 / 73 / 75), except for fp32 rows of no whole vectors from
 //    half a round on (701 x 901: 102 / 121 / 108; 2 x 3 x 71 x 654, 0.4
 //    rounds: 92 / 52 / 67);
-//  * backward from one round, 16-bit: half-height tiles (two workgroups per
-//    compute unit: 4 x 512^2 R = 7 129 / 118 / 117, 16 x 3 x 256^2 230 / 226 /
-//    207, 4096^2 R = 7, 16 rounds, 2069 / 2006 / 1806; beyond 32 rounds the
-//    wide ones, with half the spill blocks); fp32: half-height where that saves
-//    rounds (2 x 3 x 321 x 481 177 / 176 / 120; not 16 x 3 x 256^2 304 / 327 /
-//    326).
+//  * backward from one round, 16-bit: half-height tiles (4 x 512^2 R = 7 129 /
+//    118 / 117, 16 x 3 x 256^2 230 / 226 / 207, 4096^2 R = 7, 16 rounds, 2069 /
+//    2006 / 1806), unless the 64-wide ones are one round and they are not (2 x
+//    820 x 520 R = 4 - / 70 / 85); beyond 32 rounds the wide ones, with half the
+//    spill blocks; fp32: half-height where that saves rounds (2 x 3 x 321 x 481
+//    177 / 176 / 120; not 16 x 3 x 256^2 304 / 327 / 326).
 static int64_t one_round_tiles() { return nsh_host::compute_units(); }
 
 // The plan for a shape: with the wide halo asked for, the 16- or
 // 24-pixel-border tiles where they apply; else by the rule above; *var says
 // which (p.ok false if none applies).  A pass whose workspace holds `room`
 // bytes, too few for the wider border's tiles, takes those of the 8-pixel
-// border (such a table's rows then run the gather form inside the launch), and
-// a forward with too few for the 64-wide tiles but enough for the wide ones
-// (7 and 5.5 bytes a pixel) takes those.
+// border, and one with too few for the 64-wide tiles but enough for the wide
+// ones (7 and 5.5 bytes a pixel, forward) takes those.
 template <typename T, int VEC, bool BWD>
 static SPlan scatter_plan_for(const Dims& d, int64_t room, int* var) {
     if constexpr (ScatterCfg<T, VEC, BWD, kVarWide>::kWide) {
@@ -1274,19 +1320,29 @@ static SPlan scatter_plan_for(const Dims& d, int64_t room, int* var) {
         const SPlan wide = scatter_plan_cfg<T, VEC, BWD, kVarWide>(d);
         const SPlan alt = scatter_plan_cfg<T, VEC, BWD, kVarAlt>(d);
         *var = kVarAlt;
-        // one 128-wide column of tiles would idle lanes that 64-wide ones use
-        if (!wide.ok || wide.grid.ntw < 2 || wide.grid.nth < 2) return alt;
+        // one 128-wide column of tiles would idle lanes that 64-wide ones use,
+        // and so would half of the last of two or three (64-wide and wide:
+        // window R = 3 298 x 100 x 134 fp32 backward 558 / 753 us, R = 4 8 x 304^2
+        // forward 41 / 51, 16 x 288^2 16-bit backward 168 / 203; of three, fp32
+        // rows of no whole vectors want the wide ones: R = 5 8 x 279^2 237 / 206)
+        const bool fits = alt.total <= room || wide.total > room;
+        if (!wide.ok || wide.grid.ntw < 2 || wide.grid.nth < 2 ||
+            (fits && (alt.grid.ntw == 3 ||
+                      (alt.grid.ntw == 5 && (!BWD || sizeof(T) == 2 || d.W % VEC == 0)))))
+            return alt;
         const int64_t cu = one_round_tiles();
         const double rounds = 0.9 * static_cast<double>(nsh_host::ceil_div(wide.tiles, cu));
         if constexpr (!BWD) {
             const bool narrow =
                 sizeof(T) == 2 || wide.tiles < cu ||
                 (wide.tiles > cu && rounds > static_cast<double>(alt.tiles) / (2 * cu));
-            if (narrow && (alt.total <= room || wide.total > room)) return alt;
+            if (narrow && fits) return alt;
         } else {
             const SPlan half = scatter_plan_cfg<T, VEC, BWD, kVarShort>(d);
             if (wide.tiles < cu) {
                 if (sizeof(T) == 2 || d.W % VEC == 0 || 2 * wide.tiles < cu) return alt;
+            } else if (sizeof(T) == 2 && alt.tiles <= 2 * cu && half.tiles > 2 * cu) {
+                return alt;
             } else if (half.ok &&
                        ((sizeof(T) == 2 && wide.tiles <= 32 * cu) ||
                         rounds > static_cast<double>(nsh_host::ceil_div(half.tiles, 2 * cu)))) {

@@ -33,11 +33,34 @@ def _tiles(B, C, H, W, dtype, backward, TW, TH, halo=8):
 
 # S, (B, C, H, W), dtype, pass, tile (None: the gather kernels)
 CASES = [
+    # the fp32 backward on rows of whole 16s: 1-pixel lanes while three
+    # workgroups per compute unit hold them, then 2-pixel ones
+    (25, (1, 1, 512, 512), F32, BWD, (16, 32)),
+    (113, (16, 1, 128, 128), F32, BWD, (16, 32)),
+    (81, (16, 1, 144, 144), F32, BWD, (16, 32)),
+    (81, (16, 1, 160, 160), F32, BWD, (32, 32)),
+    (81, (4, 1, 384, 384), F32, BWD, (32, 32)),
+    (121, (8, 1, 352, 352), F32, BWD, (32, 32)),
+    (121, (34, 1, 361, 80), F32, BWD, (32, 32)),
+    (81, (8, 1, 304, 304), F32, BWD, (64, 32)),
+    # other rows, and two columns of 64 where 128-wide tiles idle half of one
+    (81, (3, 1, 387, 386), F32, BWD, (32, 32)),
+    (49, (298, 1, 100, 134), F32, BWD, (64, 32)),
+    (61, (8, 1, 352, 352), F16, BWD, (32, 32)),
+    (85, (192, 1, 48, 96), F16, BWD, (32, 32)),
+    (41, (2, 1, 820, 520), F16, BWD, (64, 32)),
+    (81, (8, 1, 304, 304), F16, BWD, (64, 32)),
+    # fp64: 1-pixel lanes below four workgroups per compute unit
+    (25, (17, 1, 100, 140), F64, FWD, (32, 16)),
+    (5, (3, 1, 361, 230), F64, BWD, (32, 16)),
     # tables hinted beyond 8 pixels on tiles without a wider border
     (181, (4, 1, 280, 391), F64 | WIDE, FWD, None),
     (181, (4, 1, 280, 391), F64 | WIDE, BWD, None),
     (221, (1, 3, 953, 97), F16 | WIDE, BWD, None),
     (181, (1, 1, 592, 592), F64 | WIDE, BWD, (32, 16)),
+    # and on those with one
+    (181, (4, 1, 368, 384), F32 | WIDE, FWD, (128, 32, 16)),
+    (181, (2, 1, 1251, 148), F32 | WIDE, BWD, (64, 32, 24)),
     # a few rows on many badly filled tiles
     (5, (154, 1, 259, 100), F32, FWD, None),
     (5, (3, 1, 660, 660), F64, FWD, None),
