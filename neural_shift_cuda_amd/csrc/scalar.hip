@@ -47,6 +47,7 @@ constexpr int kScChunk = 4;  // neighbouring dx taken from one set of column val
 // rows a chunk's column values may reach past the halo (never used there)
 constexpr int kScPad = kScChunk - 1;
 constexpr int kScTile = (kScLH + kScPad) * kScPitch;
+constexpr int kScBatch = 4;  // rows in flight where the table is no grid
 
 // The table's near rows (|dx|, |dy| <= kRmax) as a grid over their bounding
 // box: cell (dyi, dxi) holds the table row of displacement (dx0 + dxi,
@@ -57,20 +58,39 @@ constexpr int kScRow = kScChunks * kScChunk;  // cells of a grid row, whole chun
 struct SGrid {
     int dx0, n, dy0, m;  // first displacement and extent in dx and dy
     bool dense;          // every near row has its own cell, at least half of them taken
-    bool all_near;       // no row lies beyond the halo
+    int single, far;     // near rows outside the grid (all of them or none), rows beyond the halo
 };
 
 // Builds the grid in `cell` (m rows of kScRow; -1: empty) from the staged
-// table; ends with a barrier.
+// table, and the table's far and near rows in order as lists: far row k at
+// list[k], near row k at list[S - 1 - k]; ends with a barrier.  A table of a
+// few rows is not worth a grid (one row, 16 x 3 x 256^2 fp64: the forward took
+// 20 us with it, 15 without).
+constexpr int kScGridRows = 5;
+
 template <int SGN>
-__device__ __forceinline__ SGrid stage_grid(const int4* shl, int S, int* cell) {
+__device__ __forceinline__ SGrid stage_grid(const int4* shl, int S, int* cell, int* list) {
     const int lane = threadIdx.x & 63;
-    for (int i = threadIdx.x; i < kScBox * kScRow; i += blockDim.x) cell[i] = -1;
+    if (S >= kScGridRows)
+        for (int i = threadIdx.x; i < kScBox * kScRow; i += blockDim.x) cell[i] = -1;
     // extent and number of the near rows, by every wave for itself
-    int lox = kRmax, hix = -kRmax, loy = kRmax, hiy = -kRmax, near = 0;
-    for (int s = lane; s < S; s += 64) {
-        const int dx = SGN * shl[s].x, dy = SGN * shl[s].y;
-        if (dx < -kRmax || dx > kRmax || dy < -kRmax || dy > kRmax) continue;
+    int lox = kRmax, hix = -kRmax, loy = kRmax, hiy = -kRmax, near = 0, nlist = 0, flist = 0;
+    for (int s0 = 0; s0 < S; s0 += 64) {
+        const int s = s0 + lane;
+        const bool row = s < S;
+        const int dx = row ? SGN * shl[s].x : 0, dy = row ? SGN * shl[s].y : 0;
+        const bool in = row && dx >= -kRmax && dx <= kRmax && dy >= -kRmax && dy <= kRmax;
+        const uint64_t nm = __ballot(in), fm = __ballot(row && !in);
+        if (threadIdx.x < 64 && row) {
+            const uint64_t before = (uint64_t(1) << lane) - 1;
+            if (in)
+                list[S - 1 - nlist - __popcll(nm & before)] = s;
+            else
+                list[flist + __popcll(fm & before)] = s;
+        }
+        nlist += __popcll(nm);
+        flist += __popcll(fm);
+        if (!in) continue;
         lox = min(lox, dx);
         hix = max(hix, dx);
         loy = min(loy, dy);
@@ -91,8 +111,8 @@ __device__ __forceinline__ SGrid stage_grid(const int4* shl, int S, int* cell) {
     g.n = __builtin_amdgcn_readfirstlane(hix) - g.dx0 + 1;
     g.m = __builtin_amdgcn_readfirstlane(hiy) - g.dy0 + 1;
     const int count = __builtin_amdgcn_readfirstlane(near);
-    g.dense = count > 0 && 2 * count >= g.n * g.m;
-    g.all_near = count == S;
+    g.dense = S >= kScGridRows && count > 0 && 2 * count >= g.n * g.m;
+    g.far = S - count;
     __syncthreads();
     if (g.dense) {
         for (int s = threadIdx.x; s < S; s += blockDim.x) {
@@ -107,7 +127,24 @@ __device__ __forceinline__ SGrid stage_grid(const int4* shl, int S, int* cell) {
         for (int o = 32; o > 0; o >>= 1) taken += __shfl_xor(taken, o, 64);
         g.dense = __builtin_amdgcn_readfirstlane(taken) == count;
     }
+    g.single = g.dense ? 0 : count;
     return g;
+}
+
+// The tile of a plane with its kRmax halo, every load of a lane before its
+// first write (15 of them in flight).
+template <typename T, typename A>
+__device__ __forceinline__ void stage_scalar_tile(A* st, const T* __restrict__ plane, int H, int W,
+                                                  int h0, int w0) {
+    constexpr int N = kScLH * kScPitch / kScThreads;
+    static_assert(N * kScThreads == kScLH * kScPitch, "whole rounds");
+    const bool cheap = H >= kScLH && W >= kScPitch;
+    T v[N];
+#pragma unroll
+    for (int i = 0; i < N; ++i)
+        v[i] = plane[halo_offset(threadIdx.x + i * kScThreads, kScPitch, h0, w0, H, W, cheap)];
+#pragma unroll
+    for (int i = 0; i < N; ++i) st[threadIdx.x + i * kScThreads] = to_acc(v[i]);
 }
 
 // The weights of the grid's cells (0 in an empty one) and, per chunk of four
@@ -150,18 +187,9 @@ __device__ __forceinline__ double wave_sum(double v) {
     return v;
 }
 
-// The value at (h + dx, w + dy) of a plane, for a row beyond the halo.
-__device__ __forceinline__ uint32_t far_offset(int h, int w, int dxm, int dym, int H, int W) {
-    int hh = h + dxm;
-    hh -= hh >= H ? H : 0;
-    int ww = w + dym;
-    ww -= ww >= W ? W : 0;
-    return static_cast<uint32_t>(hh) * W + ww;
-}
-
 // MODE 0: forward (src = x, writes U and Z);  MODE 1: gx (src = gU).
 template <typename T, int MODE>
-__global__ __launch_bounds__(kScThreads) void scalar_tile_kernel(
+__global__ __launch_bounds__(kScThreads, sizeof(acc_t<T>) == 4 ? 8 : 4) void scalar_tile_kernel(
     const void* __restrict__ src_v, const T* __restrict__ w, const int64_t* __restrict__ shifts,
     int cols, int S, int B, int C, int H, int W, int ntw, int nth, void* __restrict__ out0,
     acc_t<T>* __restrict__ out1) {
@@ -176,15 +204,16 @@ __global__ __launch_bounds__(kScThreads) void scalar_tile_kernel(
     A* wl = st + kScTile;
     int* cell = reinterpret_cast<int*>(wl + S);
     int* mask = cell + kScBox * kScRow;
+    int* list = mask + kScBox * kScChunks;
 
     const TileIdx ti = tile_of(xcd_tile(blockIdx.x, gridDim.x), ntw, nth, kScTH, kScTW);
     const int64_t HW = static_cast<int64_t>(H) * W;
     const int64_t BC = static_cast<int64_t>(B) * C;
     const Src* src = static_cast<const Src*>(src_v) + ti.bc * HW;
     for (int s = threadIdx.x; s < S; s += blockDim.x) wl[s] = to_acc(w[s * BC + ti.bc]);
-    stage_tile<Src, A>(st, src, H, W, ti.h0, ti.w0, kScLH, kScPitch, kScPitch);
+    stage_scalar_tile<Src, A>(st, src, H, W, ti.h0, ti.w0);
     stage_shifts(shl, shifts, S, cols, H, W, 0);  // ends with a barrier
-    const SGrid g = stage_grid<SGN>(shl, S, cell);
+    const SGrid g = stage_grid<SGN>(shl, S, cell, list);
 
     const int col = threadIdx.x & 63;
     const int r0 = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) * P;
@@ -234,28 +263,64 @@ __global__ __launch_bounds__(kScThreads) void scalar_tile_kernel(
             }
         }
     }
+    // Near rows without a grid, kScBatch at a time: the column values of all of
+    // them in flight, the next batch's records read before this one's FMAs.
+    if (g.single > 0) {
+        int offs[kScBatch];
+        A wsn[kScBatch];
+        auto rows = [&](int k0) {
+#pragma unroll
+            for (int j = 0; j < kScBatch; ++j) {
+                const int s = list[S - 1 - min(k0 + j, g.single - 1)];
+                const int4 r = shl[s];
+                offs[j] = __builtin_amdgcn_readfirstlane(SGN * (r.x * kScPitch + r.y));
+                wsn[j] = wl[s];
+            }
+        };
+        rows(0);
+        for (int k0 = 0; k0 < g.single; k0 += kScBatch) {
+            A v[kScBatch][P], ws[kScBatch];
+#pragma unroll
+            for (int j = 0; j < kScBatch; ++j) {
+                ws[j] = wsn[j];
+#pragma unroll
+                for (int i = 0; i < P; ++i) v[j][i] = own[offs[j] + i * kScPitch];
+            }
+            rows(k0 + kScBatch);
+#pragma unroll
+            for (int j = 0; j < kScBatch; ++j)
+                if (k0 + j < g.single)
+#pragma unroll
+                    for (int i = 0; i < P; ++i) u[i] = fma_acc(ws[j], v[j][i], u[i]);
+        }
+    }
+    // Rows beyond the halo, from global memory, kScBatch at a time.  A pixel
+    // outside the image reads some pixel's value and stores nothing.
     const int w_px = ti.w0 + col;
     const bool wact = w_px < W;
-    for (int s = 0; s < S && !(g.dense && g.all_near); ++s) {
-        const ShiftRec r = read_shift(shl, s);
-        if (shift_in_lds(r)) {
-            if (g.dense) continue;
-            const A ws = wl[s];
-            const A* sr = own + SGN * (r.dx * kScPitch + r.dy);
+    for (int k0 = 0; k0 < g.far; k0 += kScBatch) {
+        A v[kScBatch][P], ws[kScBatch];
 #pragma unroll
-            for (int i = 0; i < P; ++i) u[i] = fma_acc(ws, sr[i * kScPitch], u[i]);
-        } else {
-            const A ws = wl[s];
+        for (int j = 0; j < kScBatch; ++j) {
+            const int s = __builtin_amdgcn_readfirstlane(list[min(k0 + j, g.far - 1)]);
+            const ShiftRec r = read_shift(shl, s);
+            ws[j] = wl[s];
             // (p - s) mod = (p + (H - dx mod H)) mod
             const int dxm = MODE == 0 ? r.dxm : (r.dxm ? H - r.dxm : 0);
             const int dym = MODE == 0 ? r.dym : (r.dym ? W - r.dym : 0);
+            const uint32_t ww = wrap1(min(w_px, W - 1) + dym, W);
+            int hh = wrap1(min(ti.h0 + r0, H - 1) + dxm, H);
 #pragma unroll
             for (int i = 0; i < P; ++i) {
-                const int h = ti.h0 + r0 + i;
-                if (wact && h < H)
-                    u[i] = fma_acc(ws, to_acc(src[far_offset(h, w_px, dxm, dym, H, W)]), u[i]);
+                v[j][i] = to_acc(src[static_cast<uint32_t>(hh) * static_cast<uint32_t>(W) + ww]);
+                hh = hh + 1 == H ? 0 : hh + 1;
             }
         }
+#pragma unroll
+        for (int j = 0; j < kScBatch; ++j)
+            if (k0 + j < g.far)
+#pragma unroll
+                for (int i = 0; i < P; ++i) u[i] = fma_acc(ws[j], v[j][i], u[i]);
     }
     if (!wact) return;
 #pragma unroll
@@ -303,6 +368,21 @@ __device__ __forceinline__ double wave_sum4(double (&v)[4]) {
     return t;
 }
 
+// sum over i < 16 of gu[i0 + i] value(i), as two chains of eight products: one
+// chain over a column's 32 rows made the weight gradient's error against 64
+// bits 4 to 12% larger than sums of four pixels over eight waves; with the
+// chains and their tree it is smaller.
+template <typename A, typename F>
+__device__ __forceinline__ A gu_sum(const A (&gu)[kScTH], int i0, F&& value) {
+    A a = A(0), b = A(0);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        a = fma_acc(gu[i0 + i], value(i), a);
+        b = fma_acc(gu[i0 + 8 + i], value(8 + i), b);
+    }
+    return a + b;
+}
+
 // gw partials of one tile: part[(s*BC + bc)*ntp + tile] =
 //   sum_{p in tile} gU[p] x[(p+s) mod] + gZ[p]
 // Every wave holds the whole tile's gU (a lane its column, 32 rows) and takes
@@ -320,6 +400,7 @@ __global__ __launch_bounds__(kScThreads) void scalar_gw_tile_kernel(
     A* xt = reinterpret_cast<A*>(smem + shift_lds_bytes(S));
     A* gzw = xt + kScTile;  // the waves' shares of the tile's gZ
     int* cell = reinterpret_cast<int*>(gzw + kScWaves);
+    int* list = cell + kScBox * kScRow;
 
     // plain tile order: the partial index is the tile's position in its plane
     const int64_t ntp = static_cast<int64_t>(ntw) * nth;
@@ -355,9 +436,9 @@ __global__ __launch_bounds__(kScThreads) void scalar_gw_tile_kernel(
     }
     gz = wave_sum(gz);
     if (col == 0) gzw[wave] = gz;
-    stage_tile<T, A>(xt, xp, H, W, ti.h0, ti.w0, kScLH, kScPitch, kScPitch);
+    stage_scalar_tile<T, A>(xt, xp, H, W, ti.h0, ti.w0);
     stage_shifts(shl, shifts, S, cols, H, W, 0);  // ends with a barrier
-    const SGrid g = stage_grid<1>(shl, S, cell);
+    const SGrid g = stage_grid<1>(shl, S, cell, list);
     A gz_tile = A(0);  // the sum of gZ over the tile, part of every shift's sum
 #pragma unroll
     for (int i = 0; i < kScWaves; ++i) gz_tile += gzw[i];
@@ -370,16 +451,15 @@ __global__ __launch_bounds__(kScThreads) void scalar_gw_tile_kernel(
             const A* cv = own + (g.dx0 + dxi) * kScPitch + g.dy0 + dyi;
             A acc[CH];
 #pragma unroll
-            for (int j = 0; j < CH; ++j) acc[j] = A(0);
-#pragma unroll
             for (int i0 = 0; i0 < TH; i0 += SUB) {
                 A v[SUB + CH - 1];
 #pragma unroll
                 for (int i = 0; i < SUB + CH - 1; ++i) v[i] = cv[(i0 + i) * kScPitch];
 #pragma unroll
-                for (int i = 0; i < SUB; ++i)
-#pragma unroll
-                    for (int j = 0; j < CH; ++j) acc[j] = fma_acc(gu[i0 + i], v[i + j], acc[j]);
+                for (int j = 0; j < CH; ++j) {
+                    const A t = gu_sum<A>(gu, i0, [&](int i) { return v[i + j]; });
+                    acc[j] = i0 == 0 ? t : acc[j] + t;
+                }
             }
             static_assert(CH == 4, "one value per 16-lane row");
             const int s = cell[dyi * kScRow + dxi + (col >> 4)];  // -1 beyond the box
@@ -388,22 +468,43 @@ __global__ __launch_bounds__(kScThreads) void scalar_gw_tile_kernel(
                 part[(static_cast<int64_t>(s) * BC + ti.bc) * ntp + tile] = t;
         }
     }
-    for (int s = wave; s < S && !(g.dense && g.all_near); s += kScWaves) {
+    for (int k = wave; k < g.single; k += kScWaves) {
+        const int s = __builtin_amdgcn_readfirstlane(list[S - 1 - k]);
         const ShiftRec r = read_shift(shl, s);
+        const A* sr = own + r.dx * kScPitch + r.dy;
         A acc = A(0);
-        if (shift_in_lds(r)) {
-            if (g.dense) continue;
-            const A* sr = own + r.dx * kScPitch + r.dy;
 #pragma unroll
-            for (int i = 0; i < TH; ++i) acc = fma_acc(gu[i], sr[i * kScPitch], acc);
-        } else {
-            const int rows = wact ? min(TH, H - ti.h0) : 0;
-            for (int i = 0; i < rows; ++i) {
-                const int h = ti.h0 + i;
-                const uint32_t o = static_cast<uint32_t>(h) * static_cast<uint32_t>(W) + w_px;
-                acc = fma_acc(gU[ti.bc * HW + o],
-                              to_acc(xp[far_offset(h, w_px, r.dxm, r.dym, H, W)]), acc);
+        for (int i0 = 0; i0 < TH; i0 += SUB) {
+            A v[SUB];
+#pragma unroll
+            for (int i = 0; i < SUB; ++i) v[i] = sr[(i0 + i) * kScPitch];
+            acc += gu_sum<A>(gu, i0, [&](int i) { return v[i]; });
+        }
+        const A t = wave_sum(acc) + gz_tile;
+        if (col == 0) part[(static_cast<int64_t>(s) * BC + ti.bc) * ntp + tile] = t;
+    }
+    // Rows beyond the halo, from global memory.  A pixel outside the image
+    // reads some pixel's value and takes 0 (gU is 0 there, but the value may
+    // be infinite).
+    for (int k = wave; k < g.far; k += kScWaves) {
+        const int s = __builtin_amdgcn_readfirstlane(list[k]);
+        const ShiftRec r = read_shift(shl, s);
+        const uint32_t ww = wrap1(min(w_px, W - 1) + r.dym, W);
+        int hh = wrap1(ti.h0 + r.dxm, H);
+        int rows = wact ? H - ti.h0 : 0;  // the lane's pixels
+        asm volatile("" : "+v"(rows));    // 32 comparisons a row, not 32 masks kept over all rows
+        A acc = A(0);
+#pragma unroll
+        for (int i0 = 0; i0 < TH; i0 += SUB) {
+            A v[SUB];
+#pragma unroll
+            for (int i = 0; i < SUB; ++i) {
+                v[i] = to_acc(xp[static_cast<uint32_t>(hh) * static_cast<uint32_t>(W) + ww]);
+                hh = hh + 1 == H ? 0 : hh + 1;
             }
+            acc += gu_sum<A>(gu, i0, [&](int i) {
+                return i0 + i < rows ? v[i] : A(0);
+            });
         }
         const A t = wave_sum(acc) + gz_tile;
         if (col == 0) part[(static_cast<int64_t>(s) * BC + ti.bc) * ntp + tile] = t;
@@ -436,7 +537,7 @@ static int s_tile(const void* src, const void* w, const int64_t* sh, int cols, i
     const int64_t tiles = static_cast<int64_t>(B) * C * ntw * nth;
     const size_t lds = shift_lds_bytes(S) +
                        (kScBox * kScRow + static_cast<size_t>(kScTile) + S) * sizeof(A) +
-                       kScBox * (kScRow + kScChunks) * sizeof(int);
+                       (kScBox * (kScRow + kScChunks) + S) * sizeof(int);
     hipLaunchKernelGGL((scalar_tile_kernel<T, MODE>), dim3(static_cast<unsigned>(tiles)),
                        dim3(kScThreads), lds, st, src, static_cast<const T*>(w), sh, cols, S, B, C,
                        H, W, ntw, nth, out0, static_cast<A*>(out1));
@@ -460,7 +561,7 @@ static int s_gw(const void* x, const void* gU, const void* gZ, const int64_t* sh
     const int nsplit = ntw * nth;
     const int64_t tiles = static_cast<int64_t>(B) * C * nsplit;
     const size_t lds = shift_lds_bytes(S) + (kScTile + kScWaves) * sizeof(A) +
-                       kScBox * kScRow * sizeof(int);
+                       (kScBox * kScRow + S) * sizeof(int);
     hipLaunchKernelGGL((scalar_gw_tile_kernel<T>), dim3(static_cast<unsigned>(tiles)),
                        dim3(kScThreads), lds, st, static_cast<const T*>(x),
                        static_cast<const A*>(gU), static_cast<const A*>(gZ), sh, cols, S, B, C, H,
