@@ -888,7 +888,10 @@ normalized_fwd_scatter_kernel(const T* __restrict__ x, const T* __restrict__ w,
         }
     }
 
-    if (weights_ok != nullptr) {
+    // the head-mixing kernels (NH > 1) are never asked (weights_ok is null), and
+    // their registers are full: with the check in them four heads spilled 22 to
+    // 27 registers a lane
+    if (NH == 1 && weights_ok != nullptr) {
         // every weight the box kept went into its own pixel's state
         bool bad = false;
 #pragma unroll
@@ -1808,7 +1811,11 @@ static int n_scatter_fwd_cfg(const void* x, const void* w, const int64_t* sh, ND
     A* spill = reinterpret_cast<A*>(base + kNHeader);
     A* part = reinterpret_cast<A*>(base + kNHeader + p.spill_bytes);
     const int64_t step = static_cast<int64_t>(d.B) * (NH > 1 ? NH : d.C) * d.H * d.W;
-    hipLaunchKernelGGL((normalized_fwd_scatter_kernel<T, V, TPR, RW, Cfg::D, LOGW, Cfg::WPE, NH,
+    // Four heads' ring slots take 32 registers a shift ahead: at depth 2 the
+    // kernel spilled 17 to 27 of them (4 heads, C = 3, R = 5 512^2 fp32 160 -> 146
+    // us, R = 7 1024^2 fp16 663 -> 614).
+    constexpr int D_ = NH == 4 ? 1 : Cfg::D;
+    hipLaunchKernelGGL((normalized_fwd_scatter_kernel<T, V, TPR, RW, D_, LOGW, Cfg::WPE, NH,
                                                       Cfg::HALO>),
                        dim3(static_cast<unsigned>(p.tiles)), dim3(TPR * RW), p.lds, st,
                        static_cast<const T*>(x), static_cast<const T*>(w), sh, d.S, d.codes, d.C, d.H, d.W,

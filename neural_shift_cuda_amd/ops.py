@@ -766,7 +766,13 @@ def normalized_accumulate_uz_mixed(x: torch.Tensor, head_weights: torch.Tensor,
         x_d, hw_d = _device_operands(x, head_weights)
         rules = _row_rules(shifts, periodic_inverse, box_forward)
         _require_cuda_ext("normalized_accumulate_uz_mixed", need_normalized=True)
-        out = _C.normalized_accumulate_uz_forward_mixed(
+        # fp32, three or four heads: the head planes' 4-byte reads bound the
+        # fused forward, and on an image whose last tiles are shifted mixing
+        # first is ahead (C = 3, R = 5, 321 x 481: 3 heads 149 -> 128 us, 4 heads
+        # 182 -> 135, 16-bit 4 heads 105 -> 113; 320 x 484 2 heads 104 -> 119)
+        mix_first = (x_d.dtype == torch.float32 and h >= 3
+                     and (0 < x.shape[2] % 32 < 8 or 0 < x.shape[3] % 128 < 8))
+        out = None if mix_first else _C.normalized_accumulate_uz_forward_mixed(
             x_d.contiguous(), hw_d.contiguous(), head_mix, shifts, rules=rules)
         if out is not None:
             D, log_C = out
