@@ -638,7 +638,11 @@ __device__ __forceinline__ int near_radius(const int4* shl, int S, bool only_inv
 // 0.642 -> 0.621 ms), the fp32 forward on 128-wide tiles 2% (on 64-wide
 // tiles 13% slower: c3 0.326 -> 0.368 ms); the 16-bit forward 2% slower,
 // the fp16 and fp64 backwards within the run-to-run spread (+-2%).  So:
-// nontemporal in the fp32 and fp64 forwards and the fp32 backward.
+// nontemporal in the fp64 forward and, with 32 lanes a row, in the fp32 forward
+// and backward.  Those are the 128-wide tiles and the wide border's 64-wide
+// ones of 2-pixel lanes, where it makes little difference (R = 10 1024^2 forward
+// 331 us, plain 334, backward 452 and 456; R = 9 3 x 792^2 530 and 529, 893 and
+// 860); the other 64-wide tiles load plainly.
 template <typename T, int TPR>
 constexpr bool kNormFwdNT = sizeof(T) == 8 || (sizeof(T) == 4 && TPR == 32);
 template <typename T, int TPR>
@@ -1355,7 +1359,8 @@ normalized_bwd_scatter_kernel(const T* __restrict__ x, const T* __restrict__ w,
 // of 321 x 481 R = 6 256 and 113.  Rows beyond the border take the gather form
 // here too, and that is still the faster side of the two for tables that the
 // per-channel kernels serve on the 16-pixel border (R = 10, 221 rows, fp32:
-// 1230 and 494 us; 69 rows of radius 16, 832 and 215).  Bound by the loop's
+// 1230 and 494 us; 69 rows of radius 16 under NSH_WIDE_HALO, which the Python
+// layer does not set for so few, 832 and 215).  Bound by the loop's
 // LDS accesses (13 reads and 3 writes per pixel and row) at 16 waves per CU:
 // fp16 takes 0.93 of fp32's time.
 // beta stays per channel, so that each score is formed as above: with the
@@ -1929,6 +1934,57 @@ static int64_t n_workspace(const NDims& d, bool bwd) {
     return bwd ? n_workspace<T, true>(d) : n_workspace<T, false>(d);
 }
 
+// Whether the gather kernels beat the tiles that would serve a call: rows that
+// take no vectors of 4 on few workgroups of the gather kernels (16 rows x 16
+// vectors, 256 lanes), whose one- and two-pixel lanes walk the table faster
+// than the tiles' four, as long as all of them run at once; and forwards of
+// tables of a few rows, whose spilled border and fix-up cost as much as the
+// rows.  In us, tiles and gather kernels, or the ratio of the two:
+//  * fp32, odd rows: 137 x 73 R = 4 forward 58 / 25, backward 57 / 35; window
+//    R = 5 133^2 77 / 36 and 142 / 84; at 1024 workgroups R = 5 1.16 to 1.45, at
+//    1444 0.97 to 1.28, at 2048 0.8;
+//  * fp32, W % 4 = 2: 1.0 to 1.7 at 330 workgroups, 0.8 to 1.1 at 780 (in up to
+//    96 columns a third of the gather's lanes idle: R = 8 3 x 1023 x 38 122 / 175);
+//  * 16-bit, odd rows: forward 1.0 to 1.5 at 720, backward 0.9 to 1.2 at 1024
+//    (R = 8 0.9 at 620 and 1000); W % 4 = 2: R = 3 1.0 to 1.4 at 510, R = 5 0.9 to
+//    1.2 at 360, R = 7 0.5 to 0.8;
+//  * on a wide border the tiles' lanes hold two pixels and win sooner (R = 9
+//    36 x 59 131 / 100; R = 10 953 x 97, 1260 workgroups, 170 / 250);
+//  * fp64, forward: R = 1 192 x 35 x 154 86 / 34, odd rows R = 3 1.0 to 1.3 at
+//    1024, window R = 4 53 x 71 36 / 28;
+//  * few rows: fp32 R = 1 96 x 128 20 / 14, R = 2 3 x 160^2 28 / 22; fp16 R = 1 64 x
+//    259 x 134 60 / 39;
+//  * 128-wide fp32 tiles mostly beyond a narrow image: R = 3 192 x 48 x 129
+//    121 / 94.
+template <typename T, bool BWD>
+static bool n_gather_instead(const NDims& d) {
+    const int vec = d.W % 2 ? 1 : (d.W % 4 ? 2 : 4);
+    const int64_t blocks = static_cast<int64_t>(d.B) * d.C * nsh_host::ceil_div(d.H, 16) *
+                           nsh_host::ceil_div(d.W, 16 * vec);
+    const bool few = !BWD && d.S <= 13;
+    int most;  // workgroups per compute unit up to which the gather kernels win
+    if (sizeof(T) == 8) {
+        most = d.S <= 25 ? 4 : (d.S <= 81 ? 1 : 0);
+        most = BWD || vec > 1 ? 0 : most;
+        if (few) return true;
+    } else if (vec == 1) {
+        if (few && d.S <= 5) return true;
+        const int half = BWD ? 4 : 3;  // 16-bit
+        most = sizeof(T) == 4 || d.S <= 25 ? 5 : (d.S <= 81 ? half : half - 1);
+        most = d.wide ? 1 : (few ? 8 : most);
+    } else if (vec == 2) {
+        if (few && (sizeof(T) == 4 || d.S <= 5)) return true;
+        const int half = d.S <= 25 ? 2 : (d.S <= 61 ? 1 : 0);  // 16-bit
+        most = d.wide || d.W <= 96 ? 0 : (sizeof(T) == 4 ? 2 : half);
+    } else {
+        most = few && sizeof(T) == 4 && d.W > 64 ? 2 : 0;
+    }
+    if (!BWD && sizeof(T) == 4 && vec < 4 && d.S <= 25 && d.W > 64 &&
+        5 * nsh_host::ceil_div(d.W, 128) * 128 >= 8 * d.W)
+        return true;
+    return most > 0 && blocks <= most * static_cast<int64_t>(nsh_host::compute_units());
+}
+
 // The plan that a call's workspace allows (p.ok is false if none).
 template <typename T, bool BWD>
 static NPlan n_usable_plan(const NDims& d, void* ws, int64_t ws_bytes) {
@@ -1942,7 +1998,7 @@ template <typename T, bool LOGW>
 static int n_run_fwd(const void* x, const void* w, const int64_t* sh, NDims d, void* D, void* L,
                      void* ws, int64_t ws_bytes, int* weights_ok, hipStream_t st) {
     const NPlan p = n_usable_plan<T, false>(d, ws, ws_bytes);
-    if (p.ok)
+    if (p.ok && !n_gather_instead<T, false>(d))
         return n_scatter_fwd<T, LOGW>(x, w, sh, d, D, L, p, ws, weights_ok, st);
     switch (n_pick_vec<T>(d.W, {x, w, D, L}, d.S, false)) {
         case 8: if constexpr (sizeof(T) == 2) return n_launch_fwd<T, 8, LOGW>(x, w, sh, d, D, L, weights_ok, st); break;
@@ -1958,7 +2014,7 @@ static int n_run_bwd(const void* x, const void* w, const void* D, const void* L,
                      const void* gL, const int64_t* sh, NDims d, void* gx, void* gw, void* ws,
                      int64_t ws_bytes, hipStream_t st) {
     const NPlan p = n_usable_plan<T, true>(d, ws, ws_bytes);
-    if (p.ok)
+    if (p.ok && !n_gather_instead<T, true>(d))
         return n_scatter_bwd<T, LOGW>(x, w, D, L, gD, gL, sh, d, gx, gw, p, ws, st);
     switch (n_pick_vec<T>(d.W, {x, w, D, L, gD, gL, gx, gw}, d.S, true)) {
         case 8: if constexpr (sizeof(T) == 2) return n_launch_bwd<T, 8, LOGW>(x, w, D, L, gD, gL, sh, d, gx, gw, st); break;
