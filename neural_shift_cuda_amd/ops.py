@@ -100,11 +100,11 @@ def _prep_shifts_for_cuda(shifts: torch.Tensor, device: torch.device,
     if (shifts.dtype == torch.int64 and shifts.device == device and shifts.is_contiguous()):
         return shifts
     out = shifts.to(device=device, dtype=torch.int64).contiguous()
-    if out is not shifts and _HAS_CUDA_EXT and (radius or not shifts.is_cuda):
+    if out is not shifts and _HAS_CUDA_EXT:
         # the kernels' launch shape depends on the table's radius: record it
         # from the caller's table, so that the copy is never read back (a
         # device table is read once, where the op will need the radius)
-        r = _C.table_radius(shifts)
+        r = _C.table_radius(shifts) if radius else _C.known_radius(shifts)
         if r is not None:
             _C.remember_table_radius(out, r)
     return out
@@ -540,8 +540,7 @@ class _NormalizedAccumulateUZFn(torch.autograd.Function):
     def forward(ctx, x, weights, shifts, log_weights, rules=0, shared=False, weights_ok=None):
         if shifts.dim() != 2 or shifts.size(1) != 3:
             raise ValueError("normalized_accumulate_uz requires shifts of shape (S, 3)")
-        shifts_i = _prep_shifts_for_cuda(shifts, x.device, radius=(
-            x.dtype == torch.float64 or shifts.size(0) > _C._HALO8_HALF_ROWS))
+        shifts_i = _prep_shifts_for_cuda(shifts, x.device)
         x_c, w_c = x.contiguous(), weights.contiguous()
         D, log_C = _C.normalized_accumulate_uz_forward(x_c, w_c, shifts_i, bool(log_weights),
                                                        rules=rules, shared_weights=shared,
