@@ -125,6 +125,23 @@ def _row_rules(shifts: torch.Tensor, periodic_inverse: bool, box_forward: bool) 
             | (_C.NSH_BOX_FORWARD if box_forward else 0))
 
 
+def _own_table(shifts: torch.Tensor, rules: int, x: torch.Tensor, weights: torch.Tensor,
+               radius: bool = False) -> torch.Tensor:
+    """The table that a differentiable call with row rules keeps for its
+    backward: a copy, so that the caller may rewrite its own in between (the
+    rules used to be written out into a new table).  Without rules the
+    caller's table itself is saved, as ever, and autograd reports the change."""
+    if not (rules and torch.is_grad_enabled() and (x.requires_grad or weights.requires_grad)
+            and shifts.device == x.device and shifts.dtype == torch.int64
+            and shifts.is_contiguous()):
+        return shifts  # nothing is saved, or a converted copy is
+    out = shifts.clone()
+    r = _C.table_radius(shifts) if radius else _C.known_radius(shifts)
+    if r is not None:
+        _C.remember_table_radius(out, r)
+    return out
+
+
 def _mirror_table(shifts: torch.Tensor, periodic_inverse: bool,
                   box_forward: bool = False) -> Tuple[torch.Tensor, bool]:
     """(table, row_codes).  Without an extension the caller's table is
@@ -691,6 +708,7 @@ def accumulate_uz(x: torch.Tensor, weights: torch.Tensor, shifts: torch.Tensor, 
         rules = _row_rules(shifts, periodic_inverse, box_forward)
         x_d, w_d = _device_operands(x, weights)
         _require_cuda_ext("accumulate_uz")
+        shifts = _own_table(shifts, rules, x_d, w_d, radius=True)
         return _AccumulateUZFn.apply(x_d, w_d, shifts, rules, bool(shared_weights))
     weights = _shared_operand(weights, x.shape[1], shared_weights)
     x_acc, w_acc = _promote_accumulation_inputs(x, weights)
@@ -718,6 +736,7 @@ def normalized_accumulate_uz(x: torch.Tensor, weights: torch.Tensor, shifts: tor
     if x_d.is_cuda:
         rules = _row_rules(shifts, periodic_inverse, box_forward)
         _require_cuda_ext("normalized_accumulate_uz", need_normalized=True)
+        shifts = _own_table(shifts, rules, x_d, w_d)
         # the forward kernel checks every weight as it reads it
         ok = (torch.ones((), dtype=torch.int32, device=x_d.device)
               if validate and in_kernel else None)

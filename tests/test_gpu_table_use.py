@@ -1,9 +1,10 @@
 """How the ops use a caller's shift table: the normalized op learns nothing by
-waiting for the device."""
+waiting for the device, and a differentiable call with row rules keeps a table
+of its own."""
 import pytest
 import torch
 
-from neural_shift_cuda import normalized_accumulate_uz
+from neural_shift_cuda import accumulate_uz, normalized_accumulate_uz
 from neural_shift_cuda_amd import _C
 from neural_shift_cuda_amd.workloads import halfplane_shifts, window_shifts
 
@@ -69,3 +70,31 @@ def test_hint_of_an_unread_table():
     assert _C._norm_halo_flag(known, torch.float32) == 0
     assert _C.table_radius(known) == 10
     assert _C._norm_halo_flag(known, torch.float32) == _C.NSH_WIDE_HALO
+
+
+@pytest.mark.parametrize("op", [accumulate_uz, normalized_accumulate_uz])
+@pytest.mark.parametrize("rules", [dict(periodic_inverse=True), dict(box_forward=True)])
+def test_table_rewritten_before_the_backward(op, rules):
+    """The gradients are those of the table the forward saw."""
+    want = []
+    for rewrite in (False, True):
+        sh = halfplane_shifts(3).to(DEV)
+        x, w = _inputs(sh.size(0))
+        out = op(x, w, sh, **rules)
+        out = out[0] if isinstance(out, tuple) else out
+        if rewrite:
+            sh.zero_()
+        want.append(torch.autograd.grad(out, [x, w], torch.ones_like(out)))
+    for a, b in zip(*want):
+        assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("op", [accumulate_uz, normalized_accumulate_uz])
+def test_rewritten_table_is_reported_without_rules(op):
+    sh = halfplane_shifts(3).to(DEV)
+    x, w = _inputs(sh.size(0))
+    out = op(x, w, sh)
+    out = out[0] if isinstance(out, tuple) else out
+    sh.zero_()
+    with pytest.raises(RuntimeError, match="modified by an inplace operation"):
+        torch.autograd.grad(out, [x, w], torch.ones_like(out))
