@@ -544,11 +544,12 @@ def mix_head_planes(w: torch.Tensor, mix: torch.Tensor) -> torch.Tensor:
 
 
 # Shared weights' own gradient is formed in one pass from this many pixels
-# (B * H * W) on.  Below, a forward and backward take the host longer (~150 us)
-# than the kernels either way (1x3x72x200 R = 3: 50 us per channel, 27 in one
-# pass), and the per-channel kernels' x gradient is the broadcast weights' bit
-# for bit; above, 8x3x250^2 R = 5 fp32 takes 330 us per channel
-# (two kernels and the sum) and 112 in one pass.
+# (B * H * W) on.  That form is the faster one at every size measured (backward
+# alone, one pass and per channel with the sum, C = 3, R = 5: fp32 1x64^2 48 and
+# 72 us, 1x182^2 53 and 105, 8x250^2 108 and 326; fp16 47 and 74, 52 and 100, 98
+# and 256); the line keeps a promise, not a crossing: below it, where a
+# forward and backward are mostly the host's (fp32 R = 5 1x72x200 154 and 183 us,
+# fp16 121 and 149), x gradients stay bitwise those of the broadcast weights.
 _ONE_PASS_PIXELS = 1 << 15
 
 
