@@ -374,9 +374,12 @@ def _halo_flag(shifts: torch.Tensor) -> int:
     17..24: accumulate_uz's scatter tiles then carry a 16- or 24-pixel border
     (include/neural_shift_hip.h).  Only a hint; the kernels check the radius
     themselves."""
-    r = table_radius(shifts)
+    return _halo_flag_of(table_radius(shifts), shifts.size(0))
+
+
+def _halo_flag_of(r: Optional[int], rows: int) -> int:
     if r is None:
-        return NSH_WIDE_HALO if shifts.size(0) > _HALO8_ROWS else 0
+        return NSH_WIDE_HALO if rows > _HALO8_ROWS else 0
     if 8 < r <= 16:
         return NSH_WIDE_HALO
     return NSH_WIDER_HALO if 16 < r <= 24 else 0
@@ -422,11 +425,12 @@ def accumulate_uz_forward(x: torch.Tensor, weights: torch.Tensor,
     sh, B, C, H, W, S = _check_pair("accumulate_uz", x, weights, shifts,
                                     "weights shape must be (S*B, C, H, W)", shared_weights)
     acc = _acc_dtype(x.dtype)
+    r = table_radius(shifts)
     code = (_code(x, "accumulate_uz_fwd") | _flags(row_codes, shared_weights, rules)
-            | _halo_flag(shifts))
+            | _halo_flag_of(r, S))
     U = torch.empty(x.shape, dtype=acc, device=x.device)
     Z = torch.empty(x.shape, dtype=acc, device=x.device)
-    ws, nws = _workspace(S, B, C, H, W, code, False, x.device, shifts)
+    ws, nws = _workspace(S, B, C, H, W, code, False, x.device, r)
     if band is None:
         _call_on(x, "nsh_accumulate_uz_forward", x.data_ptr(), weights.data_ptr(), sh.data_ptr(),
                  S, B, C, H, W, code, U.data_ptr(), Z.data_ptr(), _ptr(ws), nws)
@@ -438,20 +442,18 @@ def accumulate_uz_forward(x: torch.Tensor, weights: torch.Tensor,
     return [U, Z]
 
 
-def _workspace(S, B, C, H, W, code, backward, device, shifts):
+def _workspace(S, B, C, H, W, code, backward, device, r):
     """Scratch buffer of accumulate_uz (spilled window borders of the
     once-per-element weight stream); (None, 0) when the shape needs none, and
-    for a table beyond every border (24 pixels), all of whose rows would run
+    for a table of radius r beyond every border (24 pixels), all of whose rows run
     the gather form at the tiles' occupancy, which only a backward on whole
     vectors of whole tiles does as fast as the gather kernels."""
     n = _bytes_on(device.index, "nsh_accumulate_uz_workspace_bytes", S, B, C, H, W, code,
                   int(backward))
     if n <= 0:
         return None, 0
-    if not code & (NSH_WIDE_HALO | NSH_WIDER_HALO) and not (backward and W % 16 == H % 16 == 0):
-        r = table_radius(shifts)
-        if r is not None and r > 24:
-            return None, 0
+    if r is not None and r > 24 and not (backward and W % 16 == H % 16 == 0):
+        return None, 0
     return torch.empty(n, dtype=torch.uint8, device=device), n
 
 
@@ -474,11 +476,12 @@ def accumulate_uz_backward(x: torch.Tensor, weights: torch.Tensor, grad_U: torch
     acc = _acc_dtype(x.dtype)
     gU = _grad_in(grad_U, x, acc, "grad_U")
     gZ = _grad_in(grad_Z, x, acc, "grad_Z")
+    r = table_radius(shifts)
     code = (_code(x, "accumulate_uz_bwd") | _flags(row_codes, shared_weights, rules)
-            | _halo_flag(shifts))
+            | _halo_flag_of(r, S))
     gx = torch.empty_like(x)
     gw = torch.empty((S * B, C, H, W), dtype=weights.dtype, device=weights.device)
-    ws, nws = _workspace(S, B, C, H, W, code, True, x.device, shifts)
+    ws, nws = _workspace(S, B, C, H, W, code, True, x.device, r)
     if band is None:
         _call_on(x, "nsh_accumulate_uz_backward", x.data_ptr(), weights.data_ptr(),
                  gU.data_ptr(), gZ.data_ptr(), sh.data_ptr(), S, B, C, H, W, code, gx.data_ptr(),
